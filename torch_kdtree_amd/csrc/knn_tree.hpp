@@ -2,12 +2,11 @@
 //
 // One query per lane.  Each lane runs the reference's near-first depth-first search
 // (src/kdtree.cpp:16-110) without a stack or a tag array: the state is the node index, its
-// depth and the projected point pp (D registers).  Coming back up from a child, the lane
-// recomputes which side was the near one (q[a] < m) to tell whether the far side is still
-// to be tested; that is exactly the information the reference's per-node tags hold for the
-// nodes on the active path, and nodes off the path are never revisited.  The pruning bound,
-// the pp updates and the candidate insertion repeat the reference's arithmetic, so with the
-// reference tie policy every lane produces what the reference CPU search produces.
+// depth, the projected point pp (D registers) and far_mask, the levels of the current path that were
+// entered through their far child: what the reference's per-node tags hold for the nodes on the
+// active path (nodes off the path are never revisited).  Pruning takes every decision the reference
+// takes that can change the result, and the candidate insertion repeats its arithmetic, so with
+// the reference tie policy every lane produces what the reference CPU search produces.
 //
 // Queries arrive in an order given by `order` (a presort below: Morton buckets of the query
 // positions by default, or buckets by near leaf), so the lanes of a wavefront walk similar paths
@@ -96,17 +95,6 @@ constexpr int kGroupMinLeaf = 4 * kGroupRecs;
 #endif
 #ifndef TK_SCAN_LOADS_F64
 #define TK_SCAN_LOADS_F64 4
-#endif
-// Whether the batched kernels' climb also loads the next level's box ahead (on: 24.9 -> 24.5 ms
-// per 256-cloud replay; with the batch occupancy targets the k bucket 16 kernel stays at 127
-// VGPRs without spills).
-#ifndef TK_BATCH_CLIMB_PREFETCH
-#define TK_BATCH_CLIMB_PREFETCH 1
-#endif
-// The same for d > 3, where a box is 2d values (on: d = 8, k = 32, 500K queries 95.9 ms; off:
-// 99.0 ms, with the same registers).
-#ifndef TK_WIDE_CLIMB_PREFETCH
-#define TK_WIDE_CLIMB_PREFETCH 1
 #endif
 // Largest list held in registers (larger k use the LDS-list kernel).
 #ifndef TK_REG_LIST_MAX_K
@@ -535,28 +523,32 @@ __device__ __forceinline__ int axis_of_level(int l) { return l % D; }
 
 // The search of one query; `kb` must be initialised.
 //
-// Besides pp (the reference's projected point, kept exactly as the reference keeps it) each lane
-// carries far_mask, the levels at which the current path took a far child.  Leaves and far sides
-// are also tested against the distance from q to the bounding box of their points.  When the
-// reference would enter a far side whose box distance is >= worst, the lane skips it and applies
-// the only lasting effect the reference's visit would have had: pp[a] = q[a] for the axes of the
-// levels below (the reference always walks the near path down to the leaf-parent level and
-// resets each axis it leaves).
+// Besides pp (the reference's projected point) each lane carries far_mask, the levels at which the
+// current path took a far child.  Leaves and far sides are tested against the distance from q to the
+// bounding box of their points.
 //
-// Climbing: coming back up, a level whose far child is on the path (bit set in far_mask) is
-// simply left (its axis is reset in pp); only levels entered through their near child need a
-// far-side test.  So the climb jumps from one such level to the next with bit scans and
-// handles the far levels in between in one step.
+// Why the climb tests boxes alone, where the reference tests its split bound.  A level that the climb
+// leaves resets pp[axis] = q[axis], whether it was entered through its far child, its far side was
+// skipped or it is the leaf-parent.  So when level j is tested, pp is q on the axes of the path's levels
+// below j and, elsewhere, q or the split plane of a far level above j on the path, beyond which all
+// points below j lie.  The far child's points also lie beyond m_j on its axis.  On every axis the gap
+// from q to the far child's box is therefore at least |pp - q| (|m_j - q| on axis j), and since both
+// sums round one difference per axis and add the squares in axis order, the box distance is never below
+// the bound, rounded values included.  A box distance below worst thus implies a bound below worst: the
+// box decides.  A far side that the reference enters although its box distance is >= worst changes
+// nothing: all its points would be rejected, and the resets that its walk leaves (the axes of the next
+// levels below j) are among those the climb made.  Only at the leaf-parent does the reference's bound
+// round twice ((pp - q) + (m - pp), pp not yet set to m), which can exceed the box distance by an ulp;
+// there the reference's own test is kept.  The same holds for the lower-index policy's split bound,
+// which rounds once at every level; that policy needs no pp at all.
+// (Against the form that tested the split bound first wherever pp differed from q: plain workload,
+// 16M queries, k = 16, 7.62 ms a query step against 7.82; k = 8, 5.93 against 6.12; lower-index policy,
+// 8M queries, 4.50 against 4.71; d = 8, k = 32, 100K queries of 500K points, 24.1 against 29.1.)
+//
+// Climbing: a level whose far child is on the path (bit set in far_mask) is simply left; the climb jumps
+// from one level entered through its near child to the next with bit scans.
 // Lane state of one search: q, pp, the k-list, far_mask, node, level.  They are kept as
 // separate variables of the kernel (not one aggregate), so that each can live in registers.
-
-template <typename T, int D>
-__device__ __forceinline__ bool pp_is_q(const Pt<T, D>& pp, const Pt<T, D>& q) {
-    bool e = true;
-#pragma unroll
-    for (int i = 0; i < D; ++i) e = e && (pp[i] == q[i]);
-    return e;
-}
 
 // Walks the near path from `node` down to the leaf-parent level.
 template <typename T, int D, bool kB>
@@ -656,105 +648,46 @@ __device__ __forceinline__ bool lane_step(const TreeView<T, kB>& tv, const Pt<T,
 #pragma nounroll
         for (int side = 0; side < 2; ++side) {
             const int32_t leaf = side ? far_leaf : near_leaf;
-            const bool looks = side == 0 || (kLower ? lower_split_passes<T, D>(tv, q, pp, a_lp, m, kb.worst())
-                                                    : proj_bound<T, D>(q, pp, a_lp, m) < kb.worst());
+            // (under the lower-index policy the far leaf's box distance, tested next, is never below
+            // its split bound)
+            const bool looks = kLower || side == 0 || proj_bound<T, D>(q, pp, a_lp, m) < kb.worst();
             if (looks && leaf_useful<T, D, kLower>(tv, q, leaf, kb.worst()))
                 scan_leaf_staged<T, D, K, kLower, CH, LD, SB, kGroups>(tv, leaf, q, kb, st_d, st_o);
         }
-        if (level == 0) return true;
-        ax_set(pp, a_lp, qa);
     }
-    int l = level;
+    // Climb: the levels entered through their near child, deepest first; the first whose far child's
+    // box passes is entered.  The box of the next candidate level is loaded while the current one
+    // is tested.  The far child of such a level is the sibling of the path's child one level down.
+    uint32_t near_lv = ((1u << level) - 1u) & ~far_mask;
+    if (!near_lv) return true;
+    int j = 31 - __builtin_clz(near_lv);
+    int32_t c = ((node + 1) >> (level - 1 - j)) - 1;
+    BoxVals<T, D> bx = load_box<T, D>(tv.boxes, tv.box_of(((c - 1) ^ 1) + 1));
     for (;;) {
-        if (pp_is_q<T, D>(pp, q)) {
-            // With pp equal to q the reference's bound for a far side is fl(m - q[a])^2, which the
-            // distance to the far child's box never undercuts (the box lies beyond m on axis a), so
-            // the far side is entered iff that box distance passes, and a skip leaves pp as it is.
-            // The far child of a level entered through its near child is the sibling of the path's
-            // child one level down, so these tests need neither the split nor the axis.
-            uint32_t near_lv = ((1u << l) - 1u) & ~far_mask;
-            if constexpr ((kB && !TK_BATCH_CLIMB_PREFETCH) || (D > 3 && !TK_WIDE_CLIMB_PREFETCH)) {
-                while (near_lv) {
-                    const int j = 31 - __builtin_clz(near_lv);
-                    const int32_t c = ((node + 1) >> (level - 1 - j)) - 1;
-                    const int32_t fc = ((c - 1) ^ 1) + 1;
-                    const T b = aabb_bound<T, D>(tv.boxes, tv.box_of(fc), q);
-                    if (kLower ? lower_passes(b, kb.worst()) : b < kb.worst()) {
-                        ax_set(pp, axis_of_level<D>(j), tv.split_at((c - 1) >> 1));
-                        far_mask = (far_mask & ((1u << j) - 1u)) | (1u << j);
-                        node = fc;
-                        level = j + 1;
-                        lane_descend<T, D>(tv, q, node, level);
-                        return false;
-                    }
-                    near_lv ^= 1u << j;
-                }
-                return true;
-            }
-            // The box of the next candidate level is loaded while the current one is tested.
-            if (!near_lv) return true;
-            int j = 31 - __builtin_clz(near_lv);
-            int32_t c = ((node + 1) >> (level - 1 - j)) - 1;
-            BoxVals<T, D> bx = load_box<T, D>(tv.boxes, tv.box_of(((c - 1) ^ 1) + 1));
-            for (;;) {
-                const uint32_t rest = near_lv ^ (1u << j);
-                const int j2 = rest ? 31 - __builtin_clz(rest) : j;
-                const int32_t c2 = ((node + 1) >> (level - 1 - j2)) - 1;
-                const BoxVals<T, D> bx2 = load_box<T, D>(tv.boxes, tv.box_of(((c2 - 1) ^ 1) + 1));
-                const T b = box_dist<T, D>(bx, q);
-                if (kLower ? lower_passes(b, kb.worst()) : b < kb.worst()) {
-                    ax_set(pp, axis_of_level<D>(j), tv.split_at((c - 1) >> 1));
-                    far_mask = (far_mask & ((1u << j) - 1u)) | (1u << j);
-                    node = ((c - 1) ^ 1) + 1;
-                    level = j + 1;
-                    lane_descend<T, D>(tv, q, node, level);
-                    return false;
-                }
-                if (!rest) return true;
-                near_lv = rest;
-                j = j2;
-                c = c2;
-                bx = bx2;
-            }
-        }
-        const uint32_t below = (1u << l) - 1u;
-        const uint32_t near_lv = below & ~far_mask;
-        const int j = near_lv ? 31 - __builtin_clz(near_lv) : -1;
-        const uint32_t popped = far_mask & below & ~(j >= 0 ? ((2u << j) - 1u) : 0u);
-        if (popped) {
-            far_mask &= ~popped;
+        const uint32_t rest = near_lv ^ (1u << j);
+        const int j2 = rest ? 31 - __builtin_clz(rest) : j;
+        const int32_t c2 = ((node + 1) >> (level - 1 - j2)) - 1;
+        const BoxVals<T, D> bx2 = load_box<T, D>(tv.boxes, tv.box_of(((c2 - 1) ^ 1) + 1));
+        const T b = box_dist<T, D>(bx, q);
+        if (kLower ? lower_passes(b, kb.worst()) : b < kb.worst()) {
+            if constexpr (!kLower) {
+                // the levels left on the way up reset pp on their axes; level j's far side sets its own
+                const uint32_t left = ((1u << L) - 1u) & ~((2u << j) - 1u);
 #pragma unroll
-            for (int ax = 0; ax < D; ++ax)
-                if (popped & axis_levels<D>(ax)) pp[ax] = q[ax];
-        }
-        if (j < 0) return true;
-        const int32_t nj = ((node + 1) >> (level - j)) - 1;
-        const int aj = axis_of_level<D>(j);
-        const T mj = tv.split_at(nj);
-        const T qj = ax_get(q, aj);
-        const int32_t far_child = 2 * nj + (qj < mj ? 2 : 1);
-        ax_set(pp, aj, mj);
-        const int f = far_side<T, D, kLower>(tv, q, pp, aj, mj, far_child, kb.worst());
-        if (f == 1) {
-            far_mask |= 1u << j;
-            node = far_child;
+                for (int ax = 0; ax < D; ++ax) pp[ax] = (left & axis_levels<D>(ax)) ? q[ax] : pp[ax];
+                ax_set(pp, axis_of_level<D>(j), tv.split_at((c - 1) >> 1));
+            }
+            far_mask = (far_mask & ((1u << j) - 1u)) | (1u << j);
+            node = ((c - 1) ^ 1) + 1;
             level = j + 1;
             lane_descend<T, D>(tv, q, node, level);
             return false;
         }
-        if (f == 2) {
-            // the reference's pass over this side resets pp on the axes of the next
-            // min(D, L-1-j) levels
-            const int nlev = min(D, L - 1 - j);
-#pragma unroll
-            for (int i = 0; i < D; ++i) {
-                const int off = (i - aj - 1 + 2 * D) % D;
-                if (off < nlev) pp[i] = q[i];
-            }
-        }
-        ax_set(pp, aj, qj);
-        if (j == 0) return true;
-        l = j;
+        if (!rest) return true;
+        near_lv = rest;
+        j = j2;
+        c = c2;
+        bx = bx2;
     }
 }
 
