@@ -48,8 +48,9 @@ enum { TK_TIE_REFERENCE = 0, TK_TIE_LOWER_INDEX = 1 };
 /* Query presort before the traversal, so that the lanes of a wavefront get nearby queries:
  * TK_PRESORT_MORTON orders queries along a space-filling curve over a grid on the queries'
  * bounding box (the Hilbert curve for d <= 3, the Morton code for d = 8; the name is kept),
- * TK_PRESORT_LEAF by the tree leaf they fall into; AUTO = MORTON (LEAF at d = 8) from 4096 queries up.  The
- * presort changes the order of work only, never the results. */
+ * TK_PRESORT_LEAF by the tree leaf they fall into; AUTO = MORTON (LEAF at d = 8) in calls large enough
+ * that the search gains more than the sort costs, never below 4096 queries.  The presort changes the order
+ * of work only, never the results. */
 enum { TK_PRESORT_AUTO = -1, TK_PRESORT_OFF = 0, TK_PRESORT_MORTON = 1, TK_PRESORT_LEAF = 2 };
 
 /* Thread-local message of the last failure on this thread. */
@@ -131,6 +132,13 @@ int tk_tree_info(const tk_tree* tree, int32_t out[6]);
 int tk_tree_variant_info(int variant, int32_t out[3], int* count);
 int tk_tree_set_variant(tk_tree* tree, int variant);
 int tk_tree_get_variant(const tk_tree* tree, int* variant);
+
+/* Lanes per query of the tree's later GPU searches (no counterpart in the reference, whose kernel
+ * gives every query a fixed number of threads, src/kdtree_g.cu:281-283): 0 (the default) = chosen from
+ * the call's size, k, dims and dtype; 1 = one lane per query (d <= 3, k <= 32); 4 (d <= 3, k <= 8),
+ * 8 (d <= 3, k <= 16) or 16 lanes share a query.  A choice that is not prebuilt for a search is
+ * ignored by it.  Results never depend on it. */
+int tk_tree_set_lanes(tk_tree* tree, int lanes);
 
 /* The list of the tree's lower-index float GPU searches with k in 5..32 (no counterpart in the
  * reference, whose GPU kernel keeps one LDS list, src/kdtree_g.cu:285-407): mode 0 = chosen at

@@ -229,6 +229,15 @@ int tk_tree_get_variant(const tk_tree* tree, int* variant) {
     return guarded([&] { *variant = tree_of(tree).variant; });
 }
 
+int tk_tree_set_lanes(tk_tree* tree, int lanes) {
+    return guarded([&] {
+        if (!tree || !tree->t) throw std::runtime_error("null tree handle");
+        if (lanes != 0 && lanes != 1 && lanes != 4 && lanes != 8 && lanes != 16)
+            throw std::runtime_error("lanes per query must be 0, 1, 4, 8 or 16");
+        tree->t->lanes = lanes;
+    });
+}
+
 int tk_tree_set_lower_list(tk_tree* tree, int mode) {
     return guarded([&] {
         if (!tree || !tree->t) throw std::runtime_error("null tree handle");

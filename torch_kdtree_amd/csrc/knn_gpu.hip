@@ -493,6 +493,42 @@ void exclusive_scan_i32(const int32_t* in, int32_t n, int32_t* sums, int32_t* ou
     TK_HIP_CHECK(hipGetLastError());
 }
 
+// Lanes per query, measured on MI355X (float d = 3 unless said; times are whole queries without a
+// presort against one lane per query with it):
+// * k > 32 and d = 8: 16 at every size.  One lane's list does not fit its registers (100K queries, k = 100:
+//   0.99 ms; 19.3 ms with one lane's list in LDS), and at d = 8 the walks of 64 lanes part (500K
+//   queries, k = 32: 23.6 against 45.1 ms; 2M queries, k = 1: 23.5 against 32.9).
+// * few queries leave the chip idle with one lane each, and a search is then one chain of
+//   dependent loads, which more lanes shorten: k = 8, cloud of 100K points, 16 / 8 / 4 / 1 lanes:
+//   1,000 queries 19 / 25 / 37 / 100 us; 10,000 22 / 26 / 36 / 180; 65,537 64 / 54 / 54 / 197;
+//   300,000 232 / 186 / 167 / 274; 1M 695 / 550 / 476 / 461.  At k = 16: 300,000 306 / 261 / - / 356,
+//   1M 931 / 804 / - / 621; at k = 32: 300,000 525 / - / - / 616, 1M 1,657 / - / - / 1,209.
+//   Clustered clouds favour the groups longer (1M points, k = 16, 1M queries: 1,110 with 8 lanes
+//   against 1,197), uniform ones less.
+// * d = 1 and 2: 4 lanes longer (d = 2, k = 8, 1M queries: 253 against 289 us; 8M: 1,938 against 1,441).
+// * doubles: a lane's list takes twice the registers, so the groups hold longer (500K points N(0,1),
+//   500K queries, presorted: k = 1 0.42 against 0.53 ms, k = 16 0.88 against 1.43, k = 32 1.45 against
+//   2.28; uniform, 2M queries, k = 16: 2.11 against 1.96).
+// * trees of big leaves (record-group boxes), k <= 8: 4 lanes, presorted, at every larger size (4M points
+//   at depth 13, k = 8: 4M queries 3.48 against 3.92 ms, 16M 11.7 against 11.9).
+int search_lanes(const Tree& t, int64_t nq, int k) {
+    const auto prebuilt = [&](int lanes) {
+        return lanes == 16 || (t.dims <= 3 && (lanes == 1 ? k <= 32 : lanes == 4 ? k <= 8 : k <= 16));
+    };
+    if (t.lanes && prebuilt(t.lanes)) return t.lanes;
+    if (t.dims == 8 || k > 32) return 16;
+    if (t.dtype == kF64) {
+        if (nq > 1500000) return 1;
+        return k > 16 || nq <= 150000 ? 16 : 8;
+    }
+    if (nq <= 24000) return 16;
+    if (k > 16) return nq <= 400000 ? 16 : 1;
+    if (k > 8) return nq <= 500000 ? 8 : 1;
+    if (nq <= 100000) return 8;
+    if (nq <= (t.dims <= 2 ? 1500000 : 700000)) return 4;
+    return t.dev && t.dev->group_boxes ? 4 : 1;
+}
+
 namespace {
 
 constexpr int64_t kPresortMinQueries = 4096;
@@ -500,13 +536,25 @@ constexpr int kMaxBucketBits = 22;
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-int presort_mode(const Tree& t, int64_t nq, const QueryOpts& o) {
+// The presort of a call.  Asked for by name it always runs.  Auto: only from kPresortMinQueries queries,
+// and only where the search gains more than the sort costs.  One lane per query needs the order to
+// keep its wavefront's walks together.  Groups do not, and gain only cache hits: at d = 8 (500K queries,
+// k = 32) 27.4 -> 23.6 ms, equal at 100K; for lists beyond 32 equal at 100K queries and 7.6 -> 6.4 ms at
+// 1M; at d <= 3 and 300K queries a loss (k = 16, clustered cloud of 1M points: 0.41 -> 0.46 ms), at
+// 500K doubles a gain (k = 16: 0.93 -> 0.88 ms).
+// The order: the space-filling curve at d <= 3; the near-leaf order at d = 8, where the curve over a
+// 3-bit-per-axis grid groups queries more coarsely.
+int presort_mode(const Tree& t, int64_t nq, int k, const QueryOpts& o) {
     if (nq <= 0) return kPresortOff;
-    // auto: the space-filling curve at d <= 3; the near-leaf order at d = 8, where the curve over a
-    // 3-bit-per-axis grid groups queries more coarsely (d8_mixture, 2M queries, k = 32, depth 16:
-    // 222 ms per query step against 231 ms, and 246 ms without a presort)
-    if (o.presort == kPresortAuto)
-        return (nq >= kPresortMinQueries && t.levels > 1) ? (t.dims == 8 ? kPresortLeaf : kPresortMorton) : kPresortOff;
+    if (o.presort == kPresortAuto) {
+        if (nq < kPresortMinQueries || t.levels <= 1) return kPresortOff;
+        const bool exact = o.tie != kTieLowerIndex && !t.finite;
+        if (!exact && search_lanes(t, nq, k) > 1) {
+            const int64_t from = t.dims == 8 ? 65536 : k > 32 ? 131072 : t.dtype == kF64 ? 400000 : 600000;
+            if (nq < from) return kPresortOff;
+        }
+        return t.dims == 8 ? kPresortLeaf : kPresortMorton;
+    }
     if (o.presort != kPresortOff && o.presort != kPresortMorton && o.presort != kPresortLeaf)
         throw std::runtime_error("unknown presort mode");
     return o.presort;
@@ -585,7 +633,11 @@ constexpr int64_t kQuerySlice = int64_t(1) << 28;
 
 size_t query_gpu_workspace(const Tree& t, int64_t nq, const QueryOpts& o) {
     nq = std::min(nq, kQuerySlice);
-    const int mode = presort_mode(t, nq, o);
+    // (auto: what a call of this size takes if it presorts, which depends on k)
+    const int mode = o.presort != kPresortAuto ? presort_mode(t, nq, 1, o)
+                     : nq < kPresortMinQueries || t.levels <= 1 ? kPresortOff
+                     : t.dims == 8                              ? kPresortLeaf
+                                                                : kPresortMorton;
     if (mode == kPresortOff) return 0;
     return presort_layout(t, nq, mode).total;
 }
@@ -614,7 +666,7 @@ void query_gpu(const Tree& t, const void* queries, int64_t nq, int k, void* dist
     DeviceGuard g(t.dev->device);
     const int32_t* order = nullptr;
     std::unique_ptr<StreamScratch> own;
-    const int mode = presort_mode(t, nq, o);
+    const int mode = presort_mode(t, nq, k, o);
     if (mode != kPresortOff) {
         ProfScope ps("presort", stream);
         const PresortLayout l = presort_layout(t, nq, mode);

@@ -46,7 +46,7 @@ struct QueryOpts {
     int presort = kPresortAuto;
 };
 
-// Workspace (bytes) the query needs for the presort; 0 when no presort runs.
+// Workspace (bytes) that the query's presort may need, whatever k; 0 when none runs.
 size_t query_gpu_workspace(const Tree& t, int64_t nq, const QueryOpts& o);
 
 // dist [nq*k] T, idx [nq*k] int32 structured indices, orig [nq*k] int64 original indices
@@ -77,6 +77,15 @@ constexpr int kNumTreeVariants = (int)(sizeof(kTreeVariants) / sizeof(kTreeVaria
 // (knn_tree_variants.hip); returns false when it is not, and the caller launches variant 0.
 bool launch_tree_variant_f32_d3(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, int kb,
                                 float* dist, int32_t* idx, int64_t* orig, bool lower, int variant, hipStream_t s);
+
+// Lanes per query of a tree search (finite trees, or the lower-index policy): 1 (knn_tree.hpp, d <= 3
+// and k <= 32), 4, 8 or 16 (knn_group.hpp).  Results never depend on it.
+int search_lanes(const Tree& t, int64_t nq, int k);
+// Group searches (knn_group_f32.hip / knn_group_f64.hip).
+void launch_group_search_f32(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, float* dist,
+                             int32_t* idx, int64_t* orig, bool lower, int lanes, hipStream_t s);
+void launch_group_search_f64(const Tree& t, const double* q, int64_t nq, const int32_t* order, int k, double* dist,
+                             int32_t* idx, int64_t* orig, bool lower, int lanes, hipStream_t s);
 
 // Per-dtype kernel launchers (knn_tree_f32.hip / knn_tree_f64.hip).
 void launch_tree_search_f32(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, float* dist,

@@ -96,10 +96,6 @@ constexpr int kGroupMinLeaf = 4 * kGroupRecs;
 #ifndef TK_SCAN_LOADS_F64
 #define TK_SCAN_LOADS_F64 4
 #endif
-// Largest list held in registers (larger k use the LDS-list kernel).
-#ifndef TK_REG_LIST_MAX_K
-#define TK_REG_LIST_MAX_K 32
-#endif
 #ifndef TK_STAGE_CHUNK_WIDE
 #define TK_STAGE_CHUNK_WIDE 4
 #endif
@@ -112,7 +108,7 @@ constexpr int kGroupMinLeaf = 4 * kGroupRecs;
 //     64-bit keyed lists (lists of at most 4; with that list at k = 16, chunks of 4 at 7 waves had
 //     been best: 72 VGPRs and 16 bytes of spills, 9.75 ms; with chunks of 8, 92 VGPRs at 5 waves,
 //     10.62 ms).
-// Other kernels: see TK_F64_WAVES and TK_WIDE_WAVES below, no target for the rest.
+// Other kernels: see TK_F64_WAVES below, no target for the rest.
 // TK_WAVES_PER_EU overrides every target (0 = no target anywhere).
 #ifndef TK_WAVES_PER_EU
 #define TK_WAVES_PER_EU -1
@@ -129,13 +125,9 @@ constexpr int kGroupMinLeaf = 4 * kGroupRecs;
 #define TK_LOWER_TIE_LIST 1
 #endif
 // Double, d = 3, k = 16: no target (119 VGPRs, 4 waves; a 5-wave target spills 48 bytes, and a
-// 4-wave one measured neutral).  Float, d = 8, k = 32: 4 waves (128 VGPRs, 12 bytes of spills,
-// 95.9 ms per 500K queries against 99.1 ms at 3 waves and 133 VGPRs).
+// 4-wave one measured neutral).
 #ifndef TK_F64_WAVES
 #define TK_F64_WAVES 0
-#endif
-#ifndef TK_WIDE_WAVES
-#define TK_WIDE_WAVES 4
 #endif
 // kTie: the lower-index search keeps a KBestTie list (TreeList).
 template <typename T, int D, int K, bool kLower, bool kTie = false>
@@ -144,8 +136,7 @@ struct TreeOccupancy {
         TK_WAVES_PER_EU >= 0 ? TK_WAVES_PER_EU
         : (sizeof(T) == 4 && D <= 3 && K <= 16) ? (kLower && !kTie ? TK_F32_LOWER_WAVES : TK_F32_WAVES)
         : (sizeof(T) == 8 && D <= 3 && K == 16 && !kLower) ? TK_F64_WAVES
-        : (sizeof(T) == 4 && D == 8 && K == 32 && (!kLower || kTie)) ? TK_WIDE_WAVES
-                                                                     : 0;
+                                                           : 0;
 };
 #define TK_TREE_OCCUPANCY(T, D, K, L, TIE) __attribute__((amdgpu_waves_per_eu(TreeOccupancy<T, D, K, L, TIE>::kWaves > 0 ? TreeOccupancy<T, D, K, L, TIE>::kWaves : 1)))
 // The same for the batched search kernels (more live state per lane: the cloud's offsets).
@@ -174,60 +165,8 @@ struct BatchOccupancy {
 constexpr int kTreeBlock = TK_TREE_BLOCK;
 constexpr int kTreeBlockStride = kTreeBlock;
 
-// k-best list held in LDS for k beyond the register buckets: slot j of lane t lives at
-// base[j * blockDim + t] (consecutive lanes hit consecutive banks).
-template <typename T, bool kLower>
-struct KBestLds {
-    T* d;
-    int32_t* s;
-    int32_t* o;
-    int k;
-    int stride;
-    T w;        // cached worst distance
-    int32_t wo; // cached worst original index
-
-    // empty slots: (+inf, structured index s0, original index 0); see KBest for why 0
-    __device__ __forceinline__ void init(int32_t s0) {
-        for (int j = 0; j < k; ++j) {
-            d[j * stride] = pos_inf<T>();
-            s[j * stride] = s0;
-            if constexpr (kLower) o[j * stride] = 0;
-        }
-        w = pos_inf<T>();
-        wo = 0;
-    }
-    __device__ __forceinline__ T worst() const { return w; }
-    __device__ __forceinline__ bool accepts(T dist, int32_t orig) const {
-        if constexpr (kLower)
-            return dist < w || (dist == w && orig < wo);
-        else
-            return dist < w;
-    }
-    __device__ __forceinline__ bool after(int j, T dist, int32_t orig) const {
-        const T dj = d[j * stride];
-        if constexpr (kLower)
-            return dj > dist || (dj == dist && o[j * stride] > orig);
-        else
-            return dj > dist;
-    }
-    __device__ __forceinline__ void insert(T dist, int32_t sidx, int32_t orig) {
-        int j = k - 1;
-        while (j > 0 && after(j - 1, dist, orig)) {
-            d[j * stride] = d[(j - 1) * stride];
-            s[j * stride] = s[(j - 1) * stride];
-            if constexpr (kLower) o[j * stride] = o[(j - 1) * stride];
-            --j;
-        }
-        d[j * stride] = dist;
-        s[j * stride] = sidx;
-        if constexpr (kLower) o[j * stride] = orig;
-        w = d[(k - 1) * stride];
-        if constexpr (kLower) wo = o[(k - 1) * stride];
-    }
-};
-
 // The reference's own list, for trees with non-finite values under the reference tie policy.  Held
-// in LDS like KBestLds.  A candidate is rejected only when d >= worst (src/nndistance.hpp:77) and
+// in LDS: slot j of lane t lives at base[j * blockDim + t] (consecutive lanes hit consecutive banks).  A candidate is rejected only when d >= worst (src/nndistance.hpp:77) and
 // is placed by the reference's binary search (upperBound, src/nndistance.hpp:41-60), so a NaN
 // distance is taken and goes to the front, and the search's path through a list holding NaN
 // entries decides where each later value lands; a NaN reaching the last slot makes worst NaN,
@@ -691,8 +630,8 @@ __device__ __forceinline__ bool lane_step(const TreeView<T, kB>& tv, const Pt<T,
     }
 }
 
-// Reference-order search with a generic list (used with the LDS list for large k): the same walk
-// as lane_start/lane_step, one node at a time.  kBoxes false: no point-box tests, so the walk is
+// Reference-order search with a generic list: the same walk as lane_start/lane_step, one node at a
+// time (re-searches, and trees with non-finite values).  kBoxes false: no point-box tests, so the walk is
 // the reference's own (src/kdtree.cpp:16-110), step for step (trees with non-finite values).
 template <typename T, int D, bool kLower, bool kBoxes = true, typename List, bool kB>
 __device__ __forceinline__ void knn_search_one(const TreeView<T, kB>& tv, const Pt<T, D>& q, List& kb) {
@@ -1074,43 +1013,6 @@ __global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(WAVES > 0 ?
 
 constexpr int kLdsBlock = 64;
 
-template <typename T, int D, bool kLower>
-__global__ __launch_bounds__(kLdsBlock) void knn_tree_lds_kernel(TreeView<T> tv, const T* __restrict__ queries,
-                                                                  int64_t nq, const int32_t* __restrict__ order,
-                                                                  int k, T* __restrict__ out_d,
-                                                                  int32_t* __restrict__ out_i,
-                                                                  int64_t* __restrict__ out_o) {
-    extern __shared__ unsigned char smem[];
-    const int64_t t = xcd_tile(blockIdx.x, gridDim.x) * kLdsBlock + threadIdx.x;
-    if (t >= nq) return;
-    const int64_t qi = order ? (int64_t)order[t] : t;
-    T* sd = reinterpret_cast<T*>(smem);
-    int32_t* ss = reinterpret_cast<int32_t*>(sd + (size_t)k * kLdsBlock);
-    int32_t* so = ss + (size_t)k * kLdsBlock;
-    KBestLds<T, kLower> kb{sd + threadIdx.x, ss + threadIdx.x, so + threadIdx.x, k, kLdsBlock, T(0), 0};
-    kb.init(kLower ? tv.inv_shuffled[0] : 0);
-    Pt<T, D> q;
-    load_query<T, D>(queries, qi, q);
-    if (has_nan<T, D>(q)) {
-        // the reference policy's NaN result (nan_fill); the lower-index list stays empty
-        if constexpr (!kLower) {
-            int32_t beg = 0, end = 0;
-            descent_leaf<T, D>(tv, q, beg, end);
-            for (int c = 0; c < k && end - 1 - c >= beg; ++c) {
-                kb.d[c * kLdsBlock] = sq_dist<T, D>(q, load_rec<T, D>(tv.recs, end - 1 - c).c);
-                kb.s[c * kLdsBlock] = end - 1 - c;
-            }
-        }
-    } else {
-        knn_search_one<T, D, kLower>(tv, q, kb);
-    }
-    for (int j = 0; j < k; ++j) {
-        out_d[qi * k + j] = kb.d[j * kLdsBlock];
-        out_i[qi * k + j] = kb.s[j * kLdsBlock];
-        if (out_o) out_o[qi * k + j] = kLower ? kb.o[j * kLdsBlock] : tv.shuffled[kb.s[j * kLdsBlock]];
-    }
-}
-
 // Reference tie policy on a tree with a non-finite coordinate or split value: the reference's walk
 // step for step (no point boxes) with the reference's list (KBestExact), one lane per query.
 // Queries with a NaN coordinate need no special case here.
@@ -1140,10 +1042,6 @@ __global__ __launch_bounds__(kLdsBlock) void knn_tree_exact_kernel(TreeView<T> t
 }
 
 inline size_t exact_list_bytes(int k, size_t tsize) { return (size_t)k * kLdsBlock * (tsize + 4); }
-
-inline size_t lds_list_bytes(int k, size_t tsize, bool lower) {
-    return (size_t)k * kLdsBlock * (tsize + 4 + (lower ? 4 : 0));
-}
 
 // ---------------------------------------------------------------------------------------------
 // Query presorts.  Each presort kernel writes one integer key per query and the query's row; a

@@ -7,7 +7,15 @@ namespace tk {
 
 void launch_tree_search_f64(const Tree& t, const double* q, int64_t nq, const int32_t* order, int k, double* dist,
                             int32_t* idx, int64_t* orig, int tie, hipStream_t s) {
-    launch_tree_search_t<double>(t, q, nq, order, k, dist, idx, orig, tie, s);
+    if (tie != kTieLowerIndex && !t.finite) {
+        launch_exact_search_t<double>(t, q, nq, order, k, dist, idx, orig, s);
+        return;
+    }
+    const int lanes = search_lanes(t, nq, k);
+    if (lanes > 1)
+        launch_group_search_f64(t, q, nq, order, k, dist, idx, orig, tie == kTieLowerIndex, lanes, s);
+    else
+        launch_lane_search_t<double>(t, q, nq, order, k, dist, idx, orig, tie, s);
 }
 
 void launch_leaf_bucket_f64(const Tree& t, const double* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,

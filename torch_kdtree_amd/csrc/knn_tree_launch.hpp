@@ -41,7 +41,6 @@ void launch_tree_td(const TreeView<T>& tv, const T* q, int64_t nq, const int32_t
     const dim3 block(kTreeBlock);
     int kb = 1;
     while (kb < k) kb <<= 1;
-    if (kb > TK_REG_LIST_MAX_K) kb = 0;  // the LDS-list kernel
 #define TK_LAUNCH_K(KK)                                                                                         \
     case KK:                                                                                                    \
         if (tv.group_boxes)                                                                                     \
@@ -56,14 +55,7 @@ void launch_tree_td(const TreeView<T>& tv, const T* q, int64_t nq, const int32_t
         TK_LAUNCH_K(8)
         TK_LAUNCH_K(16)
         TK_LAUNCH_K(32)
-        default: {
-            const size_t shmem = lds_list_bytes(k, sizeof(T), kLower);
-            const void* fn = reinterpret_cast<const void*>(&knn_tree_lds_kernel<T, D, kLower>);
-            if (shmem > 65536)
-                TK_HIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
-            hipLaunchKernelGGL((knn_tree_lds_kernel<T, D, kLower>), dim3((unsigned)((nq + kLdsBlock - 1) / kLdsBlock)),
-                               dim3(kLdsBlock), shmem, s, tv, q, nq, order, k, dist, idx, orig);
-        }
+        default: throw std::runtime_error("list of more than 32 entries in a one-lane search");
     }
 #undef TK_LAUNCH_K
     TK_HIP_CHECK(hipGetLastError());
@@ -81,27 +73,38 @@ void launch_tree_exact(const TreeView<T>& tv, const T* q, int64_t nq, const int3
     TK_HIP_CHECK(hipGetLastError());
 }
 
+// The search with one lane per query: d <= 3, k <= 32 (search_lanes picks it).
 template <typename T>
-void launch_tree_search_t(const Tree& t, const T* q, int64_t nq, const int32_t* order, int k, T* dist, int32_t* idx,
+void launch_lane_search_t(const Tree& t, const T* q, int64_t nq, const int32_t* order, int k, T* dist, int32_t* idx,
                           int64_t* orig, int tie, hipStream_t s) {
     const TreeView<T> tv = tree_view<T>(t);
-#define TK_DIMS(DD)                                                            \
-    case DD:                                                                   \
-        if (tie != kTieLowerIndex && !t.finite)                                \
-            launch_tree_exact<T, DD>(tv, q, nq, order, k, dist, idx, orig, s); \
-        else if (tie == kTieLowerIndex)                                        \
+#define TK_DIMS(DD)                                                               \
+    case DD:                                                                      \
+        if (tie == kTieLowerIndex)                                                \
             launch_tree_td<T, DD, true>(tv, q, nq, order, k, dist, idx, orig, s); \
-        else                                                                   \
+        else                                                                      \
             launch_tree_td<T, DD, false>(tv, q, nq, order, k, dist, idx, orig, s); \
         break;
     switch (t.dims) {
         TK_DIMS(1)
         TK_DIMS(2)
         TK_DIMS(3)
-        TK_DIMS(8)
-        default: throw std::runtime_error("unsupported dims");
+        default: throw std::runtime_error("unsupported dims in a one-lane search");
     }
 #undef TK_DIMS
+}
+
+template <typename T>
+void launch_exact_search_t(const Tree& t, const T* q, int64_t nq, const int32_t* order, int k, T* dist, int32_t* idx,
+                           int64_t* orig, hipStream_t s) {
+    const TreeView<T> tv = tree_view<T>(t);
+    switch (t.dims) {
+        case 1: launch_tree_exact<T, 1>(tv, q, nq, order, k, dist, idx, orig, s); break;
+        case 2: launch_tree_exact<T, 2>(tv, q, nq, order, k, dist, idx, orig, s); break;
+        case 3: launch_tree_exact<T, 3>(tv, q, nq, order, k, dist, idx, orig, s); break;
+        case 8: launch_tree_exact<T, 8>(tv, q, nq, order, k, dist, idx, orig, s); break;
+        default: throw std::runtime_error("unsupported dims");
+    }
 }
 
 #ifndef TK_HILBERT_MAX_D

@@ -91,6 +91,7 @@ struct KDTree {
     // Every coordinate and split value finite (otherwise GPU queries under the reference tie
     // policy run the reference's own steps, without point-box pruning).
     void set_variant(int v) { check(tk_tree_set_variant(tree, v)); }
+    void set_lanes(int lanes) { check(tk_tree_set_lanes(tree, lanes)); }
     void set_lower_list(int mode) { check(tk_tree_set_lower_list(tree, mode)); }
     py::tuple get_lower_list() const {
         int32_t out[2] = {0, 0};
@@ -355,6 +356,8 @@ void bind_tree(py::module_& m, const char* name) {
         .def("set_variant", &C::set_variant, py::arg("variant"),
              "Launch variant of later GPU queries (see torch_knn.tree_variants())")
         .def("get_variant", &C::get_variant)
+        .def("set_lanes", &C::set_lanes, py::arg("lanes"),
+             "Lanes per query of later GPU queries: 0 = chosen per call, 1, 4, 8 or 16 where prebuilt")
         .def("set_lower_list", &C::set_lower_list, py::arg("mode"),
              "List of later lower-index GPU queries: 0 = chosen from the cloud, 1 = tie-flagged, 2 = (distance, index)")
         .def("get_lower_list", &C::get_lower_list, "(mode, whether mode 0 takes the (distance, index) list)")

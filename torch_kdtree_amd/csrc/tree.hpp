@@ -51,6 +51,9 @@ struct Tree {
     // (tie_prone), 1 = the reference policy's list with tie flags, each unsure lane searched again,
     // 2 = the list keyed by (distance, original index) from the start.  Results never depend on it.
     int lower_list = 0;
+    // Lanes per query of the GPU searches (0 = search_lanes' rule, else 1, 4, 8 or 16 where that form
+    // is prebuilt for the search).  Results never depend on it.
+    int lanes = 0;
     // Set at upload: exact distance ties look common among this cloud's neighbours (duplicated
     // points, coordinates on few distinct values), or the tree holds a non-finite value.
     bool tie_prone = false;
