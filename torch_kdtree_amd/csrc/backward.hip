@@ -217,7 +217,7 @@ constexpr int64_t kMaxPairs = int64_t(1) << 28;
 int64_t slice_queries(int64_t nq, int k) { return std::min<int64_t>(nq, kMaxPairs / k); }
 
 struct BwLayout {
-    size_t qkey, qrow, qkey_s, order, run_start, run_end, bbox, q_sorted, g_sorted, keys, vals, keys_s, vals_s,
+    size_t qkey, qkey_s, order, run_start, run_end, box, q_sorted, g_sorted, keys, vals, keys_s, vals_s,
         ref_s, temp, temp_bytes, total;
 };
 
@@ -230,12 +230,11 @@ BwLayout bw_layout(int64_t nq, int32_t n, int k, int dims, int dtype, bool struc
     BwLayout l{};
     size_t off = 0;
     l.qkey = off; off += a256(4 * (size_t)nq);
-    l.qrow = off; off += a256(4 * (size_t)nq);
     l.qkey_s = off; off += a256(4 * (size_t)nq);
     l.order = off; off += a256(4 * (size_t)nq);
     l.run_start = off; off += a256(4 * (size_t)n);
     l.run_end = off; off += a256(4 * (size_t)n);
-    l.bbox = off; off += a256(16 * (size_t)dims);
+    l.box = off; off += a256(box_scratch_bytes(dims, dtype));
     l.q_sorted = off; off += a256(ts * (size_t)dims * (size_t)sq);
     l.g_sorted = off; off += a256(ts * (size_t)m);
     l.keys = off; off += a256(4 * (size_t)m);
@@ -285,17 +284,16 @@ void backward_typed(const T* q, const T* ref, int64_t nq, int32_t n, int k, cons
     }
     // canonical query order
     uint32_t* qkey = reinterpret_cast<uint32_t*>(ws + l.qkey);
-    uint32_t* qrow = reinterpret_cast<uint32_t*>(ws + l.qrow);
     uint32_t* qkey_s = reinterpret_cast<uint32_t*>(ws + l.qkey_s);
     uint32_t* order = reinterpret_cast<uint32_t*>(ws + l.order);
-    auto* box = reinterpret_cast<OrderedT<T>*>(ws + l.bbox);
-    init_bbox(box, sizeof(T) == 4 ? kF32 : kF64, D, s);
-    const unsigned box_blocks = (unsigned)std::min<int64_t>(1024, ((int64_t)n + kBoxBlock - 1) / kBoxBlock);
-    hipLaunchKernelGGL((bbox_kernel<T, D>), dim3(box_blocks), dim3(kBoxBlock), 0, s, ref, (int64_t)n, box);
+    T* box = reinterpret_cast<T*>(ws + l.box);
+    const int parts = box_parts(n);
+    hipLaunchKernelGGL((bbox_kernel<T, D>), dim3(parts), dim3(kBoxBlock), 0, s, ref, (int64_t)n, box);
     const int bits = canonical_morton_bits(nq, D);
-    hipLaunchKernelGGL((morton_bucket_kernel<T, D>), qgrid, dim3(256), 0, s, q, nq, box, bits, qkey, qrow, false);
+    hipLaunchKernelGGL((morton_bucket_kernel<T, D>), dim3(key_blocks(nq)), dim3(kBoxBlock), 0, s, q, nq, box, parts,
+                       bits, qkey, false);
     TK_HIP_CHECK(hipGetLastError());
-    radix_sort_pairs(qkey, qrow, qkey_s, order, nq, bits * D, ws + l.temp, l.temp_bytes, s);
+    radix_sort_pairs(qkey, nullptr, qkey_s, order, nq, bits * D, ws + l.temp, l.temp_bytes, s);
     // dL/dq, canonical copies and pairs; pairs sorted by reference index; dL/dr per reference point
     T* q_sorted = reinterpret_cast<T*>(ws + l.q_sorted);
     T* g_sorted = reinterpret_cast<T*>(ws + l.g_sorted);

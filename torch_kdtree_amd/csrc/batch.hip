@@ -281,7 +281,6 @@ BatchPlan* batch_create(const Tree* const* trees, int n_clouds, const int64_t* n
     const size_t nq = (size_t)p->total_q, no = (size_t)p->total_out;
     dmalloc(&p->qcloud, 4 * nq);
     dmalloc(&p->key, 4 * nq);
-    dmalloc(&p->row, 4 * nq);
     dmalloc(&p->key_s, 4 * nq);
     dmalloc(&p->order, 4 * nq);
     dmalloc(&p->rank, 4 * nq);
@@ -317,7 +316,6 @@ void batch_free(BatchPlan* p) noexcept {
     dfree(p->d_clouds);
     dfree(p->qcloud);
     dfree(p->key);
-    dfree(p->row);
     dfree(p->key_s);
     dfree(p->order);
     dfree(p->rank);

@@ -72,7 +72,6 @@ struct BatchPlan {
     int32_t* rec_cloud = nullptr;  // [total_ref] cloud of each record
     // scratch
     uint32_t* key = nullptr;    // [total_q] presort keys
-    uint32_t* row = nullptr;    // [total_q] query rows
     uint32_t* key_s = nullptr;  // [total_q] sorted keys
     int32_t* order = nullptr;   // [total_q] query rows in sorted order
     uint32_t* rank = nullptr;   // [total_q] position of each query row in the sorted order

@@ -33,8 +33,7 @@ __global__ __launch_bounds__(kBatchBlock) void batch_bucket_kernel(const unsigne
                                                                     const CloudDesc* __restrict__ clouds,
                                                                     const int32_t* __restrict__ qcloud,
                                                                     const T* __restrict__ queries, int64_t total_q,
-                                                                    uint32_t* __restrict__ key,
-                                                                    uint32_t* __restrict__ row) {
+                                                                    uint32_t* __restrict__ key) {
     const int64_t i = (int64_t)blockIdx.x * kBatchBlock + threadIdx.x;
     if (i >= total_q) return;
     const CloudDesc& cd = clouds[qcloud[i]];
@@ -47,7 +46,6 @@ __global__ __launch_bounds__(kBatchBlock) void batch_bucket_kernel(const unsigne
         hi[a] = (float)box[L::kPad + a];
     }
     key[i] = (uint32_t)cd.bucket_base + morton_cell<T, D>(lo, hi, cd.morton_bits, queries + i * D);
-    row[i] = (uint32_t)i;
 }
 
 // Key of a (record, slot) pair for the dL/dr sort: the arena record position, or, with a tag shift,
@@ -500,7 +498,7 @@ void batch_presort_t(const BatchPlan& p, const T* q, hipStream_t s) {
 #define TK_DIMS(DD)                                                                                                  \
     case DD:                                                                                                         \
         hipLaunchKernelGGL((batch_bucket_kernel<T, DD>), batch_grid(p.total_q), dim3(kBatchBlock), 0, s, p.boxes,   \
-                           p.d_clouds, p.qcloud, q, p.total_q, p.key, p.row);                                        \
+                           p.d_clouds, p.qcloud, q, p.total_q, p.key);                                               \
         break;
     switch (p.dims) {
         TK_DIMS(1)
@@ -511,7 +509,7 @@ void batch_presort_t(const BatchPlan& p, const T* q, hipStream_t s) {
     }
 #undef TK_DIMS
     TK_HIP_CHECK(hipGetLastError());
-    radix_sort_pairs(p.key, p.row, p.key_s, reinterpret_cast<uint32_t*>(p.order), p.total_q, p.key_bits, p.radix_ws,
+    radix_sort_pairs(p.key, nullptr, p.key_s, reinterpret_cast<uint32_t*>(p.order), p.total_q, p.key_bits, p.radix_ws,
                      p.radix_ws_bytes, s);
     hipLaunchKernelGGL(batch_rank_kernel, batch_grid(p.total_q), dim3(kBatchBlock), 0, s, p.order, p.total_q, p.rank);
     TK_HIP_CHECK(hipGetLastError());

@@ -1,4 +1,4 @@
-// GPU tree upload, the leaf-bucket presort (scan + scatter) and the query driver.
+// GPU tree upload and the query driver.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -379,120 +379,8 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 }
 
 // ------------------------------------------------------------------------------------------
-// Scan / scatter kernels for the presort
-// ------------------------------------------------------------------------------------------
-__global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t n, int32_t v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-__device__ __forceinline__ int wave_inclusive_scan(int v) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(v, off, 64);
-        if (lane >= off) v += y;
-    }
-    return v;
-}
-
-// Exclusive scan of n int32 counts (n <= kScanChunk * kScanChunk) in three kernels.
-constexpr int kScanBlock = 1024;
-constexpr int kScanItems = 4;
-constexpr int kScanChunk = kScanBlock * kScanItems;
-
-// Exclusive scan over a block of kScanBlock threads; `total` receives the block sum.
-__device__ __forceinline__ int block_exclusive_scan(int v, int* wsum, int& total) {
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-    constexpr int kWaves = kScanBlock / 64;
-    const int inc = wave_inclusive_scan(v);
-    if (lane == 63) wsum[wid] = inc;
-    __syncthreads();
-    if (wid == 0) {
-        const int ws = lane < kWaves ? wsum[lane] : 0;
-        const int wi = wave_inclusive_scan(ws);
-        if (lane < kWaves) wsum[lane] = wi - ws;
-        if (lane == kWaves - 1) wsum[kWaves] = wi;
-    }
-    __syncthreads();
-    total = wsum[kWaves];
-    const int r = inc - v + wsum[wid];
-    __syncthreads();
-    return r;
-}
-
-__global__ __launch_bounds__(kScanBlock) void scan_block_sums_kernel(const int32_t* __restrict__ in, int32_t n,
-                                                                      int32_t* __restrict__ sums) {
-    __shared__ int wsum[kScanBlock / 64 + 1];
-    const int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * kScanItems;
-    int v = 0;
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j)
-        if (base + j < n) v += in[base + j];
-    int total;
-    (void)block_exclusive_scan(v, wsum, total);
-    if (threadIdx.x == 0) sums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kScanBlock) void scan_sums_kernel(int32_t* __restrict__ sums, int32_t nsums) {
-    __shared__ int wsum[kScanBlock / 64 + 1];
-    const int base = threadIdx.x * kScanItems;
-    int x[kScanItems];
-    int v = 0;
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        x[j] = base + j < nsums ? sums[base + j] : 0;
-        v += x[j];
-    }
-    int total;
-    int run = block_exclusive_scan(v, wsum, total);
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        if (base + j < nsums) sums[base + j] = run;
-        run += x[j];
-    }
-}
-
-__global__ __launch_bounds__(kScanBlock) void scan_apply_kernel(const int32_t* __restrict__ in, int32_t n,
-                                                                 const int32_t* __restrict__ sums,
-                                                                 int32_t* __restrict__ out) {
-    __shared__ int wsum[kScanBlock / 64 + 1];
-    const int64_t base = (int64_t)blockIdx.x * kScanChunk + (int64_t)threadIdx.x * kScanItems;
-    int x[kScanItems];
-    int v = 0;
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        x[j] = base + j < n ? in[base + j] : 0;
-        v += x[j];
-    }
-    int total;
-    int run = block_exclusive_scan(v, wsum, total) + sums[blockIdx.x];
-#pragma unroll
-    for (int j = 0; j < kScanItems; ++j) {
-        if (base + j < n) out[base + j] = run;
-        run += x[j];
-    }
-}
-
-
-// ------------------------------------------------------------------------------------------
 // Query driver
 // ------------------------------------------------------------------------------------------
-int32_t scan_sums_count(int32_t n) { return (n + kScanChunk - 1) / kScanChunk; }
-
-void exclusive_scan_i32(const int32_t* in, int32_t n, int32_t* sums, int32_t* out, hipStream_t stream) {
-    if (n > kScanChunk * kScanChunk) throw std::runtime_error("exclusive scan: too many values");
-    const int32_t nsums = scan_sums_count(n);
-    if (nsums == 0) return;
-    hipLaunchKernelGGL(scan_block_sums_kernel, dim3(nsums), dim3(kScanBlock), 0, stream, in, n, sums);
-    TK_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(kScanBlock), 0, stream, sums, nsums);
-    TK_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(scan_apply_kernel, dim3(nsums), dim3(kScanBlock), 0, stream, in, n, sums, out);
-    TK_HIP_CHECK(hipGetLastError());
-}
-
 // Lanes per query, measured on MI355X (float d = 3 unless said; times are whole queries without a
 // presort against one lane per query with it):
 // * k > 32 and d = 8: 16 at every size.  One lane's list does not fit its registers (100K queries, k = 100:
@@ -563,7 +451,7 @@ int presort_mode(const Tree& t, int64_t nq, int k, const QueryOpts& o) {
 int bucket_shift(const Tree& t) { return std::max(0, t.levels - kMaxBucketBits); }
 
 struct PresortLayout {
-    size_t key, row, key_s, order, bbox, radix, radix_bytes, total;
+    size_t key, key_s, order, box, radix, radix_bytes, total;
     int key_bits;
 };
 
@@ -578,10 +466,9 @@ PresortLayout presort_layout(const Tree& t, int64_t nq, int mode) {
     l.key_bits = mode == kPresortMorton ? bits_for(morton_bucket_count(t.dims)) : bits_for(t.n_leaves >> bucket_shift(t));
     size_t off = 0;
     l.key = off; off += align256(sizeof(int32_t) * (size_t)nq);
-    l.row = off; off += align256(sizeof(int32_t) * (size_t)nq);
     l.key_s = off; off += align256(sizeof(int32_t) * (size_t)nq);
     l.order = off; off += align256(sizeof(int32_t) * (size_t)nq);
-    l.bbox = off; off += align256(2 * 8 * (size_t)t.dims);
+    l.box = off; off += align256(box_scratch_bytes(t.dims, t.dtype));
     l.radix = off;
     l.radix_bytes = radix_sort_workspace(nq);
     off += align256(l.radix_bytes);
@@ -589,29 +476,9 @@ PresortLayout presort_layout(const Tree& t, int64_t nq, int mode) {
     return l;
 }
 
-void check_launch() { TK_HIP_CHECK(hipGetLastError()); }
-
-__global__ void fill_u64_kernel(unsigned long long* __restrict__ p, int n, unsigned long long lo_v,
-                                unsigned long long hi_v, int half) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = i < half ? lo_v : hi_v;
-}
-
 }  // namespace
 
-void init_bbox(void* bbox, int dtype, int dims, hipStream_t stream) {
-    // [min codes (all ones) | max codes (zero)] in the width of T
-    if (dtype == kF32) {
-        hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, stream, static_cast<int32_t*>(bbox), (int64_t)dims,
-                           (int32_t)-1);
-        hipLaunchKernelGGL(fill_i32_kernel, dim3(1), dim3(64), 0, stream, static_cast<int32_t*>(bbox) + dims,
-                           (int64_t)dims, 0);
-    } else {
-        hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(64), 0, stream, static_cast<unsigned long long*>(bbox),
-                           2 * dims, ~0ull, 0ull, dims);
-    }
-    TK_HIP_CHECK(hipGetLastError());
-}
+size_t box_scratch_bytes(int dims, int dtype) { return (size_t)kMaxBoxParts * 2 * (size_t)dims * dtype_size(dtype); }
 
 int canonical_morton_bits(int64_t nq, int dims) {
     int maxb = 0;
@@ -678,22 +545,19 @@ void query_gpu(const Tree& t, const void* queries, int64_t nq, int k, void* dist
             throw std::runtime_error("query workspace too small");
         }
         uint32_t* key = reinterpret_cast<uint32_t*>(ws + l.key);
-        uint32_t* row = reinterpret_cast<uint32_t*>(ws + l.row);
         uint32_t* key_s = reinterpret_cast<uint32_t*>(ws + l.key_s);
         int32_t* ord = reinterpret_cast<int32_t*>(ws + l.order);
-        void* bbox = ws + l.bbox;
         if (mode == kPresortMorton) {
-            init_bbox(bbox, t.dtype, t.dims, stream);
             if (t.dtype == kF32)
-                launch_morton_bucket_f32(t, static_cast<const float*>(queries), nq, bbox, key, row, stream);
+                launch_morton_bucket_f32(t, static_cast<const float*>(queries), nq, ws + l.box, key, stream);
             else
-                launch_morton_bucket_f64(t, static_cast<const double*>(queries), nq, bbox, key, row, stream);
+                launch_morton_bucket_f64(t, static_cast<const double*>(queries), nq, ws + l.box, key, stream);
         } else if (t.dtype == kF32) {
-            launch_leaf_bucket_f32(t, static_cast<const float*>(queries), nq, bucket_shift(t), key, row, stream);
+            launch_leaf_bucket_f32(t, static_cast<const float*>(queries), nq, bucket_shift(t), key, stream);
         } else {
-            launch_leaf_bucket_f64(t, static_cast<const double*>(queries), nq, bucket_shift(t), key, row, stream);
+            launch_leaf_bucket_f64(t, static_cast<const double*>(queries), nq, bucket_shift(t), key, stream);
         }
-        radix_sort_pairs(key, row, key_s, reinterpret_cast<uint32_t*>(ord), nq, l.key_bits, ws + l.radix,
+        radix_sort_pairs(key, nullptr, key_s, reinterpret_cast<uint32_t*>(ord), nq, l.key_bits, ws + l.radix,
                          l.radix_bytes, stream);
         order = ord;
     }

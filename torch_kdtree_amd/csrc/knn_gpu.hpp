@@ -92,17 +92,13 @@ void launch_tree_search_f32(const Tree& t, const float* q, int64_t nq, const int
                             int32_t* idx, int64_t* orig, int tie, hipStream_t s);
 void launch_tree_search_f64(const Tree& t, const double* q, int64_t nq, const int32_t* order, int k, double* dist,
                             int32_t* idx, int64_t* orig, int tie, hipStream_t s);
-void launch_leaf_bucket_f32(const Tree& t, const float* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,
-                            hipStream_t s);
-void launch_leaf_bucket_f64(const Tree& t, const double* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,
-                            hipStream_t s);
-void launch_morton_bucket_f32(const Tree& t, const float* q, int64_t nq, void* bbox, uint32_t* key, uint32_t* row,
-                              hipStream_t s);
-void launch_morton_bucket_f64(const Tree& t, const double* q, int64_t nq, void* bbox, uint32_t* key, uint32_t* row,
-                              hipStream_t s);
+void launch_leaf_bucket_f32(const Tree& t, const float* q, int64_t nq, int shift, uint32_t* key, hipStream_t s);
+void launch_leaf_bucket_f64(const Tree& t, const double* q, int64_t nq, int shift, uint32_t* key, hipStream_t s);
+void launch_morton_bucket_f32(const Tree& t, const float* q, int64_t nq, void* box, uint32_t* key, hipStream_t s);
+void launch_morton_bucket_f64(const Tree& t, const double* q, int64_t nq, void* box, uint32_t* key, hipStream_t s);
+// Bytes of the scratch `box` above (partial bounding boxes).
+size_t box_scratch_bytes(int dims, int dtype);
 int morton_bucket_count(int dims);
-// Sets a 2*dims ordered-integer bounding box to (all ones | zero), the start of a min/max reduction.
-void init_bbox(void* bbox, int dtype, int dims, hipStream_t stream);
 // Bits per axis of the Morton grid of the backward's canonical query order: about 8 queries per
 // cell, at most the grid of the forward presort.
 int canonical_morton_bits(int64_t nq, int dims);
@@ -133,14 +129,9 @@ void knn_backward_structured_gpu(const void* queries, const void* ref, int64_t n
                                  size_t workspace_bytes);
 size_t knn_backward_structured_workspace(int64_t nq, int32_t n, int k, int dims, int dtype);
 
-// Exclusive prefix sum of n int32 values (n <= 2^24) into out; sums needs scan_sums_count(n)
-// int32 of scratch.  Kernels only (no memset, no host synchronisation).
-int32_t scan_sums_count(int32_t n);
-void exclusive_scan_i32(const int32_t* in, int32_t n, int32_t* sums, int32_t* out, hipStream_t stream);
-
 // Stable LSD radix sort of (key, value) pairs of uint32 by the low key_bits bits of the keys
 // (radix_sort.hip).  Reads keys_in / vals_in, writes keys_out / vals_out (distinct from the
-// inputs); workspace of radix_sort_workspace(n) bytes.  Kernels only, so it can be captured in
+// inputs; vals_in null: the values are 0..n-1); workspace of radix_sort_workspace(n) bytes.  Kernels only, so it can be captured in
 // a graph.  n <= 2^28.
 size_t radix_sort_workspace(int64_t n);
 void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out, uint32_t* vals_out,

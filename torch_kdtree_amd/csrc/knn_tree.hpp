@@ -1044,8 +1044,8 @@ __global__ __launch_bounds__(kLdsBlock) void knn_tree_exact_kernel(TreeView<T> t
 inline size_t exact_list_bytes(int k, size_t tsize) { return (size_t)k * kLdsBlock * (tsize + 4); }
 
 // ---------------------------------------------------------------------------------------------
-// Query presorts.  Each presort kernel writes one integer key per query and the query's row; a
-// stable radix sort of (key, row) (radix_sort.hip) then gives the order, so the order is
+// Query presorts.  Each presort kernel writes one integer key per query; a stable radix sort of
+// (key, row) (radix_sort.hip) then gives the order, so the order is
 // deterministic: equal keys keep increasing rows.
 //
 // Leaf keys: each query descends to the leaf on its near side (no pruning); leaves are numbered
@@ -1056,8 +1056,7 @@ constexpr int kPresortBlock = 256;
 template <typename T, int D>
 __global__ __launch_bounds__(kPresortBlock) void leaf_bucket_kernel(TreeView<T> tv, const T* __restrict__ queries,
                                                                      int64_t nq, int shift,
-                                                                     uint32_t* __restrict__ key,
-                                                                     uint32_t* __restrict__ row) {
+                                                                     uint32_t* __restrict__ key) {
     const int64_t i = (int64_t)blockIdx.x * kPresortBlock + threadIdx.x;
     if (i >= nq) return;
     Pt<T, D> q;
@@ -1069,7 +1068,6 @@ __global__ __launch_bounds__(kPresortBlock) void leaf_bucket_kernel(TreeView<T> 
         a = ax_next<D>(a);
     }
     key[i] = (uint32_t)((node - tv.n_nodes) >> shift);
-    row[i] = (uint32_t)i;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1156,49 +1154,21 @@ __device__ __forceinline__ uint32_t hilbert_cell(const float* lo, const float* h
     return code;
 }
 
-// Order-preserving map of floating-point values onto unsigned integers (for atomicMin/Max).
-__device__ __forceinline__ uint32_t ordered_bits(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float from_ordered(uint32_t u) {
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
-}
-__device__ __forceinline__ unsigned long long ordered_bits(double f) {
-    const unsigned long long u = (unsigned long long)__double_as_longlong(f);
-    return (u >> 63) ? ~u : (u | (1ull << 63));
-}
-__device__ __forceinline__ double from_ordered(unsigned long long u) {
-    return __longlong_as_double((long long)((u >> 63) ? (u & ~(1ull << 63)) : ~u));
-}
-
-template <typename T>
-using OrderedT = typename std::conditional<sizeof(T) == 4, uint32_t, unsigned long long>::type;
-
+// Bounding box of n points, one partial box per workgroup: part[block][0..D) = min, [D..2D) = max (NaN
+// coordinates left out).  The reader reduces the partials (reduce_boxes): no atomics, whose
+// same-address updates took 20 of the 27 us of a 1M-point box, and nothing to initialise.
 constexpr int kBoxBlock = 256;
+constexpr int kMaxBoxParts = 512;  // most workgroups of bbox_kernel
 
-// Bounding box of n points: box[0..D) = min, box[D..2D) = max, as ordered integers; the caller
-// initialises it to (all ones, zero).  Reduced per wavefront, then per block in LDS, then one
-// atomic per block and value.
+inline int box_parts(int64_t n) {
+    const int64_t b = (n + 4 * kBoxBlock - 1) / (4 * kBoxBlock);
+    return (int)(b < 1 ? 1 : b > kMaxBoxParts ? kMaxBoxParts : b);
+}
+
+// min / max over the 64 lanes, then over the workgroup's wavefronts through LDS; the result is in
+// every thread.
 template <typename T, int D>
-__global__ __launch_bounds__(kBoxBlock) void bbox_kernel(const T* __restrict__ pts, int64_t n,
-                                                         OrderedT<T>* __restrict__ box) {
-    constexpr int kWaves = kBoxBlock / 64;
-    __shared__ T s_lo[kWaves][D], s_hi[kWaves][D];
-    T lo[D], hi[D];
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        lo[a] = pos_inf<T>();
-        hi[a] = -pos_inf<T>();
-    }
-    for (int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBoxBlock) {
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const T v = pts[i * D + a];
-            lo[a] = fmin(lo[a], v);
-            hi[a] = fmax(hi[a], v);
-        }
-    }
+__device__ __forceinline__ void block_box(T (&lo)[D], T (&hi)[D], T (*s_lo)[D], T (*s_hi)[D]) {
 #pragma unroll
     for (int a = 0; a < D; ++a) {
 #pragma unroll
@@ -1216,38 +1186,88 @@ __global__ __launch_bounds__(kBoxBlock) void bbox_kernel(const T* __restrict__ p
         }
     }
     __syncthreads();
-    if (threadIdx.x < D) {
-        const int a = threadIdx.x;
-        T l = s_lo[0][a], h = s_hi[0][a];
-        for (int v = 1; v < kWaves; ++v) {
-            l = fmin(l, s_lo[v][a]);
-            h = fmax(h, s_hi[v][a]);
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        lo[a] = s_lo[0][a];
+        hi[a] = s_hi[0][a];
+        for (int v = 1; v < kBoxBlock / 64; ++v) {
+            lo[a] = fmin(lo[a], s_lo[v][a]);
+            hi[a] = fmax(hi[a], s_hi[v][a]);
         }
-        atomicMin(&box[a], ordered_bits(l));
-        atomicMax(&box[D + a], ordered_bits(h));
     }
 }
 
-// Cell key over a box held as ordered integers (from bbox_kernel): the Hilbert index when hilbert
-// (the forward presort at d <= 3: plain workload traversal 7.78 ms against 7.88 with the Morton
-// code, fp64 workload 1.41 against 1.49; at d = 8 the Morton code is faster, 90.6 against 92.2 ms),
-// else the Morton code (always for the backward's canonical order).
 template <typename T, int D>
-__global__ __launch_bounds__(kPresortBlock) void morton_bucket_kernel(const T* __restrict__ queries, int64_t nq,
-                                                                       const OrderedT<T>* __restrict__ box, int bits,
-                                                                       uint32_t* __restrict__ key,
-                                                                       uint32_t* __restrict__ row,
-                                                                       bool hilbert) {
-    const int64_t i = (int64_t)blockIdx.x * kPresortBlock + threadIdx.x;
-    if (i >= nq) return;
+__global__ __launch_bounds__(kBoxBlock) void bbox_kernel(const T* __restrict__ pts, int64_t n, T* __restrict__ part) {
+    __shared__ T s_lo[kBoxBlock / 64][D], s_hi[kBoxBlock / 64][D];
+    T lo[D], hi[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        lo[a] = pos_inf<T>();
+        hi[a] = -pos_inf<T>();
+    }
+    const int64_t stride = (int64_t)gridDim.x * kBoxBlock;
+#pragma unroll 4
+    for (int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x; i < n; i += stride) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const T v = pts[i * D + a];
+            lo[a] = fmin(lo[a], v);
+            hi[a] = fmax(hi[a], v);
+        }
+    }
+    block_box<T, D>(lo, hi, s_lo, s_hi);
+    if (threadIdx.x < D) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            if (a == (int)threadIdx.x) {
+                part[(int64_t)blockIdx.x * 2 * D + a] = lo[a];
+                part[(int64_t)blockIdx.x * 2 * D + D + a] = hi[a];
+            }
+        }
+    }
+}
+
+// Cell keys over the box of n_part partials (bbox_kernel): the Hilbert index when hilbert (the forward
+// presort at d <= 3: plain workload traversal 7.78 ms against 7.88 with the Morton code, fp64
+// workload 1.41 against 1.49; at d = 8 the Morton code is faster, 90.6 against 92.2 ms), else the
+// Morton code (always for the backward's canonical order).  Every workgroup reduces the partials,
+// then strides over the queries (at most kMaxKeyBlocks workgroups, so that the reduction stays small
+// beside the queries).
+constexpr int kMaxKeyBlocks = 4096;
+inline unsigned key_blocks(int64_t nq) {
+    const int64_t b = (nq + kBoxBlock - 1) / kBoxBlock;
+    return (unsigned)(b > kMaxKeyBlocks ? kMaxKeyBlocks : b);
+}
+template <typename T, int D>
+__global__ __launch_bounds__(kBoxBlock) void morton_bucket_kernel(const T* __restrict__ queries, int64_t nq,
+                                                                  const T* __restrict__ part, int n_part, int bits,
+                                                                  uint32_t* __restrict__ key, bool hilbert) {
+    __shared__ T s_lo[kBoxBlock / 64][D], s_hi[kBoxBlock / 64][D];
+    T blo[D], bhi[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        blo[a] = pos_inf<T>();
+        bhi[a] = -pos_inf<T>();
+    }
+    for (int p = threadIdx.x; p < n_part; p += kBoxBlock) {
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            blo[a] = fmin(blo[a], part[(int64_t)p * 2 * D + a]);
+            bhi[a] = fmax(bhi[a], part[(int64_t)p * 2 * D + D + a]);
+        }
+    }
+    block_box<T, D>(blo, bhi, s_lo, s_hi);
     float lo[D], hi[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) {
-        lo[a] = (float)from_ordered(box[a]);
-        hi[a] = (float)from_ordered(box[D + a]);
+        lo[a] = (float)blo[a];
+        hi[a] = (float)bhi[a];
     }
-    key[i] = hilbert ? hilbert_cell<T, D>(lo, hi, bits, queries + i * D) : morton_cell<T, D>(lo, hi, bits, queries + i * D);
-    row[i] = (uint32_t)i;
+    const int64_t stride = (int64_t)gridDim.x * kBoxBlock;
+    for (int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x; i < nq; i += stride)
+        key[i] = hilbert ? hilbert_cell<T, D>(lo, hi, bits, queries + i * D)
+                         : morton_cell<T, D>(lo, hi, bits, queries + i * D);
 }
 
 }  // namespace tk

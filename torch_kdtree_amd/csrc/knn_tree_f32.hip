@@ -25,14 +25,12 @@ void launch_tree_search_f32(const Tree& t, const float* q, int64_t nq, const int
     launch_lane_search_t<float>(t, q, nq, order, k, dist, idx, orig, tie, s);
 }
 
-void launch_leaf_bucket_f32(const Tree& t, const float* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,
-                            hipStream_t s) {
-    launch_leaf_bucket_t<float>(t, q, nq, shift, key, row, s);
+void launch_leaf_bucket_f32(const Tree& t, const float* q, int64_t nq, int shift, uint32_t* key, hipStream_t s) {
+    launch_leaf_bucket_t<float>(t, q, nq, shift, key, s);
 }
 
-void launch_morton_bucket_f32(const Tree& t, const float* q, int64_t nq, void* bbox, uint32_t* key, uint32_t* row,
-                              hipStream_t s) {
-    launch_morton_bucket_t<float>(t, q, nq, bbox, key, row, s);
+void launch_morton_bucket_f32(const Tree& t, const float* q, int64_t nq, void* box, uint32_t* key, hipStream_t s) {
+    launch_morton_bucket_t<float>(t, q, nq, box, key, s);
 }
 
 int morton_bucket_count(int dims) { return morton_buckets(dims); }

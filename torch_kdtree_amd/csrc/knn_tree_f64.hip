@@ -18,14 +18,12 @@ void launch_tree_search_f64(const Tree& t, const double* q, int64_t nq, const in
         launch_lane_search_t<double>(t, q, nq, order, k, dist, idx, orig, tie, s);
 }
 
-void launch_leaf_bucket_f64(const Tree& t, const double* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,
-                            hipStream_t s) {
-    launch_leaf_bucket_t<double>(t, q, nq, shift, key, row, s);
+void launch_leaf_bucket_f64(const Tree& t, const double* q, int64_t nq, int shift, uint32_t* key, hipStream_t s) {
+    launch_leaf_bucket_t<double>(t, q, nq, shift, key, s);
 }
 
-void launch_morton_bucket_f64(const Tree& t, const double* q, int64_t nq, void* bbox, uint32_t* key, uint32_t* row,
-                              hipStream_t s) {
-    launch_morton_bucket_t<double>(t, q, nq, bbox, key, row, s);
+void launch_morton_bucket_f64(const Tree& t, const double* q, int64_t nq, void* box, uint32_t* key, hipStream_t s) {
+    launch_morton_bucket_t<double>(t, q, nq, box, key, s);
 }
 
 }  // namespace tk

@@ -110,18 +110,16 @@ void launch_exact_search_t(const Tree& t, const T* q, int64_t nq, const int32_t*
 #ifndef TK_HILBERT_MAX_D
 #define TK_HILBERT_MAX_D 3
 #endif
-// bbox: 2*dims ordered integers of sizeof(T) bytes each, initialised by the caller (init_bbox).
+// box: scratch for kMaxBoxParts partial boxes of 2*dims values.
 template <typename T>
-void launch_morton_bucket_t(const Tree& t, const T* q, int64_t nq, void* bbox, uint32_t* key, uint32_t* row,
-                            hipStream_t s) {
-    auto* box = static_cast<OrderedT<T>*>(bbox);
-    const unsigned box_blocks = (unsigned)std::min<int64_t>(1024, (nq + kBoxBlock - 1) / kBoxBlock);
-    const dim3 grid((unsigned)((nq + kPresortBlock - 1) / kPresortBlock));
-#define TK_DIMS(DD)                                                                                              \
-    case DD:                                                                                                     \
-        hipLaunchKernelGGL((bbox_kernel<T, DD>), dim3(box_blocks), dim3(kBoxBlock), 0, s, q, nq, box);          \
-        hipLaunchKernelGGL((morton_bucket_kernel<T, DD>), grid, dim3(kPresortBlock), 0, s, q, nq, box,           \
-                           MortonBits<DD>::kBits, key, row, DD <= TK_HILBERT_MAX_D);                                                     \
+void launch_morton_bucket_t(const Tree& t, const T* q, int64_t nq, void* box, uint32_t* key, hipStream_t s) {
+    T* part = static_cast<T*>(box);
+    const int parts = box_parts(nq);
+#define TK_DIMS(DD)                                                                                                  \
+    case DD:                                                                                                         \
+        hipLaunchKernelGGL((bbox_kernel<T, DD>), dim3(parts), dim3(kBoxBlock), 0, s, q, nq, part);                   \
+        hipLaunchKernelGGL((morton_bucket_kernel<T, DD>), dim3(key_blocks(nq)), dim3(kBoxBlock), 0, s, q, nq, part, \
+                           parts, MortonBits<DD>::kBits, key, DD <= TK_HILBERT_MAX_D);                              \
         break;
     switch (t.dims) {
         TK_DIMS(1)
@@ -145,14 +143,12 @@ inline int morton_buckets(int dims) {
 }
 
 template <typename T>
-void launch_leaf_bucket_t(const Tree& t, const T* q, int64_t nq, int shift, uint32_t* key, uint32_t* row,
-                          hipStream_t s) {
+void launch_leaf_bucket_t(const Tree& t, const T* q, int64_t nq, int shift, uint32_t* key, hipStream_t s) {
     const TreeView<T> tv = tree_view<T>(t);
     const dim3 grid((unsigned)((nq + kPresortBlock - 1) / kPresortBlock));
 #define TK_DIMS(DD)                                                                                              \
     case DD:                                                                                                     \
-        hipLaunchKernelGGL((leaf_bucket_kernel<T, DD>), grid, dim3(kPresortBlock), 0, s, tv, q, nq, shift, key,  \
-                           row);                                                                                 \
+        hipLaunchKernelGGL((leaf_bucket_kernel<T, DD>), grid, dim3(kPresortBlock), 0, s, tv, q, nq, shift, key); \
         break;
     switch (t.dims) {
         TK_DIMS(1)
