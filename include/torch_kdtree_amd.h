@@ -84,7 +84,8 @@ int tk_tree_build_many(const void* const* points, const int64_t* n_points, int n
  * split values and leaf ranges as tk_tree_build whenever no node has two points with equal
  * coordinates on its split axis; with such ties the tied points may be ordered (and split)
  * differently, because the reference orders them by an unstable std::sort.  Fails when a
- * coordinate it sorts on is NaN.  The tree is uploaded to `device`.  At most 2^28 points. */
+ * coordinate it sorts on is NaN.  The tree stays on `device`; its host arrays (for the getters, saving
+ * and the host search) are copied from there when first asked for.  At most 2^28 points. */
 int tk_tree_build_gpu(const void* points, int64_t n_points, int dims, int dtype, int levels, int device, void* stream,
                       tk_tree** out);
 
@@ -157,6 +158,11 @@ int tk_tree_get_shuffled_inds(const tk_tree* tree, int32_t* out);
 
 /* Replaces KDTree::get_structured_points (src/interface.cpp:52-58): out[n_points*dims]. */
 int tk_tree_get_structured_points(const tk_tree* tree, void* out);
+
+/* The same two arrays of a GPU tree written to device memory on its GPU, without a copy through the
+ * host: points[n_points*dims] (dtype) and shuffled[n_points] (int64), either may be NULL.  Runs on
+ * `stream` and waits for it. */
+int tk_tree_export_gpu(const tk_tree* tree, void* points, int64_t* shuffled, void* stream);
 
 /* Node and leaf arrays of the tree (the reference's PartitionInfo, src/kdtree.hpp:165-206):
  * axis[2^levels-1], split[2^levels-1] (dtype), leaf_off[2^levels+1].  Any may be NULL. */

@@ -1,6 +1,6 @@
 """The radix sort's paths against torch's stable sort, at the sizes where one hands over to the next: one
-workgroup (4,096 pairs), counts summed by the passes (32 tiles of 4,096), look-back (2^21 pairs), and
-at a look-back over more tiles than run at a time."""
+workgroup (4,096 pairs), counts summed by the passes (32 tiles of 4,096) and look-back
+(2^21 pairs)."""
 import pytest
 import torch
 

@@ -150,6 +150,7 @@ BatchPlan* batch_create(const Tree* const* trees, int n_clouds, const int64_t* n
                                      " holds a non-finite coordinate or split value; the reference tie policy "
                                      "follows the reference's own steps for it, on its own tree (query it with "
                                      "build_kd_tree(...).query) or use the lower-index tie policy");
+        ensure_host(t);
         if (ks[c] > t.n_points)
             throw std::runtime_error("You requested more nearest neighbors than there are in the KD-Tree");
     }

@@ -45,6 +45,13 @@ const tk::Tree& tree_of(const tk_tree* h) {
     return *h->t;
 }
 
+// The tree with its host arrays filled.
+const tk::Tree& host_tree_of(const tk_tree* h) {
+    const tk::Tree& t = tree_of(h);
+    tk::ensure_host(t);
+    return t;
+}
+
 void check_dtype(int dtype) {
     if (dtype != TK_F32 && dtype != TK_F64) throw std::runtime_error("unsupported dtype");
 }
@@ -123,11 +130,7 @@ int tk_tree_build_gpu(const void* points, int64_t n_points, int dims, int dtype,
         if (!out) throw std::runtime_error("invalid arguments");
         *out = nullptr;
         check_dtype(dtype);
-        const int32_t lv = levels;
-        std::vector<tk::Tree*> t = tk::build_trees_gpu(points, &n_points, &lv, 1, dims, dtype, device, stream);
-        std::unique_ptr<tk::Tree> owned(t[0]);
-        tk::upload_tree(*owned, device);
-        *out = new tk_tree{owned.release()};
+        *out = new tk_tree{tk::build_tree_gpu(points, n_points, levels, dims, dtype, device, stream)};
     });
 }
 
@@ -145,7 +148,7 @@ int tk_tree_build_many_gpu(const void* points, const int64_t* n_points, int n_tr
 int tk_tree_serialize(const tk_tree* tree, void* buf, size_t* bytes) {
     return guarded([&] {
         if (!tree || !tree->t || !bytes) throw std::runtime_error("invalid arguments");
-        const std::vector<unsigned char> img = tk::serialize_tree(*tree->t);
+        const std::vector<unsigned char> img = tk::serialize_tree(host_tree_of(tree));
         if (buf) {
             if (*bytes < img.size()) throw std::runtime_error("serialization buffer too small");
             std::memcpy(buf, img.data(), img.size());
@@ -165,7 +168,7 @@ int tk_tree_deserialize(const void* buf, size_t bytes, tk_tree** out) {
 int tk_tree_save(const tk_tree* tree, const char* path) {
     return guarded([&] {
         if (!tree || !tree->t || !path) throw std::runtime_error("invalid arguments");
-        tk::save_tree(*tree->t, path);
+        tk::save_tree(host_tree_of(tree), path);
     });
 }
 
@@ -256,21 +259,27 @@ int tk_tree_get_lower_list(const tk_tree* tree, int32_t out[2]) {
 
 int tk_tree_get_shuffled_inds(const tk_tree* tree, int32_t* out) {
     return guarded([&] {
-        const tk::Tree& t = tree_of(tree);
+        const tk::Tree& t = host_tree_of(tree);
         std::memcpy(out, t.shuffled.data(), sizeof(int32_t) * (size_t)t.n_points);
     });
 }
 
 int tk_tree_get_structured_points(const tk_tree* tree, void* out) {
     return guarded([&] {
-        const tk::Tree& t = tree_of(tree);
+        const tk::Tree& t = host_tree_of(tree);
         std::memcpy(out, t.points.data(), t.points.size());
+    });
+}
+
+int tk_tree_export_gpu(const tk_tree* tree, void* points, int64_t* shuffled, void* stream) {
+    return guarded([&] {
+        tk::export_tree_gpu(tree_of(tree), points, shuffled, static_cast<hipStream_t>(stream));
     });
 }
 
 int tk_tree_get_nodes(const tk_tree* tree, int32_t* axis, void* split, int32_t* leaf_off) {
     return guarded([&] {
-        const tk::Tree& t = tree_of(tree);
+        const tk::Tree& t = host_tree_of(tree);
         if (axis)
             for (int32_t i = 0; i < t.n_nodes; ++i) axis[i] = t.axis[i];
         if (split) std::memcpy(split, t.split.data(), t.split.size());
@@ -281,7 +290,7 @@ int tk_tree_get_nodes(const tk_tree* tree, int32_t* axis, void* split, int32_t* 
 int tk_knn_query_cpu(const tk_tree* tree, const void* queries, int64_t n_queries, int k, void* dist, int32_t* idx,
                      int64_t* orig_idx, int n_threads) {
     return guarded([&] {
-        const tk::Tree& t = tree_of(tree);
+        const tk::Tree& t = host_tree_of(tree);
         if (n_queries < 0) throw std::runtime_error("negative query count");
         tk::query_cpu(t, queries, n_queries, k, dist, idx, orig_idx, n_threads);
     });
@@ -290,7 +299,7 @@ int tk_knn_query_cpu(const tk_tree* tree, const void* queries, int64_t n_queries
 int tk_knn_search_stats(const tk_tree* tree, const void* queries, int64_t n_queries, int k, int64_t out[2],
                         int n_threads) {
     return guarded([&] {
-        const tk::Tree& t = tree_of(tree);
+        const tk::Tree& t = host_tree_of(tree);
         if (n_queries < 0 || !out) throw std::runtime_error("invalid arguments");
         const size_t kk = (size_t)std::max(k, 1);
         std::vector<unsigned char> dist((size_t)n_queries * kk * tk::dtype_size(t.dtype));

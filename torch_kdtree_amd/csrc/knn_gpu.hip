@@ -130,14 +130,7 @@ void free_device_tree(Tree& t) noexcept {
     int prev = -1;
     (void)hipGetDevice(&prev);
     if (d->device >= 0) (void)hipSetDevice(d->device);
-    (void)hipFree(d->split);
-    (void)hipFree(d->recs);
-    (void)hipFree(d->leaf_off);
-    (void)hipFree(d->shuffled);
-    (void)hipFree(d->inv_shuffled);
-    (void)hipFree(d->boxes);
-    (void)hipFree(d->group_boxes);
-    (void)hipFree(d->group_base);
+    (void)hipFree(d->arena);
     if (prev >= 0) (void)hipSetDevice(prev);
     delete d;
     t.dev = nullptr;
@@ -189,35 +182,70 @@ bool cloud_ties_often(const Tree& t) {
 
 }  // namespace
 
+bool tree_wants_groups(const Tree& t) { return (int64_t)t.n_points >= (int64_t)kGroupMinLeaf * t.n_leaves; }
+
+DeviceTree* alloc_device_tree(const Tree& t, int device, int64_t n_group_boxes) {
+    std::unique_ptr<DeviceTree> d(new DeviceTree());
+    d->device = device;
+    d->rec_bytes = rec_bytes_for(t.dtype, t.dims);
+    d->box_bytes = box_bytes_for(t.dtype, t.dims);
+    const size_t n = (size_t)t.n_points;
+    size_t off = 0;
+    const auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) & ~size_t(255);
+        return at;
+    };
+    const size_t split = take((size_t)t.n_nodes * dtype_size(t.dtype));
+    // kRecPad zero records after the last point: chunked leaf scans read them and ignore them
+    const size_t recs = take((n + kRecPad) * (size_t)d->rec_bytes);
+    const size_t leaf_off = take(4 * ((size_t)t.n_leaves + 1));
+    const size_t shuffled = take(4 * n), inv = take(4 * n);
+    const size_t boxes = take(((size_t)t.n_nodes + (size_t)t.n_leaves) * (size_t)d->box_bytes);
+    const size_t gboxes = take(n_group_boxes ? (size_t)n_group_boxes * (size_t)d->box_bytes : 0);
+    const size_t gbase = take(n_group_boxes ? 4 * ((size_t)t.n_leaves + 1) : 0);
+    TK_HIP_CHECK(hipMalloc(&d->arena, off));
+    unsigned char* base = static_cast<unsigned char*>(d->arena);
+    d->split = base + split;
+    d->recs = base + recs;
+    d->leaf_off = reinterpret_cast<int32_t*>(base + leaf_off);
+    d->shuffled = reinterpret_cast<int32_t*>(base + shuffled);
+    d->inv_shuffled = reinterpret_cast<int32_t*>(base + inv);
+    d->boxes = base + boxes;
+    if (n_group_boxes) {
+        d->group_boxes = base + gboxes;
+        d->group_base = reinterpret_cast<int32_t*>(base + gbase);
+    }
+    return d.release();
+}
+
 void upload_tree(Tree& t, int device) {
+    ensure_host(t);
     free_device_tree(t);
     t.tie_prone = !t.finite || (t.dtype == kF32 ? cloud_ties_often<float>(t) : cloud_ties_often<double>(t));
     if (device < 0) TK_HIP_CHECK(hipGetDevice(&device));
     DeviceGuard g(device);
-    std::unique_ptr<DeviceTree> d(new DeviceTree());
-    d->device = device;
-    d->rec_bytes = rec_bytes_for(t.dtype, t.dims);
+    const int rec_bytes = rec_bytes_for(t.dtype, t.dims), box_bytes = box_bytes_for(t.dtype, t.dims);
     const size_t ts = dtype_size(t.dtype);
     const size_t coord_bytes = ts * (size_t)t.dims;
     const size_t n = (size_t)t.n_points;
     // kRecPad zero records after the last point: chunked leaf scans read them and ignore them
-    std::vector<unsigned char> recs((n + kRecPad) * (size_t)d->rec_bytes, 0);
+    std::vector<unsigned char> recs((n + kRecPad) * (size_t)rec_bytes, 0);
     std::vector<int32_t> inv(n);
     for (size_t s = 0; s < n; ++s) inv[(size_t)t.shuffled[s]] = (int32_t)s;
-    const bool rec_idx = (size_t)d->rec_bytes >= coord_bytes + 4;  // RecLayout::kHasIdx
+    const bool rec_idx = (size_t)rec_bytes >= coord_bytes + 4;  // RecLayout::kHasIdx
     for (size_t s = 0; s < n; ++s) {
-        unsigned char* r = &recs[s * (size_t)d->rec_bytes];
+        unsigned char* r = &recs[s * (size_t)rec_bytes];
         std::memcpy(r, &t.points[s * coord_bytes], coord_bytes);
         if (rec_idx) std::memcpy(r + coord_bytes, &t.shuffled[s], 4);
     }
     // boxes: lo then hi, each padded from dims to box_bytes / (2 * ts) elements
-    d->box_bytes = box_bytes_for(t.dtype, t.dims);
     const size_t n_boxes = (size_t)t.n_nodes + (size_t)t.n_leaves;
-    const size_t half = (size_t)d->box_bytes / 2;
-    std::vector<unsigned char> boxes(n_boxes * (size_t)d->box_bytes, 0);
+    const size_t half = (size_t)box_bytes / 2;
+    std::vector<unsigned char> boxes(n_boxes * (size_t)box_bytes, 0);
     for (size_t b = 0; b < n_boxes; ++b) {
         const unsigned char* src = &t.aabb[b * 2 * coord_bytes];
-        unsigned char* dst = &boxes[b * (size_t)d->box_bytes];
+        unsigned char* dst = &boxes[b * (size_t)box_bytes];
         std::memcpy(dst, src, coord_bytes);
         std::memcpy(dst + half, src + coord_bytes, coord_bytes);
     }
@@ -226,7 +254,7 @@ void upload_tree(Tree& t, int device) {
     // (plain workload, 4M points: at depth 13, 488 points a leaf, the traversal takes 14.0 instead of
     // 20.1 ms; at depth 17, 30 a leaf, no gain), and only for finite trees, which prune with
     // boxes (a NaN coordinate would be dropped by min / max).
-    const bool use_groups = t.finite && (int64_t)t.n_points >= (int64_t)kGroupMinLeaf * t.n_leaves;
+    const bool use_groups = t.finite && tree_wants_groups(t);
     std::vector<int32_t> gbase;
     std::vector<unsigned char> gboxes;
     auto group_box = [&](auto tag) {
@@ -246,7 +274,7 @@ void upload_tree(Tree& t, int device) {
                         lo[a] = std::min(lo[a], pts[(size_t)s * D + a]);
                         hi[a] = std::max(hi[a], pts[(size_t)s * D + a]);
                     }
-                unsigned char* dst = &gboxes[((size_t)gbase[(size_t)l] + g) * (size_t)d->box_bytes];
+                unsigned char* dst = &gboxes[((size_t)gbase[(size_t)l] + g) * (size_t)box_bytes];
                 std::memcpy(dst, lo, sizeof(TT) * D);
                 std::memcpy(dst + half, hi, sizeof(TT) * D);
             }
@@ -258,44 +286,79 @@ void upload_tree(Tree& t, int device) {
             const int32_t nl = t.leaf_off[(size_t)l + 1] - t.leaf_off[(size_t)l];
             gbase[(size_t)l + 1] = gbase[(size_t)l] + (nl + kGroupRecs - 1) / kGroupRecs;
         }
-        gboxes.assign(std::max<size_t>((size_t)gbase[(size_t)t.n_leaves], 1) * (size_t)d->box_bytes, 0);
+        gboxes.assign(std::max<size_t>((size_t)gbase[(size_t)t.n_leaves], 1) * (size_t)box_bytes, 0);
         if (t.dtype == kF32)
             group_box(float());
         else
             group_box(double());
     }
+    std::unique_ptr<DeviceTree> d(alloc_device_tree(t, device, use_groups ? (int64_t)(gboxes.size() / box_bytes) : 0));
     try {
-        TK_HIP_CHECK(hipMalloc(&d->split, (size_t)t.n_nodes * ts));
-        TK_HIP_CHECK(hipMalloc((void**)&d->recs, recs.size()));
-        TK_HIP_CHECK(hipMalloc((void**)&d->leaf_off, sizeof(int32_t) * t.leaf_off.size()));
-        TK_HIP_CHECK(hipMalloc((void**)&d->shuffled, sizeof(int32_t) * n));
-        TK_HIP_CHECK(hipMalloc((void**)&d->inv_shuffled, sizeof(int32_t) * n));
-        TK_HIP_CHECK(hipMalloc((void**)&d->boxes, boxes.size()));
-        TK_HIP_CHECK(hipMemcpy(d->split, t.split.data(), (size_t)t.n_nodes * ts, hipMemcpyHostToDevice));
-        TK_HIP_CHECK(hipMemcpy(d->recs, recs.data(), recs.size(), hipMemcpyHostToDevice));
-        TK_HIP_CHECK(hipMemcpy(d->leaf_off, t.leaf_off.data(), sizeof(int32_t) * t.leaf_off.size(),
-                               hipMemcpyHostToDevice));
-        TK_HIP_CHECK(hipMemcpy(d->shuffled, t.shuffled.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-        TK_HIP_CHECK(hipMemcpy(d->inv_shuffled, inv.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice));
-        TK_HIP_CHECK(hipMemcpy(d->boxes, boxes.data(), boxes.size(), hipMemcpyHostToDevice));
+        const auto copy = [](void* dst, const void* src, size_t bytes) {
+            TK_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+        };
+        copy(d->split, t.split.data(), (size_t)t.n_nodes * ts);
+        copy(d->recs, recs.data(), recs.size());
+        copy(d->leaf_off, t.leaf_off.data(), sizeof(int32_t) * t.leaf_off.size());
+        copy(d->shuffled, t.shuffled.data(), sizeof(int32_t) * n);
+        copy(d->inv_shuffled, inv.data(), sizeof(int32_t) * n);
+        copy(d->boxes, boxes.data(), boxes.size());
         if (use_groups) {
-            TK_HIP_CHECK(hipMalloc((void**)&d->group_boxes, gboxes.size()));
-            TK_HIP_CHECK(hipMalloc((void**)&d->group_base, sizeof(int32_t) * gbase.size()));
-            TK_HIP_CHECK(hipMemcpy(d->group_boxes, gboxes.data(), gboxes.size(), hipMemcpyHostToDevice));
-            TK_HIP_CHECK(hipMemcpy(d->group_base, gbase.data(), sizeof(int32_t) * gbase.size(), hipMemcpyHostToDevice));
+            copy(d->group_boxes, gboxes.data(), gboxes.size());
+            copy(d->group_base, gbase.data(), sizeof(int32_t) * gbase.size());
         }
     } catch (...) {
-        (void)hipFree(d->split);
-        (void)hipFree(d->recs);
-        (void)hipFree(d->leaf_off);
-        (void)hipFree(d->shuffled);
-        (void)hipFree(d->inv_shuffled);
-        (void)hipFree(d->boxes);
-        (void)hipFree(d->group_boxes);
-        (void)hipFree(d->group_base);
+        (void)hipFree(d->arena);
         throw;
     }
     t.dev = d.release();
+}
+
+void ensure_host(const Tree& ct) {
+    if (ct.host_ready.load(std::memory_order_acquire)) return;
+    Tree& t = const_cast<Tree&>(ct);  // the host arrays are a cache of the GPU copy
+    std::lock_guard<std::mutex> lk(t.host_mu);
+    if (t.host_ready.load(std::memory_order_relaxed)) return;
+    if (!t.dev) throw std::runtime_error("the tree has neither host arrays nor a GPU copy");
+    DeviceGuard g(t.dev->device);
+    const size_t n = (size_t)t.n_points, rb = (size_t)t.dev->rec_bytes;
+    const size_t coord_bytes = dtype_size(t.dtype) * (size_t)t.dims;
+    std::vector<unsigned char> recs(n * rb);
+    t.split.resize((size_t)t.n_nodes * dtype_size(t.dtype));
+    t.leaf_off.resize((size_t)t.n_leaves + 1);
+    t.shuffled.resize(n);
+    t.points.resize(n * coord_bytes);
+    TK_HIP_CHECK(hipMemcpy(recs.data(), t.dev->recs, recs.size(), hipMemcpyDeviceToHost));
+    TK_HIP_CHECK(hipMemcpy(t.split.data(), t.dev->split, t.split.size(), hipMemcpyDeviceToHost));
+    TK_HIP_CHECK(hipMemcpy(t.leaf_off.data(), t.dev->leaf_off, 4 * t.leaf_off.size(), hipMemcpyDeviceToHost));
+    TK_HIP_CHECK(hipMemcpy(t.shuffled.data(), t.dev->shuffled, 4 * n, hipMemcpyDeviceToHost));
+    for (size_t s = 0; s < n; ++s) std::memcpy(&t.points[s * coord_bytes], &recs[s * rb], coord_bytes);
+    finish_tree(t);
+    t.host_ready.store(true, std::memory_order_release);
+}
+
+// out[s] = coordinates of record s (words 32-bit words of each record), idx[s] = its original index.
+__global__ __launch_bounds__(256) void export_kernel(const unsigned char* __restrict__ recs, int rec_words, int words,
+                                                     const int32_t* __restrict__ shuffled, int64_t n,
+                                                     uint32_t* __restrict__ out, int64_t* __restrict__ idx) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (out && i < n * words)
+        out[i] = reinterpret_cast<const uint32_t*>(recs)[(i / words) * rec_words + i % words];
+    if (idx && i < n) idx[i] = shuffled[i];
+}
+
+void export_tree_gpu(const Tree& t, void* points, int64_t* shuffled, hipStream_t stream) {
+    if (!t.dev) throw std::runtime_error("The tree has no GPU copy (it was built for the CPU)");
+    if (!points && !shuffled) return;
+    DeviceGuard g(t.dev->device);
+    const int words = (int)(dtype_size(t.dtype) * (size_t)t.dims / 4);
+    const int64_t total = (int64_t)t.n_points * (points ? words : 1);
+    hipLaunchKernelGGL(export_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, t.dev->recs,
+                       t.dev->rec_bytes / 4, words, t.dev->shuffled, (int64_t)t.n_points,
+                       static_cast<uint32_t*>(points), shuffled);
+    TK_HIP_CHECK(hipGetLastError());
+    // (complete on return, like the getters: the caller may read the arrays on any stream)
+    TK_HIP_CHECK(hipStreamSynchronize(stream));
 }
 
 // ------------------------------------------------------------------------------------------

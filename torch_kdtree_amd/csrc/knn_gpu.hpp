@@ -13,6 +13,7 @@ namespace tk {
 // different layout: split values in heap order, one record per point, leaf offsets).
 struct DeviceTree {
     int device = -1;
+    void* arena = nullptr;            // the one allocation that holds every array below
     void* split = nullptr;            // T[n_nodes]
     unsigned char* recs = nullptr;    // records, RecLayout<T, dims>::kBytes each
     int32_t* leaf_off = nullptr;      // [n_leaves + 1]
@@ -31,7 +32,16 @@ struct DeviceTree {
 
 int rec_bytes_for(int dtype, int dims);
 int box_bytes_for(int dtype, int dims);
+// A device tree for t's sizes with its arrays allocated (on the current device) and not filled:
+// group boxes for n_group_boxes of them (0: none).
+DeviceTree* alloc_device_tree(const Tree& t, int device, int64_t n_group_boxes);
+// Whether the tree gets group boxes if it is finite: leaves of kGroupMinLeaf points on average.
+bool tree_wants_groups(const Tree& t);
 void upload_tree(Tree& t, int device);
+// Fills the host arrays of a tree that has them on the GPU alone.
+void ensure_host(const Tree& t);
+// Device arrays of the tree's structured points (dense rows) and their original indices; either null.
+void export_tree_gpu(const Tree& t, void* points, int64_t* shuffled, hipStream_t stream);
 void free_device_tree(Tree& t) noexcept;
 
 enum TiePolicy : int { kTieReference = 0, kTieLowerIndex = 1 };

@@ -104,6 +104,17 @@ struct KDTree {
         return v;
     }
 
+    // Structured points and their original indices (int64) into device arrays (tk_tree_export_gpu).
+    void export_gpu(size_t points_ptr, size_t shuffled_ptr, size_t stream) const {
+        int rc;
+        {
+            py::gil_scoped_release release;
+            rc = tk_tree_export_gpu(tree, reinterpret_cast<void*>(points_ptr), reinterpret_cast<int64_t*>(shuffled_ptr),
+                                    reinterpret_cast<void*>(stream));
+        }
+        check(rc);
+    }
+
     // Leaves and points scanned by the search of host queries (summed), see tk_knn_search_stats.
     py::tuple search_stats(const py::array_t<T, py::array::c_style | py::array::forcecast>& q, int k, int n_threads) {
         int64_t out[2] = {0, 0};
@@ -347,6 +358,8 @@ void bind_tree(py::module_& m, const char* name) {
              "Returns the shuffled indices to translate from local to global indices")
         .def("get_structured_points", &C::get_structured_points,
              "Returns the ordered points how they are used in the KD-Tree")
+        .def("export_gpu", &C::export_gpu, py::arg("points_ptr"), py::arg("shuffled_ptr"), py::arg("stream") = 0,
+             "Writes the structured points and their int64 original indices to device arrays (GPU trees)")
         .def("get_nodes", &C::get_nodes, "Returns (axis[int32], split[T], leaf_offsets[int32]) of the tree")
         .def("is_finite", &C::is_finite, "True when every coordinate and split value of the tree is finite")
         .def("backward", &C::backward, py::arg("queries_ptr"), py::arg("ref_ptr"), py::arg("n_queries"), py::arg("k"),

@@ -9,8 +9,10 @@
 //   * leaves are contiguous runs of the structured point array; leaf_off[j] .. leaf_off[j+1].
 #pragma once
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -58,6 +60,11 @@ struct Tree {
     // points, coordinates on few distinct values), or the tree holds a non-finite value.
     bool tie_prone = false;
     DeviceTree* dev = nullptr;          // GPU copy, owned
+    // A tree built on the GPU has its arrays there alone until something asks for them on the host:
+    // axis, split, leaf_off, points, shuffled and aabb are then filled from the GPU copy
+    // (ensure_host, knn_gpu.hpp), once, under host_mu.
+    std::atomic<bool> host_ready{true};
+    std::mutex host_mu;
 
     template <typename T> T* split_ptr() { return reinterpret_cast<T*>(split.data()); }
     template <typename T> const T* split_ptr() const { return reinterpret_cast<const T*>(split.data()); }
@@ -76,6 +83,9 @@ inline bool dims_supported(int d) { return d == 1 || d == 2 || d == 3 || d == 8;
 
 // Builds the tree on the host.  Throws std::runtime_error with the reference's messages.
 Tree* build_tree(const void* points, int64_t n_points, int dims, int levels, int dtype, int n_threads);
+
+// Builds one tree on the GPU and leaves it there, uploaded (its host arrays are made when first asked for).
+Tree* build_tree_gpu(const void* points, int64_t n_points, int levels, int dims, int dtype, int device, void* stream);
 
 // Builds trees on the GPU (tree_build_gpu.hip): tree c from points[base_c .. base_c + n_points[c])
 // of the concatenated device array `points` ([sum n_points, dims] values of dtype, on `device`),

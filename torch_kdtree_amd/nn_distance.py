@@ -136,9 +136,15 @@ class TorchKDTree:
             raise ValueError("builder must be 'cpu' or 'gpu'")
         self.levels = levels
 
-        self.structured_points = torch.from_numpy(self.kdtree.get_structured_points())
-        self.shuffled_ind = torch.from_numpy(self.kdtree.get_shuffled_inds()).long()
-        self.use_gpu = use_gpu = (device.type == 'cuda')
+        self.use_gpu = (device.type == 'cuda')
+        if self.use_gpu:  # written on the GPU from its copy of the tree
+            self.structured_points = torch.empty((self.nr_ref_points, self.dims), dtype=self.dtype, device=device)
+            self.shuffled_ind = torch.empty(self.nr_ref_points, dtype=torch.int64, device=device)
+            self.kdtree.export_gpu(self.structured_points.data_ptr(), self.shuffled_ind.data_ptr(),
+                                   _stream_handle(device))
+        else:
+            self.structured_points = torch.from_numpy(self.kdtree.get_structured_points())
+            self.shuffled_ind = torch.from_numpy(self.kdtree.get_shuffled_inds()).long()
         self.device = device
         self.dtype_idx = torch.int32  # Restriction in the compiled library
         self.ref_requires_grad = points_ref.requires_grad
@@ -153,10 +159,6 @@ class TorchKDTree:
         # launch variant of GPU queries: None = the autotuner's choice for each k (autotune.variant_for)
         self.variant = variant
         self._applied_variant = 0
-
-        if self.use_gpu:
-            self.structured_points = self.structured_points.to(self.device)
-            self.shuffled_ind = self.shuffled_ind.to(self.device)
 
     def save(self, path: str) -> None:
         """Writes the tree (structured points, indices, nodes and leaves) to ``path``; ``load_kd_tree``
