@@ -2,14 +2,14 @@
 //
 // Up to kSmallItems pairs: one workgroup runs every pass in LDS (one launch).  Up to kLookBackMax:
 //   1. radix_count_kernel reads the keys once and counts the digits of every pass, per workgroup;
-//   2. one radix_pass_kernel<true> per pass.  Workgroups take tiles of kRadixTile pairs by a ticket, rank
+//   2. one look-back radix_pass_kernel per pass.  Workgroups take tiles of pairs by a ticket, rank
 //      their tile, publish its digit counts and find the pairs of each digit in all earlier
 //      tiles by looking back over the earlier tiles' published counts (each tile publishes first its
 //      own counts, then the sum up to and including it), so a pass is one launch.
 // More, per pass:
 //   1. radix_hist_kernel counts the digits of every tile;
 //   2. radix_scan_kernel scans the counts of each digit over the tiles;
-//   3. radix_pass_kernel<false> ranks the tiles and writes them out.
+//   3. radix_pass_kernel ranks the tiles and writes them out.
 // In a pass every wavefront ranks its quarter of the tile in index order, 64 pairs per round (lanes
 // holding the same digit are found with one ballot per digit bit; per-digit running counts live in
 // the wavefront's own LDS row).  The tile, rearranged by digit in LDS, is written out slot by slot:
@@ -38,8 +38,12 @@ namespace tk {
 namespace {
 
 constexpr int kRadixBlock = 256;
-constexpr int kRadixItems = 16;
+constexpr int kRadixItems = 16;  // pairs per thread of a tile
 constexpr int kRadixTile = kRadixBlock * kRadixItems;
+// Smaller tiles for sorts whose 4,096-pair tiles would leave CUs idle (65,537 pairs 47 -> 37 us, 500K of
+// 32 bits 78 -> 73; 1M of 24 bits 71 -> 82: more tiles to look back over).
+constexpr int kRadixItemsFew = 8;
+constexpr int64_t kFewMax = int64_t(512) << 10;
 constexpr int kRadixBins = 256;
 constexpr int kMaxPasses = 4;
 constexpr int64_t kLookBackMax = int64_t(2) << 20;
@@ -119,7 +123,7 @@ __device__ __forceinline__ int32_t scan_256(int32_t c, int32_t* tmp) {
 
 // Digit counts of all passes, per workgroup: part[block][pass][digit].  Also clears the tickets and
 // the first pass's status words.
-template <int P>
+template <int P, int kItems>
 __global__ __launch_bounds__(kRadixBlock) void radix_count_kernel(const uint32_t* __restrict__ keys, int64_t n,
                                                                   int32_t n_tiles, uint32_t* __restrict__ part,
                                                                   uint32_t* __restrict__ tickets,
@@ -134,15 +138,15 @@ __global__ __launch_bounds__(kRadixBlock) void radix_count_kernel(const uint32_t
     __syncthreads();
     for (int32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
         status[(int64_t)tile * kRadixBins + t] = 0;
-        const int64_t base = (int64_t)tile * kRadixTile;
-        uint32_t k[kRadixItems];
+        const int64_t base = (int64_t)tile * (kRadixBlock * kItems);
+        uint32_t k[kItems];
 #pragma unroll
-        for (int s = 0; s < kRadixItems; ++s) {
+        for (int s = 0; s < kItems; ++s) {
             const int64_t i = base + (int64_t)s * kRadixBlock + t;
             k[s] = i < n ? keys[i] : 0u;
         }
 #pragma unroll
-        for (int s = 0; s < kRadixItems; ++s) {
+        for (int s = 0; s < kItems; ++s) {
             if (base + (int64_t)s * kRadixBlock + t < n) {
 #pragma unroll
                 for (int p = 0; p < P; ++p) count_digit(cnt[w][p], (k[s] >> (8 * p)) & (kRadixBins - 1));
@@ -251,14 +255,15 @@ struct PassArgs {
 };
 
 // One pass.  vals_in null: the values are the pairs' indices.
-template <bool kLookBack>
+template <bool kLookBack, int kItems>
 __global__ __launch_bounds__(kRadixBlock) void radix_pass_kernel(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int64_t n, int shift, PassArgs args,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
     constexpr int kWaves = kRadixBlock / 64;
-    constexpr int kRounds = kRadixTile / kRadixBlock;
-    __shared__ uint32_t tile_k[kRadixTile];           // the tile in digit order (stable)
-    __shared__ uint32_t tile_v[kRadixTile];
+    constexpr int kTile = kRadixBlock * kItems;
+    constexpr int kRounds = kItems;
+    __shared__ uint32_t tile_k[kTile];           // the tile in digit order (stable)
+    __shared__ uint32_t tile_v[kTile];
     __shared__ int32_t tile_start[kRadixBins];        // first tile slot of each digit
     __shared__ int32_t wave_cnt[kWaves][kRadixBins];  // per wavefront: pairs of each digit, then their first slot
     __shared__ int32_t tmp[4];
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(kRadixBlock) void radix_pass_kernel(
         total = args.total[t];
         before = args.hist[(int64_t)t * args.n_tiles + tile];
     }
-    const int64_t base = tile * kRadixTile + (int64_t)w * kRounds * 64;
+    const int64_t base = tile * kTile + (int64_t)w * kRounds * 64;
     uint32_t key[kRounds], val[kRounds];
     int32_t rank[kRounds];
 #pragma unroll
@@ -348,7 +353,7 @@ __global__ __launch_bounds__(kRadixBlock) void radix_pass_kernel(
     blk_off[t] = (int32_t)(start + before) - tile_start[t];
     __syncthreads();
     // write out in tile order: each digit's slots go to consecutive output positions
-    const int n_tile = (int)min((int64_t)kRadixTile, n - tile * kRadixTile);
+    const int n_tile = (int)min((int64_t)kTile, n - tile * kTile);
     for (int x = t; x < n_tile; x += kRadixBlock) {
         const uint32_t k = tile_k[x];
         const int32_t pos = blk_off[(k >> shift) & (kRadixBins - 1)] + x;
@@ -441,7 +446,8 @@ struct RadixLayout {
 
 RadixLayout radix_layout(int64_t n) {
     RadixLayout l{};
-    l.n_tiles = (int32_t)std::max<int64_t>(1, (n + kRadixTile - 1) / kRadixTile);
+    const int64_t tile = kRadixBlock * (n <= kFewMax ? kRadixItemsFew : kRadixItems);
+    l.n_tiles = (int32_t)std::max<int64_t>(1, (n + tile - 1) / tile);
     const bool look_back = n <= kLookBackMax;
     l.n_parts = std::min(l.n_tiles, kCountBlocks);
     size_t off = 0;
@@ -490,12 +496,16 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
         return;
     }
     const bool look_back = n <= kLookBackMax;
-    const bool direct = l.n_parts <= kDirectParts;
+    const bool direct = l.n_parts <= kDirectParts, few = n <= kFewMax;
     if (look_back) {
 #define TK_COUNT(P)                                                                                               \
     case P:                                                                                                       \
-        hipLaunchKernelGGL(radix_count_kernel<P>, dim3(l.n_parts), block, 0, stream, keys_in, n, l.n_tiles, part, \
-                           tickets, status[0]);                                                                   \
+        if (few)                                                                                                  \
+            hipLaunchKernelGGL((radix_count_kernel<P, kRadixItemsFew>), dim3(l.n_parts), block, 0, stream,        \
+                               keys_in, n, l.n_tiles, part, tickets, status[0]);                                  \
+        else                                                                                                      \
+            hipLaunchKernelGGL((radix_count_kernel<P, kRadixItems>), dim3(l.n_parts), block, 0, stream, keys_in,  \
+                               n, l.n_tiles, part, tickets, status[0]);                                           \
         break;
         switch (passes) {
             TK_COUNT(1)
@@ -528,14 +538,20 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
             args.ticket = tickets + p;
             args.status = status[p & 1];
             args.status_next = status[(p + 1) & 1];
-            hipLaunchKernelGGL(radix_pass_kernel<true>, grid, block, 0, stream, ks, vs, n, 8 * p, args, kd, vd);
+            if (few)
+                hipLaunchKernelGGL((radix_pass_kernel<true, kRadixItemsFew>), grid, block, 0, stream, ks, vs, n, 8 * p,
+                                   args, kd, vd);
+            else
+                hipLaunchKernelGGL((radix_pass_kernel<true, kRadixItems>), grid, block, 0, stream, ks, vs, n, 8 * p, args,
+                                   kd, vd);
         } else {
             args.hist = status[0];
             args.total = base;
             hipLaunchKernelGGL(radix_hist_kernel, grid, block, 0, stream, ks, n, 8 * p, l.n_tiles, status[0]);
             hipLaunchKernelGGL(radix_scan_kernel, dim3(kRadixBins), dim3(kScanBlock), 0, stream, status[0], l.n_tiles,
                                base);
-            hipLaunchKernelGGL(radix_pass_kernel<false>, grid, block, 0, stream, ks, vs, n, 8 * p, args, kd, vd);
+            hipLaunchKernelGGL((radix_pass_kernel<false, kRadixItems>), grid, block, 0, stream, ks, vs, n, 8 * p, args,
+                               kd, vd);
         }
         TK_HIP_CHECK(hipGetLastError());
         ks = kd;

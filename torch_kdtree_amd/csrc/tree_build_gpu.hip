@@ -17,8 +17,8 @@
 // group boxes straight into the device tree, and look at a sample of the cloud for exact ties.  The
 // trees of a forest are copied to the host.
 //
-// Bound: the depths above the tail, each a chain of short launches (500K points: 8 of 14 depths).
-// 500K points, depth 14, the whole build: 6.9 -> 1.33 ms against a form that sorted every depth over the
+// Bound: the depths above the tail, each a chain of short launches (500K points: 7 of 14 depths).
+// 500K points, depth 14, the whole build: 6.9 -> 1.16 ms against a form that sorted every depth over the
 // whole array and made records, boxes and the tie sample on the host.
 //
 // Exactness: the node sizes, split values and leaf contents equal those of the reference
@@ -239,28 +239,84 @@ std::vector<int32_t> leaf_offsets(int64_t n, int levels) {
     return off;
 }
 
-// Depths from l0 to the end for one node of depth l0 per workgroup, its points in LDS.  Descendant
-// node c of depth l0 + i keeps its points in slots [c * P, (c + 1) * P) of the sort array, P =
-// kTailPoints >> i (a node of at most kTailPoints points has descendants of at most P).  A slot holds the
-// sortable coordinate, then the point's rank in its node (the order of the depth before, which breaks
-// ties as a stable sort does) above its index in the workgroup's tile; empty slots sort last.  A
-// bitonic sort orders all descendants of a depth at once.
-constexpr int kTailPoints = 2048;
-constexpr int kTailBlock = 512;
+// The word of lane ^ M (M a power of two below 64) of the wavefront.
+template <int M>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    const int x = (int)v;
+    if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0xb1, 0xf, 0xf, false);       // quad_perm 1,0,3,2
+    else if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0x4e, 0xf, 0xf, false);  // quad_perm 2,3,0,1
+    else if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0x128, 0xf, 0xf, false); // row_ror 8
+    else if constexpr (M < 32) return (uint32_t)__builtin_amdgcn_ds_swizzle(x, (M << 10) | 0x1f);
+    else return (uint32_t)__shfl_xor(x, M, 64);
+}
+template <int M>
+__device__ __forceinline__ uint64_t lane_xor(uint64_t v) {
+    return (uint64_t)lane_xor<M>((uint32_t)(v >> 32)) << 32 | lane_xor<M>((uint32_t)v);
+}
+
+// Depths from l0 to the end for one node of depth l0 per workgroup.  Descendant node c of depth l0 + i
+// keeps its points in slots [c * P, (c + 1) * P), P = kTailPoints >> i (a node of at most kTailPoints points
+// has descendants of at most P).  A slot holds the sortable coordinate and a tag: the point's rank in its
+// node (the order of the depth before, which breaks ties as a stable sort does) above its index in the
+// workgroup's tile; empty slots sort last.  A bitonic sort orders all descendants of a depth at once, each
+// thread holding kTailItems consecutive slots in registers: exchanges within them are register moves,
+// within a wavefront lane permutations, and only the few of 256 slots and more go through LDS.  Bound by
+// VALU issue (500K points: 138 us for 7 depths from nodes of 3,907; with every exchange in LDS 137 us for 6 from
+// nodes of 1,954, and one more 120 us depth over the whole array).
+constexpr int kTailPoints = 4096;
+constexpr int kTailItems = 4;
+constexpr int kTailBlock = kTailPoints / kTailItems;
 constexpr uint32_t kTailEmpty = 0xffffffffu;
 
 template <typename T>
 using Sortable = decltype(sortable(T()));
+
+// (key, tag) of the slot pair's other element, and which of the two this slot keeps.
+template <typename K>
+__device__ __forceinline__ void keep_one(K& k, uint32_t& t, K ok, uint32_t ot, bool want_min) {
+    const bool less = k < ok || (k == ok && t < ot);
+    const bool take = less != want_min;  // (an empty slot equals only empty slots: either choice is the same)
+    k = take ? ok : k;
+    t = take ? ot : t;
+}
+
+// Exchanges at distance J slots of a bitonic stage with runs of `run` slots (whole descendants, run == P,
+// ascending; e0 = the thread's first slot).
+template <int J, typename K>
+__device__ __forceinline__ void bitonic_step(K (&k)[kTailItems], uint32_t (&t)[kTailItems], int e0, int run, int P) {
+    if constexpr (J < kTailItems) {
+#pragma unroll
+        for (int u = 0; u < kTailItems; ++u) {
+            if (u & J) continue;
+            const bool up = ((e0 + u) & run) == 0 || run == P;
+            K ka = k[u], kb = k[u | J];
+            uint32_t ta = t[u], tb = t[u | J];
+            const bool swap = (ka > kb || (ka == kb && ta > tb)) == up;
+            k[u] = swap ? kb : ka;
+            k[u | J] = swap ? ka : kb;
+            t[u] = swap ? tb : ta;
+            t[u | J] = swap ? ta : tb;
+        }
+    } else {
+        constexpr int M = J / kTailItems;
+        const bool low = (e0 & J) == 0;
+#pragma unroll
+        for (int u = 0; u < kTailItems; ++u) {
+            const bool up = ((e0 + u) & run) == 0 || run == P;
+            keep_one(k[u], t[u], lane_xor<M>(k[u]), lane_xor<M>(t[u]), low == up);
+        }
+    }
+}
 
 template <typename T>
 __global__ __launch_bounds__(kTailBlock) void gb_tail_kernel(const T* __restrict__ pts, int dims, uint32_t* perm,
                                                              ForestDev f, int l0, const int64_t* __restrict__ task_base,
                                                              T* __restrict__ split, int32_t* __restrict__ flags) {
     using K = Sortable<T>;
-    __shared__ K key[kTailPoints];
-    __shared__ uint32_t tag[kTailPoints];   // rank << 16 | tile index
-    __shared__ uint32_t point[kTailPoints]; // the tile's points (arena indices)
-    const int t = threadIdx.x;
+    __shared__ K s_key[kTailPoints];
+    __shared__ uint32_t s_tag[kTailPoints];  // rank << 16 | tile index
+    __shared__ uint32_t point[kTailPoints];  // the tile's points (arena indices)
+    const int t = threadIdx.x, e0 = t * kTailItems;
     const int c = tree_of(task_base, f.nc, blockIdx.x);
     const uint32_t seg = (uint32_t)((int64_t)blockIdx.x - task_base[c]);
     int64_t off, cnt;
@@ -268,53 +324,65 @@ __global__ __launch_bounds__(kTailBlock) void gb_tail_kernel(const T* __restrict
     const int64_t first = f.base[c] + off;
     const int n = (int)cnt;
     const int levels = f.levels[c];
-    for (int e = t; e < kTailPoints; e += kTailBlock) {
-        if (e < n) point[e] = perm[first + e];
-        tag[e] = e < n ? ((uint32_t)e << 16 | (uint32_t)e) : kTailEmpty;
-    }
+    for (int e = t; e < n; e += kTailBlock) point[e] = perm[first + e];
+    K key[kTailItems];
+    uint32_t tag[kTailItems];
+#pragma unroll
+    for (int u = 0; u < kTailItems; ++u) tag[u] = e0 + u < n ? (uint32_t)(e0 + u) << 16 | (uint32_t)(e0 + u) : kTailEmpty;
     __syncthreads();
     int bad = 0;
     int P = kTailPoints;
     for (int l = l0; l < levels; ++l, P >>= 1) {
         const int axis = l % dims;
-        for (int e = t; e < kTailPoints; e += kTailBlock) {
-            K k = ~K(0);
-            if (tag[e] != kTailEmpty) {
-                const T x = pts[(size_t)point[tag[e] & 0xffffu] * dims + axis];
+#pragma unroll
+        for (int u = 0; u < kTailItems; ++u) {
+            key[u] = ~K(0);
+            if (tag[u] != kTailEmpty) {
+                const T x = pts[(size_t)point[tag[u] & 0xffffu] * dims + axis];
                 if (x != x) bad |= kFlagNan;
-                k = sortable(x);
+                key[u] = sortable(x);
             }
-            key[e] = k;
         }
-        __syncthreads();
-        for (int k = 2; k <= P; k <<= 1) {
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int i = t; i < kTailPoints / 2; i += kTailBlock) {
-                    const int a = 2 * i - (i & (j - 1)), b = a + j;
-                    const K ka = key[a], kb = key[b];
-                    const uint32_t ta = tag[a], tb = tag[b];
-                    const bool gt = ka > kb || (ka == kb && ta > tb);
-                    // ascending runs; whole descendants (k == P) always ascending
-                    if (gt == ((a & k) == 0 || k == P)) {
-                        key[a] = kb;
-                        key[b] = ka;
-                        tag[a] = tb;
-                        tag[b] = ta;
-                    }
+        for (int run = 2; run <= P; run <<= 1) {
+            for (int j = run >> 1; j >= 64 * kTailItems; j >>= 1) {
+                // distances beyond a wavefront's slots
+#pragma unroll
+                for (int u = 0; u < kTailItems; ++u) {
+                    s_key[e0 + u] = key[u];
+                    s_tag[e0 + u] = tag[u];
+                }
+                __syncthreads();
+                const bool low = (e0 & j) == 0;
+#pragma unroll
+                for (int u = 0; u < kTailItems; ++u) {
+                    const int o = (e0 + u) ^ j;
+                    const bool up = ((e0 + u) & run) == 0 || run == P;
+                    keep_one(key[u], tag[u], s_key[o], s_tag[o], low == up);
                 }
                 __syncthreads();
             }
+            if (run >= 256) bitonic_step<128>(key, tag, e0, run, P);
+            if (run >= 128) bitonic_step<64>(key, tag, e0, run, P);
+            if (run >= 64) bitonic_step<32>(key, tag, e0, run, P);
+            if (run >= 32) bitonic_step<16>(key, tag, e0, run, P);
+            if (run >= 16) bitonic_step<8>(key, tag, e0, run, P);
+            if (run >= 8) bitonic_step<4>(key, tag, e0, run, P);
+            if (run >= 4) bitonic_step<2>(key, tag, e0, run, P);
+            bitonic_step<1>(key, tag, e0, run, P);
         }
+#pragma unroll
+        for (int u = 0; u < kTailItems; ++u) s_tag[e0 + u] = tag[u];
+        __syncthreads();
         // medians, one descendant node per thread
         const int nodes = 1 << (l - l0);
         for (int s = t; s < nodes; s += kTailBlock) {
             int64_t o, m;
             node_range(n, l - l0, (uint32_t)s, o, m);
             const int mid = s * P + (int)(m >> 1);
-            const T hi = pts[(size_t)point[tag[mid] & 0xffffu] * dims + axis];
+            const T hi = pts[(size_t)point[s_tag[mid] & 0xffffu] * dims + axis];
             T med = hi;
             if ((m & 1) == 0) {
-                const T lo = pts[(size_t)point[tag[mid - 1] & 0xffffu] * dims + axis];
+                const T lo = pts[(size_t)point[s_tag[mid - 1] & 0xffffu] * dims + axis];
                 med = (lo + hi) * T(0.5);
             }
             if (!__builtin_isfinite(med)) bad |= kFlagSplit;
@@ -322,29 +390,25 @@ __global__ __launch_bounds__(kTailBlock) void gb_tail_kernel(const T* __restrict
         }
         __syncthreads();
         // ranks: the next depth's children take their slots, or the order goes out
-        uint32_t moved[kTailPoints / kTailBlock], slot[kTailPoints / kTailBlock];
 #pragma unroll
-        for (int u = 0; u < kTailPoints / kTailBlock; ++u) {
-            const int e = u * kTailBlock + t;
-            slot[u] = kTailEmpty;
-            if (tag[e] == kTailEmpty) continue;
-            const int s = e / P, r = e % P;
+        for (int u = 0; u < kTailItems; ++u) s_tag[e0 + u] = kTailEmpty;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kTailItems; ++u) {
+            if (tag[u] == kTailEmpty) continue;
+            const int s = (e0 + u) / P, r = (e0 + u) & (P - 1);
             int64_t o, m;
             node_range(n, l - l0, (uint32_t)s, o, m);
             if (l + 1 == levels) {
-                perm[first + o + r] = point[tag[e] & 0xffffu];
+                perm[first + o + r] = point[tag[u] & 0xffffu];
                 continue;
             }
             const int h = (int)(m >> 1), child = r < h ? 0 : 1, rank = r - child * h;
-            moved[u] = (uint32_t)rank << 16 | (tag[e] & 0xffffu);
-            slot[u] = (uint32_t)(s * P + child * (P >> 1) + rank);
+            s_tag[s * P + child * (P >> 1) + rank] = (uint32_t)rank << 16 | (tag[u] & 0xffffu);
         }
         __syncthreads();
-        for (int e = t; e < kTailPoints; e += kTailBlock) tag[e] = kTailEmpty;
-        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < kTailPoints / kTailBlock; ++u)
-            if (slot[u] != kTailEmpty) tag[slot[u]] = moved[u];
+        for (int u = 0; u < kTailItems; ++u) tag[u] = s_tag[e0 + u];
         __syncthreads();
     }
     if (bad) atomicOr(flags, bad);
