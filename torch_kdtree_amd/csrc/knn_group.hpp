@@ -46,7 +46,6 @@ __device__ __forceinline__ V per_word(const V& a, const V& b, F&& f) {
 
 constexpr int kDppRowShr1 = 0x111;
 constexpr int kDppRowBcast = 0x150;  // row_newbcast: lane n of each row of 16 to the whole row
-constexpr int kDppQuad3 = 0xff;      // quad_perm [3,3,3,3]
 
 // v of the previous lane of the group; `first` in the group's first lane (g == 0).
 template <int G, typename V>
@@ -59,20 +58,21 @@ __device__ __forceinline__ V group_prev(const V& v, const V& first, int g) {
     }
 }
 
-// v of the last lane of the group.
-template <int G, typename V>
-__device__ __forceinline__ V group_last(const V& v) {
+// v of lane I of the group.
+template <int G, int I, typename V>
+__device__ __forceinline__ V group_lane(const V& v) {
     return per_word(v, v, [](int, int s) {
-        if constexpr (G == 16) return dpp_i32<kDppRowBcast + 15>(s, s);
-        else if constexpr (G == 8) return dpp_i32<kDppRowBcast + 15, 0xc>(dpp_i32<kDppRowBcast + 7, 0x3>(s, s), s);
-        else return dpp_i32<kDppQuad3>(s, s);
+        if constexpr (G == 16) return dpp_i32<kDppRowBcast + I>(s, s);
+        else if constexpr (G == 8) return dpp_i32<kDppRowBcast + 8 + I, 0xc>(dpp_i32<kDppRowBcast + I, 0x3>(s, s), s);
+        else return dpp_i32<I * 0x55>(s, s);  // quad_perm [I,I,I,I]
     });
 }
 
-// v of lane `src` of the wavefront.
-template <typename V>
-__device__ __forceinline__ V lane_value(const V& v, int src) {
-    return per_word(v, v, [&](int, int s) { return __builtin_amdgcn_ds_bpermute(src << 2, s); });
+// v0 + v1 + .. + v(D-1) over the group's lanes 0..D-1, left to right.
+template <int G, int D, int I = 1, typename V>
+__device__ __forceinline__ V group_sum(const V& v, V s) {
+    if constexpr (I < D) return group_sum<G, D, I + 1>(v, s + group_lane<G, I>(v));
+    else return s;
 }
 
 // Bit g: p in lane g of this lane's group, whose first lane is `base`.
@@ -140,15 +140,15 @@ struct GroupShape {
     static constexpr int kU = kGroups ? kGroupRecs / G : G == 16 ? (kWideRec ? 1 : 2) : G == 8 ? (kWideRec ? 2 : 4) : 4;
 };
 
-// Axis of level l + r for 0 <= r <= 4, given a = axis of level l.
-template <int D>
-__device__ __forceinline__ int axis_below(int a, int r) {
-    int x = a + r;
-    if constexpr (D == 1) return 0;
-    if constexpr (D == 2) return x & 1;
-    if constexpr (D == 8) return x & 7;
-    x = x >= D ? x - D : x;
-    return x >= D ? x - D : x;
+// base[i] through a 32-bit byte offset, for the arrays of nodes and leaves (at most 2^25 entries of at most
+// 128 bytes): one shift beside the uniform base address.
+template <typename V>
+__device__ __forceinline__ V load_at(const V* __restrict__ base, int32_t i) {
+    return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + (uint32_t)i * (uint32_t)sizeof(V));
+}
+template <typename T, int D>
+__device__ __forceinline__ T node_box_dist(const unsigned char* __restrict__ boxes, int32_t node, const Pt<T, D>& q) {
+    return box_dist<T, D>(load_box<T, D>(boxes + (uint32_t)node * (uint32_t)BoxLayout<T, D>::kBytes, 0), q);
 }
 
 template <typename T, int D, int G, int E, bool kLower, bool kGroups>
@@ -161,9 +161,12 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
     constexpr int K = G * E;
     constexpr int S = G == 16 ? 4 : G == 8 ? 3 : 2;  // levels per descent round
     constexpr int CH = U * G;
-    static_assert(CH <= 32 && CH <= 2 * kRecPad, "candidate mask");
+    static_assert(CH <= 32 && G - 1 <= kRecPad, "candidate mask and padding records");
+    static_assert(D <= G, "a lane per axis");
     __shared__ T stage_d[QB * (CH + 1)];
     __shared__ int32_t stage_o[kLower ? QB * (CH + 1) : 1];
+    constexpr int kLevelQs = 24 + 4;  // kMaxLevels and the levels a descent round may look past them
+    __shared__ T s_q[QB * kLevelQs];
 
     const int g = (int)(threadIdx.x & (G - 1));
     const int gq = (int)threadIdx.x / G;                  // group of the block
@@ -201,13 +204,29 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
     } else {
         const int L = tv.levels;
         const int a_lp = axis_of_level<D>(L - 1);
+        // q by level, q[l mod D], for the descent (up to S levels past the last)
+        T* const s_qg = s_q + gq * kLevelQs;
+        for (int l = g; l < kLevelQs; l += G) s_qg[l] = ax_get(q, axis_of_level<D>(l));
         // this lane's place in the descent's subtree (1-based heap index g: depth r, offset g - 2^r)
         const int r = g ? 31 - __builtin_clz(g) : 0;
         const int off = g ? g - (1 << r) : 0;
-        [[maybe_unused]] Pt<T, D> pp = q;  // the reference policy's projected point (knn_tree.hpp)
-        uint32_t far_mask = 0;
+        // Lane i < D keeps axis i of the reference policy's projected point: pp, q, the levels from the
+        // leaf-parents up to the first of that axis, and as a mask the levels c above them of that axis.
+        [[maybe_unused]] const int ax_up = (a_lp - g + 2 * D * G) % D;
+        [[maybe_unused]] T qv = T(0), pp = T(0);
+        [[maybe_unused]] uint32_t ax_mask = 0;
+        if constexpr (!kLower) {
+            qv = ax_get(q, g < D ? g : 0);
+            pp = qv;
+            ax_mask = axis_levels<D>(ax_up);
+        }
+        // Level L - 1 - c is bit c, lane c of batch 0: far_c, the levels entered through their far child.
+        uint32_t far_c = 0;
         int32_t node = 0;
         int level = 0;
+        // Lanes past the path's levels (and with them the last lane when L < G) take the leaf's own box.
+        const int own_sh = g < L ? g : 0, own_xor = g < L ? 1 : 0;
+        wave_lds_sync();
 
         // Candidates of the records [c0, min(c0 + CH, end)): distances tested against the worst
         // at the chunk's start, then inserted in scan order (knn_tree.hpp's two-pass scan).
@@ -215,7 +234,7 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
             Rec<T, D> rec[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                // (at most G - 1 <= kRecPad records past the last point)
+                // (at most G - 1 records past the last point)
                 const int32_t s = c0 + u * G < end ? c0 + u * G + g : c0 + g;
                 rec[u] = load_rec<T, D>(tv.recs, s);
             }
@@ -223,19 +242,19 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
             uint32_t mask = 0;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int32_t s = c0 + u * G + g;
                 const T dd = sq_dist<T, D>(q, rec[u].c);
-                bool acc = s < end;
+                bool acc = dd < w;
                 if constexpr (kLower) {
+                    const int32_t s = c0 + u * G + g;
                     const int32_t o = RecLayout<T, D>::kHasIdx ? rec[u].o : load_i32_at(tv.shuffled, min(s, end - 1));
-                    acc = acc && (dd < w || (dd == w && o < wx));
+                    acc = acc || (dd == w && o < wx);
                     st_o[u * G + g] = o;
-                } else {
-                    acc = acc && dd < w;
                 }
                 mask |= group_ballot<G>(acc, base) << (u * G);
                 st_d[u * G + g] = dd;
             }
+            const int n = end - c0;  // only the leaf's records
+            mask &= n >= 32 ? ~0u : (1u << n) - 1u;
             if (mask) {
                 wave_lds_sync();
                 int j = __builtin_ctz(mask);
@@ -253,8 +272,8 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
                     dj = dn;
                     oj = on;
                 }
-                w = group_last<G>(kb.d[E - 1]);
-                if constexpr (kLower) wx = group_last<G>(kb.x[E - 1]);
+                w = group_lane<G, G - 1>(kb.d[E - 1]);
+                if constexpr (kLower) wx = group_lane<G, G - 1>(kb.x[E - 1]);
             }
             wave_lds_sync();
         };
@@ -281,75 +300,76 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
                 for (int32_t c0 = beg; c0 < end; c0 += CH) chunk(c0, end);
             }
         };
-        // Box distance of the far side at level j = L - 1 - c, for the lane's c = g + b*G; lanes whose
-        // level does not exist or was entered through its far child (not valid) take the leaf's own.
-        auto path_box = [&](int b, bool& valid) -> T {
-            const int c = g + b * G;
-            const int j = L - 1 - c;
-            valid = j >= 0 && !((far_mask >> (j & 31)) & 1u);
-            return aabb_bound<T, D>(tv.boxes, (valid ? ((node + 1) >> c) ^ 1 : node + 1) - 1, q);
-        };
-
         for (;;) {
             // down the near path to a leaf, S levels per round
-            int a = axis_of_level<D>(level);
             while (level < L) {
-                const bool in = level + r < L && g > 0;
-                const int32_t sub = in ? ((node + 1) << r) - 1 + off : node;
-                const T m = tv.split_at(sub);
-                const uint32_t lt = group_ballot<G>(ax_get(q, axis_below<D>(a, r)) < m, base);
-                int idx = 1;
-                const int steps = min(S, L - level);
+                // (lanes of levels past the last read a split value that no step uses)
+                const int32_t sub = min(((node + 1) << r) + (off - 1), tv.n_nodes - 1);
+                const T m = load_at(tv.split, sub);
+                const uint32_t ge = ~group_ballot<G>(s_qg[level + r] < m, base);
+                uint32_t idx = 1;
 #pragma unroll
-                for (int s = 0; s < S; ++s)
-                    if (s < steps) idx = 2 * idx + (((lt >> idx) & 1u) ? 0 : 1);
-                node = ((node + 1) << steps) - 1 + (idx - (1 << steps));
+                for (int s = 0; s < S; ++s) idx = 2 * idx + ((ge >> idx) & 1u);
+                const int steps = min(S, L - level);
+                idx >>= S - steps;
+                node = (int32_t)(((uint32_t)node << steps) + idx) - 1;
                 level += steps;
-                a = axis_below<D>(a, steps);
             }
-            const int32_t lp = (node - 1) >> 1;
+            const int32_t child1 = node + 1;  // 1-based
+            const int32_t lp = (child1 >> 1) - 1;
             const int32_t left_leaf = 2 * lp + 1 - tv.n_nodes;
-            const int32_t o0 = tv.leaf_begin(left_leaf), o1 = tv.leaf_begin(left_leaf + 1),
-                          o2 = tv.leaf_end(left_leaf + 1);
-            const bool right = node != 2 * lp + 1;
-            [[maybe_unused]] const T m_lp = kLower ? T(0) : tv.split_at(lp);
-            bool valid;
-            T tb = path_box(0, valid);
-            // the leaf's own box: the last lane has it when the path is shorter than the group
-            uint32_t hit = group_ballot<G>(passes(tb), base);
+            const int32_t o0 = load_at(tv.leaf_off, left_leaf), o1 = load_at(tv.leaf_off, left_leaf + 1),
+                          o2 = load_at(tv.leaf_off, left_leaf + 2);
+            const bool right = child1 & 1;
+            [[maybe_unused]] const T m_lp = kLower ? T(0) : load_at(tv.split, lp);
+            // box distances of the far sides at the path's last G levels, a level per lane
+            T tb = node_box_dist<T, D>(tv.boxes, ((child1 >> own_sh) ^ own_xor) - 1, q);
+            const uint32_t levels_here = L < G ? (1u << L) - 1u : (1u << G) - 1u;
+            uint32_t near = ~far_c & levels_here;
             bool own;
             if (L < G)
-                own = (hit >> (G - 1)) & 1u;
+                own = (group_ballot<G>(passes(tb), base) >> (G - 1)) & 1u;
             else
-                own = passes(aabb_bound<T, D>(tv.boxes, node, q));
+                own = passes(node_box_dist<T, D>(tv.boxes, node, q));
             if (own) scan(left_leaf + (right ? 1 : 0), right ? o1 : o0, right ? o2 : o1);
-            hit = group_ballot<G>(valid && passes(tb), base);
-            // the sibling leaf; there the reference's bound rounds differently from the box distance
-            if ((hit & 1u) && (kLower || proj_bound<T, D>(q, pp, a_lp, m_lp) < w)) {
+            uint32_t hit = group_ballot<G>(passes(tb), base) & near;
+            // The sibling leaf: there the reference's bound (v = pp - q, v[a] += m - pp[a] on the
+            // leaf-parents' axis a) rounds differently from the box distance.
+            bool looks = hit & 1u;
+            if constexpr (!kLower) {
+                if (looks) {
+                    T v = pp - qv;
+                    v = ax_up == 0 ? v + (m_lp - pp) : v;
+                    v = v * v;
+                    looks = group_sum<G, D>(v, group_lane<G, 0>(v)) < w;
+                }
+            }
+            if (looks) {
                 scan(left_leaf + (right ? 0 : 1), right ? o0 : o1, right ? o1 : o2);
-                hit = group_ballot<G>(valid && passes(tb), base);
+                hit = group_ballot<G>(passes(tb), base) & near;
             }
             hit &= ~1u;
             int b = 0;
             while (!hit && L > (b + 1) * G) {
                 ++b;
-                tb = path_box(b, valid);
-                hit = group_ballot<G>(valid && passes(tb), base);
+                const int c = g + b * G;
+                tb = node_box_dist<T, D>(tv.boxes, (c < L ? (child1 >> c) ^ 1 : child1) - 1, q);
+                hit = group_ballot<G>(passes(tb), base) & ~(far_c >> (b * G));
+                if (L < (b + 1) * G) hit &= (1u << (L - b * G)) - 1u;
             }
             if (!hit) break;
             // enter the far side of the deepest level that passes
             const int c = __builtin_ctz(hit) + b * G;
-            const int j = L - 1 - c;
-            const int32_t child = (node + 1) >> c;  // 1-based, on the path below level j
+            const int32_t child = child1 >> c;  // 1-based, on the path below that level
             if constexpr (!kLower) {
-#pragma unroll
-                for (int i = 0; i < D; ++i)
-                    if ((a_lp - i + D) % D < c) pp[i] = q[i];  // an axis of the c levels below j
-                ax_set(pp, axis_of_level<D>(j), tv.split_at((child >> 1) - 1));
+                // the c levels left reset pp on their axes, the entered one sets its own
+                const T m = load_at(tv.split, (child >> 1) - 1);
+                pp = ax_up < c ? qv : pp;
+                pp = (ax_mask >> c) & 1u ? m : pp;
             }
-            far_mask = (far_mask & ((1u << j) - 1u)) | (1u << j);
+            far_c = (far_c & ~((2u << c) - 1u)) | (1u << c);
             node = (child ^ 1) - 1;
-            level = j + 1;
+            level = L - c;
         }
     }
 
