@@ -226,6 +226,19 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
         int level = 0;
         // Lanes past the path's levels (and with them the last lane when L < G) take the leaf's own box.
         const int own_sh = g < L ? g : 0, own_xor = g < L ? 1 : 0;
+        // Box distances of the far sides on the path, batch b holding the levels c = b*G .. b*G + G - 1, one
+        // a lane.  With kKeep they are kept for the levels above the one last entered, where they still
+        // hold: batch 0 renews its lanes below `renew`, a later batch is renewed whole, when it is next
+        // needed, if its bit in `stale` is set.  For the 64-byte boxes of d = 8, whose loads (a line per
+        // lane) bound the search (500K queries, k = 32: 23.2 -> 19.0 ms); at d <= 3 the bookkeeping costs more
+        // than the loads (depth-13 tree, k = 8, 1M queries: 0.58 -> 0.63 ms).
+        constexpr bool kKeep = D > 3;
+        constexpr int NB = (24 + G - 1) / G;  // kMaxLevels
+        T tb[kKeep ? NB : 1];
+#pragma unroll
+        for (int b = 0; b < (kKeep ? NB : 1); ++b) tb[b] = T(0);
+        [[maybe_unused]] int renew = G;
+        [[maybe_unused]] uint32_t stale = ~0u;
         wave_lds_sync();
 
         // Candidates of the records [c0, min(c0 + CH, end)): distances tested against the worst
@@ -322,17 +335,17 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
                           o2 = load_at(tv.leaf_off, left_leaf + 2);
             const bool right = child1 & 1;
             [[maybe_unused]] const T m_lp = kLower ? T(0) : load_at(tv.split, lp);
-            // box distances of the far sides at the path's last G levels, a level per lane
-            T tb = node_box_dist<T, D>(tv.boxes, ((child1 >> own_sh) ^ own_xor) - 1, q);
+            if (!kKeep || g < renew || g >= L)
+                tb[0] = node_box_dist<T, D>(tv.boxes, ((child1 >> own_sh) ^ own_xor) - 1, q);
             const uint32_t levels_here = L < G ? (1u << L) - 1u : (1u << G) - 1u;
             uint32_t near = ~far_c & levels_here;
             bool own;
             if (L < G)
-                own = (group_ballot<G>(passes(tb), base) >> (G - 1)) & 1u;
+                own = (group_ballot<G>(passes(tb[0]), base) >> (G - 1)) & 1u;
             else
                 own = passes(node_box_dist<T, D>(tv.boxes, node, q));
             if (own) scan(left_leaf + (right ? 1 : 0), right ? o1 : o0, right ? o2 : o1);
-            uint32_t hit = group_ballot<G>(passes(tb), base) & near;
+            uint32_t hit = group_ballot<G>(passes(tb[0]), base) & near;
             // The sibling leaf: there the reference's bound (v = pp - q, v[a] += m - pp[a] on the
             // leaf-parents' axis a) rounds differently from the box distance.
             bool looks = hit & 1u;
@@ -346,20 +359,35 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
             }
             if (looks) {
                 scan(left_leaf + (right ? 0 : 1), right ? o0 : o1, right ? o1 : o2);
-                hit = group_ballot<G>(passes(tb), base) & near;
+                hit = group_ballot<G>(passes(tb[0]), base) & near;
             }
             hit &= ~1u;
-            int b = 0;
-            while (!hit && L > (b + 1) * G) {
-                ++b;
-                const int c = g + b * G;
-                tb = node_box_dist<T, D>(tv.boxes, (c < L ? (child1 >> c) ^ 1 : child1) - 1, q);
-                hit = group_ballot<G>(passes(tb), base) & ~(far_c >> (b * G));
-                if (L < (b + 1) * G) hit &= (1u << (L - b * G)) - 1u;
+            int cb = 0;  // first level of the batch that hit
+            const auto later_batch = [&](T& t, bool renew_it) {
+                const int c = g + cb;
+                if (renew_it) t = node_box_dist<T, D>(tv.boxes, (c < L ? (child1 >> c) ^ 1 : child1) - 1, q);
+                hit = group_ballot<G>(passes(t), base) & ~(far_c >> cb);
+                if (L < cb + G) hit &= (1u << (L - cb)) - 1u;
+            };
+            if constexpr (kKeep) {
+#pragma unroll
+                for (int b = 1; b < NB; ++b) {
+                    if (!hit && L > b * G) {
+                        cb = b * G;
+                        later_batch(tb[b], (stale >> b) & 1u);
+                        stale &= ~(1u << b);
+                    }
+                }
+            } else {
+                while (!hit && L > cb + G) {
+                    T t;
+                    cb += G;
+                    later_batch(t, true);
+                }
             }
             if (!hit) break;
             // enter the far side of the deepest level that passes
-            const int c = __builtin_ctz(hit) + b * G;
+            const int c = __builtin_ctz(hit) + cb;
             const int32_t child = child1 >> c;  // 1-based, on the path below that level
             if constexpr (!kLower) {
                 // the c levels left reset pp on their axes, the entered one sets its own
@@ -368,6 +396,10 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
                 pp = (ax_mask >> c) & 1u ? m : pp;
             }
             far_c = (far_c & ~((2u << c) - 1u)) | (1u << c);
+            if constexpr (kKeep) {
+                renew = c;
+                stale |= (1u << ((c + G - 1) / G)) - 1u;  // the batches that hold a level below c
+            }
             node = (child ^ 1) - 1;
             level = L - c;
         }
