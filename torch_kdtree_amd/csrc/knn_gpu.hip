@@ -444,24 +444,26 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 // ------------------------------------------------------------------------------------------
 // Query driver
 // ------------------------------------------------------------------------------------------
-// Lanes per query, measured on MI355X (float d = 3 unless said; times are whole queries without a
-// presort against one lane per query with it):
-// * k > 32 and d = 8: 16 at every size.  One lane's list does not fit its registers (100K queries, k = 100:
-//   0.99 ms; 19.3 ms with one lane's list in LDS), and at d = 8 the walks of 64 lanes part (500K
-//   queries, k = 32: 23.6 against 45.1 ms; 2M queries, k = 1: 23.5 against 32.9).
-// * few queries leave the chip idle with one lane each, and a search is then one chain of
-//   dependent loads, which more lanes shorten: k = 8, cloud of 100K points, 16 / 8 / 4 / 1 lanes:
-//   1,000 queries 19 / 25 / 37 / 100 us; 10,000 22 / 26 / 36 / 180; 65,537 64 / 54 / 54 / 197;
-//   300,000 232 / 186 / 167 / 274; 1M 695 / 550 / 476 / 461.  At k = 16: 300,000 306 / 261 / - / 356,
-//   1M 931 / 804 / - / 621; at k = 32: 300,000 525 / - / - / 616, 1M 1,657 / - / - / 1,209.
-//   Clustered clouds favour the groups longer (1M points, k = 16, 1M queries: 1,110 with 8 lanes
-//   against 1,197), uniform ones less.
-// * d = 1 and 2: 4 lanes longer (d = 2, k = 8, 1M queries: 253 against 289 us; 8M: 1,938 against 1,441).
-// * doubles: a lane's list takes twice the registers, so the groups hold longer (500K points N(0,1),
-//   500K queries, presorted: k = 1 0.42 against 0.53 ms, k = 16 0.88 against 1.43, k = 32 1.45 against
-//   2.28; uniform, 2M queries, k = 16: 2.11 against 1.96).
-// * trees of big leaves (record-group boxes), k <= 8: 4 lanes, presorted, at every larger size (4M points
-//   at depth 13, k = 8: 4M queries 3.48 against 3.92 ms, 16M 11.7 against 11.9).
+// Lanes per query, measured on MI355X (whole queries in us or ms; "/" separates the forms, "s" marks one
+// with the presort, which one lane always has).
+// * k > 32 and d = 8: 16 lanes at every size.  One lane's list does not fit its registers (100K queries, k =
+//   100: 0.85 ms; 19.3 ms with one lane's list in LDS), and at d = 8 the walks of 64 lanes part (500K
+//   queries, k = 32: 19 ms against 45).
+// * few queries leave the chip idle with one lane each, and a search is then one chain of dependent
+//   loads, which more lanes shorten.  d = 3, k = 8, 16 / 8 / 4 / 1 lanes: cloud of 100K points, 1,000 queries
+//   19 / 25 / 37 / 100 us; 30,000 32 / 31 / 35 / 146; 120,000 84 / 73 / 74 / 176; 300,000 188 / 160 / 150 / 223;
+//   600,000 355 / 294 / 274 / 326.  Larger calls, 4s / 1 lanes: 1M 427 / 425 (100K points), 533 / 553 (1M,
+//   uniform), 599 / 715 (1M on a surface), 637 / 854 (1M, clustered); 2M 978 / 937, 1,103 / 1,114, 1,096 / 1,312;
+//   4M 2,060 / 1,924.
+// * k = 16: 30,000 41 / 42 / - / 186; 120,000 110 / 108 / - / 224; 300,000 250 / 231 / - / 306.  8s / 1 lanes, 1M:
+//   636 / 579, 733 / 747, 865 / 989, 869 / 1,141; 2M 1,312 / 1,210, 1,526 / 1,497, 1,517 / 1,706.
+// * k = 32, 16 / 1: 120,000 204 / 351; 300,000 465 / 576; 16s / 1: 600,000 900 / 1,049; 1M 1,420 / 1,534; 2M 2,672 /
+//   2,644.
+// * d = 1 and 2, 4 / 1: d = 2, k = 8: 100,000 37 / 103; 1M 243 / 255; 3M 696 / 536.  d = 1, 4M: 559 / 629.
+// * doubles, a lane's list being twice the registers: k = 16, 16 / 8 / 1: 150,000 302 / 321 / 912; 16s / 8s / 1: 500,000
+//   777 / 788 / 1,450; 1.5M 1,937 / 1,890 / 2,428; 2M of a uniform cloud - / 2.11 / 1.96 ms.
+// * trees of big leaves (record-group boxes), k <= 8: 4s at every larger size (depth 13, k = 8: 1M of 1M points
+//   584 / 679; 4M of 4M points 3.48 / 3.92 ms, 16M 11.7 / 11.9).
 int search_lanes(const Tree& t, int64_t nq, int k) {
     const auto prebuilt = [&](int lanes) {
         return lanes == 16 || (t.dims <= 3 && (lanes == 1 ? k <= 32 : lanes == 4 ? k <= 8 : k <= 16));
@@ -469,14 +471,15 @@ int search_lanes(const Tree& t, int64_t nq, int k) {
     if (t.lanes && prebuilt(t.lanes)) return t.lanes;
     if (t.dims == 8 || k > 32) return 16;
     if (t.dtype == kF64) {
-        if (nq > 1500000) return 1;
-        return k > 16 || nq <= 150000 ? 16 : 8;
+        if (nq > 1750000) return 1;
+        return k > 16 || nq <= 500000 ? 16 : 8;
     }
     if (nq <= 24000) return 16;
-    if (k > 16) return nq <= 400000 ? 16 : 1;
-    if (k > 8) return nq <= 500000 ? 8 : 1;
-    if (nq <= 100000) return 8;
-    if (nq <= (t.dims <= 2 ? 1500000 : 700000)) return 4;
+    if (k > 16) return nq <= 1200000 ? 16 : 1;
+    if (k > 8) return nq <= 60000 ? 16 : nq <= 1200000 ? 8 : 1;
+    if (t.dims <= 2) return nq <= (t.dims == 1 ? 4000000 : 1250000) ? 4 : 1;
+    if (nq <= 250000) return 8;
+    if (nq <= 2250000) return 4;
     return t.dev && t.dev->group_boxes ? 4 : 1;
 }
 
@@ -487,23 +490,28 @@ constexpr int kMaxBucketBits = 22;
 
 inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-// The presort of a call.  Asked for by name it always runs.  Auto: only from kPresortMinQueries queries,
-// and only where the search gains more than the sort costs.  One lane per query needs the order to
-// keep its wavefront's walks together.  Groups do not, and gain only cache hits: at d = 8 (500K queries,
-// k = 32) 27.4 -> 23.6 ms, equal at 100K; for lists beyond 32 equal at 100K queries and 7.6 -> 6.4 ms at
-// 1M; at d <= 3 and 300K queries a loss (k = 16, clustered cloud of 1M points: 0.41 -> 0.46 ms), at
-// 500K doubles a gain (k = 16: 0.93 -> 0.88 ms).
-// The order: the space-filling curve at d <= 3; the near-leaf order at d = 8, where the curve over a
-// 3-bit-per-axis grid groups queries more coarsely.
+// Queries from which a group search gains more from the presort than the sort costs.  One lane per query
+// always needs the order, to keep its wavefront's walks together; groups gain cache hits.  Without / with:
+// d = 8, k = 32, 500K queries 27.4 / 23.6 ms, equal at 100K; k = 100, 1M 7.6 / 6.4 ms, equal at 100K; d = 3, k = 8: 600K
+// 384 / 365 us (1M points), 274 / 303 (100K points), 1M 618 / 533; k = 16: 300K 276 / 300, 600K 528 / 486; k = 32: 300K
+// 515 / 519, 600K 1,003 / 900; doubles, k = 16: 150K 302 / 320, 500K 835 / 777; d = 2, k = 8, 1M 243 / 267.
+int64_t group_presort_from(const Tree& t, int k) {
+    if (t.dims == 8) return 65536;
+    if (k > 32) return 131072;
+    if (t.dtype == kF64) return 400000;
+    if (t.dims <= 2 && k <= 8) return INT64_MAX;
+    return k > 16 ? 400000 : k > 8 ? 550000 : 700000;
+}
+
+// The presort of a call.  Asked for by name it always runs.  Auto: from kPresortMinQueries queries, and for
+// groups from group_presort_from.  The order: the space-filling curve at d <= 3; the near-leaf order at d = 8,
+// where the curve over a 3-bit-per-axis grid groups queries more coarsely.
 int presort_mode(const Tree& t, int64_t nq, int k, const QueryOpts& o) {
     if (nq <= 0) return kPresortOff;
     if (o.presort == kPresortAuto) {
         if (nq < kPresortMinQueries || t.levels <= 1) return kPresortOff;
         const bool exact = o.tie != kTieLowerIndex && !t.finite;
-        if (!exact && search_lanes(t, nq, k) > 1) {
-            const int64_t from = t.dims == 8 ? 65536 : k > 32 ? 131072 : t.dtype == kF64 ? 400000 : 600000;
-            if (nq < from) return kPresortOff;
-        }
+        if (!exact && search_lanes(t, nq, k) > 1 && nq < group_presort_from(t, k)) return kPresortOff;
         return t.dims == 8 ? kPresortLeaf : kPresortMorton;
     }
     if (o.presort != kPresortOff && o.presort != kPresortMorton && o.presort != kPresortLeaf)
