@@ -96,11 +96,11 @@ void enqueue_forward(BatchPlan& p, const void* q, void* dist, int32_t* idx, int6
                      void* dq, hipStream_t s) {
     if (p.total_q == 0) return;
     if (p.dtype == kF32) {
-        batch_presort_f32(p, static_cast<const float*>(q), s);
+        batch_presort_f32(p, static_cast<const float*>(q), false, s);
         batch_traverse_f32(p, static_cast<const float*>(q), static_cast<float*>(dist), idx, orig, emit,
                            static_cast<const float*>(g), static_cast<float*>(dq), s);
     } else {
-        batch_presort_f64(p, static_cast<const double*>(q), s);
+        batch_presort_f64(p, static_cast<const double*>(q), false, s);
         batch_traverse_f64(p, static_cast<const double*>(q), static_cast<double*>(dist), idx, orig, emit,
                            static_cast<const double*>(g), static_cast<double*>(dq), s);
     }
@@ -110,9 +110,9 @@ void enqueue_backward(BatchPlan& p, const void* q, const int32_t* idx, const voi
                       bool from_forward, hipStream_t s) {
     if (!from_forward && p.total_q > 0) {
         if (p.dtype == kF32)
-            batch_presort_f32(p, static_cast<const float*>(q), s);
+            batch_presort_f32(p, static_cast<const float*>(q), true, s);
         else
-            batch_presort_f64(p, static_cast<const double*>(q), s);
+            batch_presort_f64(p, static_cast<const double*>(q), true, s);
     }
     if (p.dtype == kF32)
         batch_backward_f32(p, static_cast<const float*>(q), idx, static_cast<const float*>(g), static_cast<float*>(dq),
@@ -289,7 +289,6 @@ BatchPlan* batch_create(const Tree* const* trees, int n_clouds, const int64_t* n
     dmalloc(&p->run_end, 4 * (size_t)p->total_ref);
     dmalloc(reinterpret_cast<unsigned char**>(&p->q_sorted), ts * (size_t)p->dims * nq);
     dmalloc(&p->keys, 4 * no);
-    dmalloc(&p->vals, 4 * no);
     dmalloc(&p->keys_s, 4 * no);
     dmalloc(&p->vals_s, 4 * no);
     p->radix_ws_bytes = std::max(radix_sort_workspace((int64_t)no), radix_sort_workspace((int64_t)nq));
@@ -325,7 +324,6 @@ void batch_free(BatchPlan* p) noexcept {
     dfree(p->q_sorted);
     dfree(p->g_sorted);
     dfree(p->keys);
-    dfree(p->vals);
     dfree(p->keys_s);
     dfree(p->vals_s);
     dfree(p->radix_ws);

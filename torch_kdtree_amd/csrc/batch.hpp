@@ -80,8 +80,7 @@ struct BatchPlan {
     void* q_sorted = nullptr;   // [total_q * dims] queries in sorted order
     void* g_sorted = nullptr;   // [total_out] upstream gradient by canonical slot (captured training steps)
     bool g_sorted_valid = false;  // the captured graph's forward writes g_sorted before its backward
-    uint32_t* keys = nullptr;   // [total_out] pairs (record, canonical slot)
-    uint32_t* vals = nullptr;
+    uint32_t* keys = nullptr;   // [total_out] the record of each canonical slot (pair keys)
     uint32_t* keys_s = nullptr;
     uint32_t* vals_s = nullptr;
     bool persistent = false;    // one work-queue traversal launch for every k bucket
@@ -112,8 +111,9 @@ void batch_launch(BatchPlan& p, hipStream_t s);
 
 // Per-dtype kernel launchers (batch_f32.hip / batch_f64.hip).
 void batch_init_qcloud(const BatchPlan& p, hipStream_t s);
-void batch_presort_f32(const BatchPlan& p, const float* q, hipStream_t s);
-void batch_presort_f64(const BatchPlan& p, const double* q, hipStream_t s);
+// with_rank: also plan.rank, which only the separate backward reads.
+void batch_presort_f32(const BatchPlan& p, const float* q, bool with_rank, hipStream_t s);
+void batch_presort_f64(const BatchPlan& p, const double* q, bool with_rank, hipStream_t s);
 // emit: also write the training outputs (the queries at their sorted positions and the
 // (record, canonical slot) pairs) for a following batch_backward_*(from_forward = true).
 // dq (with g, the upstream gradient of the distances, already in place): also write dL/dq.

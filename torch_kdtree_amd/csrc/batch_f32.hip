@@ -3,7 +3,9 @@
 
 namespace tk {
 
-void batch_presort_f32(const BatchPlan& p, const float* q, hipStream_t s) { batch_presort_t<float>(p, q, s); }
+void batch_presort_f32(const BatchPlan& p, const float* q, bool with_rank, hipStream_t s) {
+    batch_presort_t<float>(p, q, with_rank, s);
+}
 
 void batch_traverse_f32(const BatchPlan& p, const float* q, float* dist, int32_t* idx, int64_t* orig, bool emit,
                         const float* g, float* dq, hipStream_t s) {

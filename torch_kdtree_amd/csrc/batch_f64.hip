@@ -3,7 +3,9 @@
 
 namespace tk {
 
-void batch_presort_f64(const BatchPlan& p, const double* q, hipStream_t s) { batch_presort_t<double>(p, q, s); }
+void batch_presort_f64(const BatchPlan& p, const double* q, bool with_rank, hipStream_t s) {
+    batch_presort_t<double>(p, q, with_rank, s);
+}
 
 void batch_traverse_f64(const BatchPlan& p, const double* q, double* dist, int32_t* idx, int64_t* orig, bool emit,
                         const double* g, double* dq, hipStream_t s) {

@@ -68,13 +68,30 @@ struct BatchArgs {
     int32_t* __restrict__ out_i;
     int64_t* __restrict__ out_o;
     uint32_t* __restrict__ pair_keys;
-    uint32_t* __restrict__ pair_vals;
     T* __restrict__ q_sorted;
     int tag_shift;
     const T* __restrict__ fuse_g;
     T* __restrict__ fuse_dq;
     T* __restrict__ g_sorted;
 };
+
+// v[j] = p[j - pad] for the slots j >= pad (0 below); with vec in 16-byte loads.
+template <typename V, int K>
+__device__ __forceinline__ void load_slots(const V* __restrict__ p, bool vec, int pad, V (&v)[K]) {
+    constexpr int kPer = 16 / (int)sizeof(V);
+    if constexpr (K % kPer == 0) {
+        if (vec) {
+#pragma unroll
+            for (int j = 0; j < K; j += kPer) {
+                const uint4 w = *reinterpret_cast<const uint4*>(p + j);
+                __builtin_memcpy(&v[j], &w, 16);
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < K; ++j) v[j] = j >= pad ? p[j - pad] : V(0);
+}
 
 // The search of the query at sorted position tpos (in the k bucket K), with its outputs.
 template <typename T, int D, int K, bool kLower, int CH, int LD>
@@ -87,7 +104,6 @@ __device__ __forceinline__ void batch_lane(const BatchArgs<T>& ba, int64_t tpos,
     int32_t* __restrict__ out_i = ba.out_i;
     int64_t* __restrict__ out_o = ba.out_o;
     uint32_t* __restrict__ pair_keys = ba.pair_keys;
-    uint32_t* __restrict__ pair_vals = ba.pair_vals;
     T* __restrict__ q_sorted = ba.q_sorted;
     const int tag_shift = ba.tag_shift;
     const T* __restrict__ fuse_g = ba.fuse_g;
@@ -142,35 +158,32 @@ __device__ __forceinline__ void batch_lane(const BatchArgs<T>& ba, int64_t tpos,
 #pragma unroll
         for (int j = 0; j < K; ++j) orig[j] = load_i32_at(arena.shuffled, x[j]);
     }
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        if (j >= pad) {
-            out_d[ob + j - pad] = kb.dist(j);
-            out_i[ob + j - pad] = loc[j];
-            if (out_o) out_o[ob + j - pad] = kLower ? x[j] : orig[j];
-            if (pair_keys) {
-                pair_keys[sb + j - pad] = pair_key(cloud, loc[j], cd.rec_base, tag_shift);
-                pair_vals[sb + j - pad] = (uint32_t)(sb + j - pad);
-            }
-        }
-    }
+    // Rows without padding slots go out in 16-byte stores where they lie on 16 bytes (a cloud's rows start
+    // wherever the clouds before it end).
+    const auto vec = [&](const auto* p) { return pad == 0 && ((uintptr_t)p & 15u) == 0; };
+    store_slots<T, 0, K>(out_d + ob, vec(out_d + ob), pad, [&](int j) { return kb.dist(j); });
+    store_slots<int32_t, 0, K>(out_i + ob, vec(out_i + ob), pad, [&](int j) { return loc[j]; });
+    if (out_o)
+        store_slots<int64_t, 0, K>(out_o + ob, vec(out_o + ob), pad,
+                                   [&](int j) { return (int64_t)(kLower ? x[j] : orig[j]); });
+    if (pair_keys)
+        store_slots<uint32_t, 0, K>(pair_keys + sb, vec(pair_keys + sb), pad,
+                                    [&](int j) { return pair_key(cloud, loc[j], cd.rec_base, tag_shift); });
     // dL/dq of a training step whose upstream gradient is already in place (a captured step):
     // the terms of batch_grad_q_sorted_kernel, in neighbour order, without a second pass
     if (fuse_dq) {
         Rec<T, D> r[K];
         T gij[K];
 #pragma unroll
-        for (int j = 0; j < K; ++j) {
-            r[j] = load_rec<T, D>(arena.recs, cd.rec_base + loc[j]);
-            gij[j] = j >= pad ? fuse_g[ob + j - pad] : T(0);
-        }
+        for (int j = 0; j < K; ++j) r[j] = load_rec<T, D>(arena.recs, cd.rec_base + loc[j]);
+        load_slots<T, K>(fuse_g + ob, vec(fuse_g + ob), pad, gij);
+        if (g_sorted) store_slots<T, 0, K>(g_sorted + sb, vec(g_sorted + sb), pad, [&](int j) { return gij[j]; });
         T acc[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) acc[a] = T(0);
 #pragma unroll
         for (int j = 0; j < K; ++j) {
             if (j >= pad) {
-                if (g_sorted) g_sorted[sb + j - pad] = gij[j];
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
                     const T diff = q[a] - r[j].c[a];
@@ -291,7 +304,7 @@ __global__ __launch_bounds__(kBatchBlock) void batch_grad_q_pairs_kernel(
     const unsigned char* __restrict__ recs, const CloudDesc* __restrict__ clouds, const int32_t* __restrict__ qcloud,
     const uint32_t* __restrict__ rank, const T* __restrict__ queries, int64_t total_q, const int32_t* __restrict__ idx,
     const T* __restrict__ g, T* __restrict__ dq, T* __restrict__ q_sorted, uint32_t* __restrict__ keys,
-    uint32_t* __restrict__ vals, int tag_shift) {
+    int tag_shift) {
     const int64_t i = (int64_t)blockIdx.x * kBatchBlock + threadIdx.x;
     if (i >= total_q) return;
     const int32_t cloud = qcloud[i];
@@ -320,7 +333,6 @@ __global__ __launch_bounds__(kBatchBlock) void batch_grad_q_pairs_kernel(
         }
         if (q_sorted) {
             keys[sb + j] = pair_key(cloud, idx[ob + j], cd.rec_base, tag_shift);
-            vals[sb + j] = (uint32_t)(sb + j);
         }
     }
     if (dq) {
@@ -493,8 +505,9 @@ TreeView<T, true> batch_arena_view(const BatchPlan& p) {
 
 inline dim3 batch_grid(int64_t n) { return dim3((unsigned)((n + kBatchBlock - 1) / kBatchBlock)); }
 
+// with_rank: also each query row's position in the order (the separate backward scatters by it).
 template <typename T>
-void batch_presort_t(const BatchPlan& p, const T* q, hipStream_t s) {
+void batch_presort_t(const BatchPlan& p, const T* q, bool with_rank, hipStream_t s) {
 #define TK_DIMS(DD)                                                                                                  \
     case DD:                                                                                                         \
         hipLaunchKernelGGL((batch_bucket_kernel<T, DD>), batch_grid(p.total_q), dim3(kBatchBlock), 0, s, p.boxes,   \
@@ -511,6 +524,7 @@ void batch_presort_t(const BatchPlan& p, const T* q, hipStream_t s) {
     TK_HIP_CHECK(hipGetLastError());
     radix_sort_pairs(p.key, nullptr, p.key_s, reinterpret_cast<uint32_t*>(p.order), p.total_q, p.key_bits, p.radix_ws,
                      p.radix_ws_bytes, s);
+    if (!with_rank) return;
     hipLaunchKernelGGL(batch_rank_kernel, batch_grid(p.total_q), dim3(kBatchBlock), 0, s, p.order, p.total_q, p.rank);
     TK_HIP_CHECK(hipGetLastError());
 }
@@ -521,9 +535,8 @@ void batch_traverse_td(const BatchPlan& p, const T* q, T* dist, int32_t* idx, in
     // the captured training step also stores the upstream gradient by canonical slot
     T* gs = (emit && g && dq && p.g_sorted) ? static_cast<T*>(p.g_sorted) : nullptr;
     uint32_t* pk = emit ? p.keys : nullptr;
-    uint32_t* pv = emit ? p.vals : nullptr;
     T* qs = emit ? static_cast<T*>(p.q_sorted) : nullptr;
-    const BatchArgs<T> ba{batch_arena_view<T>(p), p.d_clouds, p.qcloud, q, p.order, dist, idx, orig, pk, pv, qs,
+    const BatchArgs<T> ba{batch_arena_view<T>(p), p.d_clouds, p.qcloud, q, p.order, dist, idx, orig, pk, qs,
                           p.pair_tag_shift, g, dq, gs};
     if (p.persistent) {
         // units of 64 queries per range, largest lists first (the longest work starts first)
@@ -630,11 +643,12 @@ void batch_backward_t(const BatchPlan& p, const T* q, const int32_t* idx, const 
         } else if (p.total_q > 0 && !from_forward && (dq || pairs)) {                                                \
             hipLaunchKernelGGL((batch_grad_q_pairs_kernel<T, DD>), batch_grid(p.total_q), dim3(kBatchBlock), 0, s,   \
                                p.recs, p.d_clouds, p.qcloud, p.rank, q, p.total_q, idx, g, dq,                       \
-                               pairs ? qs : nullptr, p.keys, p.vals, p.pair_tag_shift);                              \
+                               pairs ? qs : nullptr, p.keys, p.pair_tag_shift);                                      \
             TK_HIP_CHECK(hipGetLastError());                                                                         \
         }                                                                                                            \
         if (pairs) {                                                                                                 \
-            radix_sort_pairs(p.keys, p.vals, p.keys_s, p.vals_s, p.total_out, p.pair_bits,                           \
+            /* the canonical slots number the pairs: no values to read */                                             \
+            radix_sort_pairs(p.keys, nullptr, p.keys_s, p.vals_s, p.total_out, p.pair_bits,                          \
                              p.radix_ws, p.radix_ws_bytes, s);                                                       \
             hipLaunchKernelGGL(batch_zero_runs_kernel, batch_grid(p.total_ref), dim3(kBatchBlock), 0, s,             \
                                p.run_start, p.run_end, p.total_ref);                                                 \

@@ -1234,7 +1234,7 @@ __global__ __launch_bounds__(kBoxBlock) void bbox_kernel(const T* __restrict__ p
 // Morton code (always for the backward's canonical order).  Every workgroup reduces the partials,
 // then strides over the queries (at most kMaxKeyBlocks workgroups, so that the reduction stays small
 // beside the queries).
-constexpr int kMaxKeyBlocks = 4096;
+constexpr int kMaxKeyBlocks = 1024;
 inline unsigned key_blocks(int64_t nq) {
     const int64_t b = (nq + kBoxBlock - 1) / kBoxBlock;
     return (unsigned)(b > kMaxKeyBlocks ? kMaxKeyBlocks : b);

@@ -465,7 +465,14 @@ RadixLayout radix_layout(int64_t n) {
 
 }  // namespace
 
-size_t radix_sort_workspace(int64_t n) { return radix_layout(n).total; }
+// What any sort of up to n pairs takes (the largest sort of a path can take more than the smallest of the
+// next, and a workspace taken for n serves smaller sorts too).
+size_t radix_sort_workspace(int64_t n) {
+    size_t bytes = radix_layout(n).total;
+    if (n > kFewMax) bytes = std::max(bytes, radix_layout(kFewMax).total);
+    if (n > kLookBackMax) bytes = std::max(bytes, radix_layout(kLookBackMax).total);
+    return bytes;
+}
 
 void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out, uint32_t* vals_out,
                       int64_t n, int key_bits, void* workspace, size_t workspace_bytes, hipStream_t stream) {
