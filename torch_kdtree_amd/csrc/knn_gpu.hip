@@ -452,18 +452,19 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 // * few queries leave the chip idle with one lane each, and a search is then one chain of dependent
 //   loads, which more lanes shorten.  d = 3, k = 8, 16 / 8 / 4 / 1 lanes: cloud of 100K points, 1,000 queries
 //   19 / 25 / 37 / 100 us; 30,000 32 / 31 / 35 / 146; 120,000 84 / 73 / 74 / 176; 300,000 188 / 160 / 150 / 223;
-//   600,000 355 / 294 / 274 / 326.  Larger calls, 4s / 1 lanes: 1M 427 / 425 (100K points), 533 / 553 (1M,
-//   uniform), 599 / 715 (1M on a surface), 637 / 854 (1M, clustered); 2M 978 / 937, 1,103 / 1,114, 1,096 / 1,312;
-//   4M 2,060 / 1,924.
-// * k = 16: 30,000 41 / 42 / - / 186; 120,000 110 / 108 / - / 224; 300,000 250 / 231 / - / 306.  8s / 1 lanes, 1M:
-//   636 / 579, 733 / 747, 865 / 989, 869 / 1,141; 2M 1,312 / 1,210, 1,526 / 1,497, 1,517 / 1,706.
-// * k = 32, 16 / 1: 120,000 204 / 351; 300,000 465 / 576; 16s / 1: 600,000 900 / 1,049; 1M 1,420 / 1,534; 2M 2,672 /
-//   2,644.
-// * d = 1 and 2, 4 / 1: d = 2, k = 8: 100,000 37 / 103; 1M 243 / 255; 3M 696 / 536.  d = 1, 4M: 559 / 629.
+//   600,000 355 / 294 / 274 / 308.  Larger calls, 4s / 1 lanes: 1M 421 / 402 (100K points), 526 / 514 (1M,
+//   uniform), 584 / 611 (4M), 611 / 683 (1M on a surface), 624 / 816 (1M, clustered); 2M 1,017 / 886, 1,139 / 1,053,
+//   1,109 / 1,051, 1,117 / 1,257 (clustered); 4M 2,238 / 1,789.
+// * k = 16: 30,000 41 / 42 / - / 186; 120,000 108 / 111 / - / 219; 300,000 249 / 229 / - / 284.  8s / 1 lanes, 1M:
+//   650 / 567, 735 / 717, 838 / 820, 858 / 934, 836 / 1,105; 2M 1,317 / 1,172, 1,568 / 1,375, 1,524 / 1,450, 1,531 / 1,663.
+// * k = 32, 16 / 1: 120,000 201 / 344; 300,000 456 / 566; 16s / 1: 600,000 911 / 1,020; 1M 1,419 / 1,503; 2M 2,646 /
+//   2,578.
+// * d = 1 and 2, 4 / 1: d = 2, k = 8: 300,000 84 / 140; 1M 244 / 231; 2M 468 / 398; k = 4: 1M 194 / 207, 2M 371 / 314.
+//   d = 1, 4M: 559 / 629.
 // * doubles, a lane's list being twice the registers: k = 16, 16 / 8 / 1: 150,000 302 / 321 / 912; 16s / 8s / 1: 500,000
 //   777 / 788 / 1,450; 1.5M 1,937 / 1,890 / 2,428; 2M of a uniform cloud - / 2.11 / 1.96 ms.
 // * trees of big leaves (record-group boxes), k <= 8: 4s at every larger size (depth 13, k = 8: 1M of 1M points
-//   584 / 679; 4M of 4M points 3.48 / 3.92 ms, 16M 11.7 / 11.9).
+//   588 / 658; 4M of 4M points 3.48 / 3.92 ms, 16M 11.7 / 11.9).
 int search_lanes(const Tree& t, int64_t nq, int k) {
     const auto prebuilt = [&](int lanes) {
         return lanes == 16 || (t.dims <= 3 && (lanes == 1 ? k <= 32 : lanes == 4 ? k <= 8 : k <= 16));
@@ -476,10 +477,10 @@ int search_lanes(const Tree& t, int64_t nq, int k) {
     }
     if (nq <= 24000) return 16;
     if (k > 16) return nq <= 1200000 ? 16 : 1;
-    if (k > 8) return nq <= 60000 ? 16 : nq <= 1200000 ? 8 : 1;
-    if (t.dims <= 2) return nq <= (t.dims == 1 ? 4000000 : 1250000) ? 4 : 1;
+    if (k > 8) return nq <= 60000 ? 16 : nq <= 1000000 ? 8 : 1;
+    if (t.dims <= 2) return nq <= (t.dims == 1 ? 4000000 : 1000000) ? 4 : 1;
     if (nq <= 250000) return 8;
-    if (nq <= 2250000) return 4;
+    if (nq <= 1500000) return 4;
     return t.dev && t.dev->group_boxes ? 4 : 1;
 }
 
