@@ -403,7 +403,7 @@ def _extra_tree_build(np, torch, tk, workloads, dev, w, cpu_build_s, reps):
                                    "host_build_s": cpu_batch_s, "gpu_build_s": gpu_batch_s,
                                    "speedup": cpu_batch_s / gpu_batch_s},
             "note": "host build = the reference's algorithm, OpenMP over subtrees (one tree) or over trees (256); "
-                    "GPU build = one level-by-level radix-sort build, host copies and upload included"}
+                    "GPU build = one level-by-level radix-sort build, the tree left on the GPU (the batch trees copied to the host)"}
 
 
 def _parse():

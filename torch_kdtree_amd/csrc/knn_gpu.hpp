@@ -45,7 +45,8 @@ void export_tree_gpu(const Tree& t, void* points, int64_t* shuffled, hipStream_t
 void free_device_tree(Tree& t) noexcept;
 
 enum TiePolicy : int { kTieReference = 0, kTieLowerIndex = 1 };
-// Query presort: auto = Morton buckets when there are enough queries to matter.
+// Query presort: auto = a space-filling curve (d <= 3) or the near leaf (d = 8), where the order gains more
+// than the sort costs.
 enum PresortMode : int { kPresortAuto = -1, kPresortOff = 0, kPresortMorton = 1, kPresortLeaf = 2 };
 
 // Largest k served on the GPU (the reference's limit, src/kdtree_g.cu:283,421-422).
@@ -75,7 +76,7 @@ void query_gpu_noalloc(const Tree& t, const void* queries, int64_t nq, int k, vo
 // Prebuilt launch variants of the traversal kernel that an autotuner picks among: leaf-scan chunk
 // (records staged in LDS per pass), occupancy target (waves per SIMD) and threads per block.
 // Variant 0 is the built-in choice (StageBytes / TreeOccupancy in knn_tree.hpp, blocks of 128).
-// The others exist for float searches at d = 3 with lists of 8 or 16 entries (k = 5..16); any
+// The others exist for one-lane float searches at d = 3 with lists of 8 or 16 entries (k = 5..16); any
 // other search runs variant 0 whatever is asked.  Results never depend on the variant.
 struct TreeVariant {
     int chunk, waves, block;
@@ -141,8 +142,8 @@ size_t knn_backward_structured_workspace(int64_t nq, int32_t n, int k, int dims,
 
 // Stable LSD radix sort of (key, value) pairs of uint32 by the low key_bits bits of the keys
 // (radix_sort.hip).  Reads keys_in / vals_in, writes keys_out / vals_out (distinct from the
-// inputs; vals_in null: the values are 0..n-1); workspace of radix_sort_workspace(n) bytes.  Kernels only, so it can be captured in
-// a graph.  n <= 2^28.
+// inputs; vals_in null: the values are 0..n-1); workspace of radix_sort_workspace(n) bytes.  Kernels
+// only, so it can be captured in a graph.  n <= 2^28.
 size_t radix_sort_workspace(int64_t n);
 void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out, uint32_t* vals_out,
                       int64_t n, int key_bits, void* workspace, size_t workspace_bytes, hipStream_t stream);

@@ -277,15 +277,15 @@ def build_kd_tree(points_ref: Union[torch.Tensor, np.ndarray], device: torch.dev
         "lower_index": ties ordered by the lower original index.
     presort : "auto", "on"/"morton", "leaf" or "off"
         How GPU queries are ordered before the traversal (along a space-filling curve over their
-        positions, Hilbert for d <= 3 and Morton for d = 8, or by tree leaf); the order changes
-        speed only, never results.
+        positions, Hilbert for d <= 3 and Morton for d = 8, or by tree leaf); "auto" orders them where
+        that gains more than it costs.  The order changes speed only, never results.
     builder : "cpu" (default) or "gpu"
         "gpu" builds a GPU tree on the device.  It gives the same tree as the CPU build whenever no
         node has two points with equal coordinates on its split axis; points with such ties may be
         ordered and split differently (the reference orders them by an unstable sort), so
         structured indices can differ while the neighbour distances do not.
     variant : None (default) or int
-        Launch variant of the GPU traversal (``torch_knn.tree_variants()``): None takes the one
+        Launch variant of GPU traversals with one lane a query (``torch_knn.tree_variants()``): None takes the one
         ``autotune.tune`` stored for this dims, dtype and k (0, the built-in shape, without one).
         Results never depend on it.
 
