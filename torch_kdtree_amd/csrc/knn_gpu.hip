@@ -511,7 +511,7 @@ int presort_mode(const Tree& t, int64_t nq, int k, const QueryOpts& o) {
     if (nq <= 0) return kPresortOff;
     if (o.presort == kPresortAuto) {
         if (nq < kPresortMinQueries || t.levels <= 1) return kPresortOff;
-        const bool exact = o.tie != kTieLowerIndex && !t.finite;
+        const bool exact = o.tie != kTieLowerIndex && !(t.finite && t.split_bounds);
         if (!exact && search_lanes(t, nq, k) > 1 && nq < group_presort_from(t, k)) return kPresortOff;
         return t.dims == 8 ? kPresortLeaf : kPresortMorton;
     }

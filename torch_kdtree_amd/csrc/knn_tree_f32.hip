@@ -7,7 +7,7 @@ namespace tk {
 
 void launch_tree_search_f32(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, float* dist,
                             int32_t* idx, int64_t* orig, int tie, hipStream_t s) {
-    if (tie != kTieLowerIndex && !t.finite) {
+    if (tie != kTieLowerIndex && !(t.finite && t.split_bounds)) {
         launch_exact_search_t<float>(t, q, nq, order, k, dist, idx, orig, s);
         return;
     }

@@ -7,7 +7,7 @@ namespace tk {
 
 void launch_tree_search_f64(const Tree& t, const double* q, int64_t nq, const int32_t* order, int k, double* dist,
                             int32_t* idx, int64_t* orig, int tie, hipStream_t s) {
-    if (tie != kTieLowerIndex && !t.finite) {
+    if (tie != kTieLowerIndex && !(t.finite && t.split_bounds)) {
         launch_exact_search_t<double>(t, q, nq, order, k, dist, idx, orig, s);
         return;
     }

@@ -11,7 +11,7 @@ template <typename T>
 TreeView<T> tree_view(const Tree& t) {
     TreeView<T> v{static_cast<const T*>(t.dev->split), t.dev->recs, t.dev->leaf_off, t.dev->shuffled,
                   t.dev->inv_shuffled, t.dev->boxes, t.levels, t.n_nodes};
-    v.split_bounds = t.finite;
+    v.split_bounds = t.finite && t.split_bounds;
     v.lower_direct = t.lower_list == 2 || (t.lower_list == 0 && t.tie_prone);
     v.group_boxes = t.dev->group_boxes;
     v.group_base = t.dev->group_base;

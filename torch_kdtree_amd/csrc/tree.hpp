@@ -47,6 +47,10 @@ struct Tree {
     // can be NaN, and the reference's insertion (src/nndistance.hpp:41-85) takes a NaN distance
     // into the list; the searches then follow the reference step by step, without point boxes.
     bool finite = true;
+    // Every split value lies between its two sides' points on its axis, as every build makes it; an image that
+    // was written by other means need not.  GPU searches whose climbs take it for granted then leave the
+    // tree to the reference's own walk.  (Only set where `finite` is.)
+    bool split_bounds = true;
     // Launch variant of the GPU traversal (kTreeVariants in knn_gpu.hpp; 0 = the built-in choice).
     int variant = 0;
     // List of the GPU's lower-index float searches with 8 to 32 entries: 0 = chosen from the cloud

@@ -84,7 +84,7 @@ struct Builder {
 // Point bounding boxes: leaves from their points, internal nodes as the union of their children.
 // NaN coordinates are left out of the boxes (a NaN distance is never below a bound, and the
 // searches that meet one, on trees that are not `finite`, use no boxes under the reference tie
-// policy).  Also sets t.finite: every coordinate and every split value finite.
+// policy).  Also sets t.finite (every coordinate and every split value finite) and t.split_bounds.
 template <typename T, int D>
 void compute_aabb(Tree& t, int n_threads) {
     const int32_t nn = t.n_nodes, nl = t.n_leaves;
@@ -121,6 +121,17 @@ void compute_aabb(Tree& t, int n_threads) {
     const T* split = t.split_ptr<T>();
     for (int32_t i = 0; i < nn && finite; ++i) finite = std::isfinite(split[i]);
     t.finite = finite;
+    bool bounds = true;
+    for (int32_t i = 0, a = 0, next = 1; i < nn && finite && bounds; ++i) {
+        if (i == next) {  // (the first node of the next depth)
+            next = 2 * next + 1;
+            a = (a + 1) % D;
+        }
+        const T* l = box + (size_t)(2 * i + 1) * 2 * D;
+        const T* r = box + (size_t)(2 * i + 2) * 2 * D;
+        bounds = l[D + a] <= split[i] && split[i] <= r[a];  // (an empty side's box is +inf .. -inf)
+    }
+    t.split_bounds = bounds;
 }
 
 template <typename T, int D>
