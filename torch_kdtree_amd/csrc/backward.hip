@@ -322,8 +322,8 @@ void backward_typed(const T* q, const T* ref, int64_t nq, int32_t n, int k, cons
     const int parts = box_parts(n);
     hipLaunchKernelGGL((bbox_kernel<T, D>), dim3(parts), dim3(kBoxBlock), 0, s, ref, (int64_t)n, box);
     const int bits = canonical_morton_bits(nq, D);
-    hipLaunchKernelGGL((morton_bucket_kernel<T, D>), dim3(key_blocks(nq)), dim3(kBoxBlock), 0, s, q, nq, box, parts,
-                       bits, qkey, false);
+    hipLaunchKernelGGL((morton_bucket_kernel<T, D, false>), dim3(key_blocks(nq)), dim3(kBoxBlock), 0, s, q, nq, box, parts,
+                       bits, qkey);
     TK_HIP_CHECK(hipGetLastError());
     radix_sort_pairs(qkey, nullptr, qkey_s, order, nq, bits * D, ws + l.temp, l.temp_bytes, s);
     // dL/dq, canonical copies and pairs; pairs sorted by reference index; dL/dr per reference point

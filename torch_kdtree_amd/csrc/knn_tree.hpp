@@ -1111,64 +1111,94 @@ struct MortonBits {
     static constexpr int kBuckets = 1 << (kBits * D);
 };
 
-// Morton code of q's cell; lo/hi are the box, converted to float.  Queries outside the box fall
-// into the boundary cells.
-template <typename T, int D>
-__device__ __forceinline__ uint32_t morton_cell(const float* lo, const float* hi, int bits, const T* __restrict__ q) {
-    const float cells = (float)(1 << bits);
-    uint32_t code = 0;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-        const float scale = hi[a] > lo[a] ? cells / (hi[a] - lo[a]) : 0.0f;
-        const float x = ((float)q[a] - lo[a]) * scale;
-        const uint32_t g = (uint32_t)fminf(fmaxf(x, 0.0f), cells - 1.0f);
-        for (int b = 0; b < bits; ++b) code |= ((g >> b) & 1u) << (b * D + a);
+// Bits 0, 1, 2, .. of v at bits 0, D, 2D, .. (D = 2: 16 of them, D = 3: 10).
+template <int D>
+__host__ __device__ __forceinline__ uint32_t spread_bits(uint32_t v) {
+    static_assert(D == 2 || D == 3, "interleaves of two and three axes");
+    if constexpr (D == 2) {
+        v = (v | (v << 8)) & 0x00ff00ffu;
+        v = (v | (v << 4)) & 0x0f0f0f0fu;
+        v = (v | (v << 2)) & 0x33333333u;
+        v = (v | (v << 1)) & 0x55555555u;
+    } else {
+        v = (v | (v << 16)) & 0x030000ffu;
+        v = (v | (v << 8)) & 0x0300f00fu;
+        v = (v | (v << 4)) & 0x030c30c3u;
+        v = (v | (v << 2)) & 0x09249249u;
     }
-    return code;
+    return v;
 }
 
-// Hilbert index of q's cell in the same grid as morton_cell: the cell's integer coordinates go
-// through Skilling's transpose transform (J. Skilling, "Programming the Hilbert curve", AIP Conf.
-// Proc. 707, 2004: undo the excess work, then Gray-encode), and the transposed coordinates are
-// interleaved most significant bit first.  Consecutive indices are adjacent cells, which the
-// Z-order's jumps between blocks of cells are not.
+// Integer coordinates of q's cell; lo/hi are the box, converted to float.  Queries outside the box fall
+// into the boundary cells.
 template <typename T, int D>
-__device__ __forceinline__ uint32_t hilbert_cell(const float* lo, const float* hi, int bits, const T* __restrict__ q) {
+__device__ __forceinline__ void grid_cell(const float* lo, const float* hi, int bits, const T* __restrict__ q,
+                                          uint32_t (&x)[D]) {
     const float cells = (float)(1 << bits);
-    uint32_t x[D];
 #pragma unroll
     for (int a = 0; a < D; ++a) {
         const float scale = hi[a] > lo[a] ? cells / (hi[a] - lo[a]) : 0.0f;
         const float v = ((float)q[a] - lo[a]) * scale;
         x[a] = (uint32_t)fminf(fmaxf(v, 0.0f), cells - 1.0f);
     }
-    if (bits > 0) {
-        const uint32_t m = 1u << (bits - 1);
-        for (uint32_t qb = m; qb > 1; qb >>= 1) {
-            const uint32_t p = qb - 1;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                if (x[a] & qb) {
-                    x[0] ^= p;
-                } else {
-                    const uint32_t t = (x[0] ^ x[a]) & p;
-                    x[0] ^= t;
-                    x[a] ^= t;
-                }
-            }
-        }
-#pragma unroll
-        for (int a = 1; a < D; ++a) x[a] ^= x[a - 1];
-        uint32_t t = 0;
-        for (uint32_t qb = m; qb > 1; qb >>= 1)
-            if (x[D - 1] & qb) t ^= qb - 1;
-#pragma unroll
-        for (int a = 0; a < D; ++a) x[a] ^= t;
-    }
+}
+
+// Morton code of q's cell: bit b of axis a at bit b * D + a.
+template <typename T, int D>
+__device__ __forceinline__ uint32_t morton_cell(const float* lo, const float* hi, int bits, const T* __restrict__ q) {
+    uint32_t x[D];
+    grid_cell<T, D>(lo, hi, bits, q, x);
     uint32_t code = 0;
-    for (int b = bits - 1; b >= 0; --b) {
 #pragma unroll
-        for (int a = 0; a < D; ++a) code = (code << 1) | ((x[a] >> b) & 1u);
+    for (int a = 0; a < D; ++a) {
+        if constexpr (D == 1) {
+            code = x[a];
+        } else if constexpr (D <= 3) {
+            code |= spread_bits<D>(x[a]) << a;
+        } else {
+            for (int b = 0; b < bits; ++b) code |= ((x[a] >> b) & 1u) << (b * D + a);
+        }
+    }
+    return code;
+}
+
+// Hilbert index of a cell of the grid with kBits bits an axis: the cell's integer coordinates go
+// through Skilling's transpose transform (J. Skilling, "Programming the Hilbert curve", AIP Conf.
+// Proc. 707, 2004: undo the excess work, then Gray-encode), and the transposed coordinates are
+// interleaved most significant bit first.  Consecutive indices are adjacent cells, which the
+// Z-order's jumps between blocks of cells are not.  Bound by VALU issue; without branches, with the Gray
+// code's suffix parities and the interleave by doubling shifts: 16M queries, d = 3,
+// 127 -> 78 us against the loops over bits.
+template <int D, int kBits>
+__host__ __device__ __forceinline__ uint32_t hilbert_index(uint32_t (&x)[D]) {
+    static_assert(D <= 3 && kBits >= 1 && kBits <= (D == 1 ? 31 : D == 2 ? 16 : 10), "one, two and three axes");
+#pragma unroll
+    for (int k = kBits - 1; k > 0; --k) {
+        const uint32_t p = (1u << k) - 1u;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            // bit k of x[a] set: invert the low bits of x[0]; else exchange those of x[0] and x[a]
+            const uint32_t set = 0u - ((x[a] >> k) & 1u);
+            const uint32_t t = (x[0] ^ x[a]) & p & ~set;
+            x[0] ^= t | (p & set);
+            if (a > 0) x[a] ^= t;
+        }
+    }
+#pragma unroll
+    for (int a = 1; a < D; ++a) x[a] ^= x[a - 1];
+    uint32_t t = x[D - 1] >> 1;  // bit j becomes the parity of the bits above j
+    t ^= t >> 1;
+    t ^= t >> 2;
+    t ^= t >> 4;
+    t ^= t >> 8;
+    t ^= t >> 16;
+#pragma unroll
+    for (int a = 0; a < D; ++a) x[a] ^= t;
+    uint32_t code = 0;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        if constexpr (D == 1) code = x[a];
+        else code |= spread_bits<D>(x[a]) << (D - 1 - a);
     }
     return code;
 }
@@ -1247,7 +1277,7 @@ __global__ __launch_bounds__(kBoxBlock) void bbox_kernel(const T* __restrict__ p
     }
 }
 
-// Cell keys over the box of n_part partials (bbox_kernel): the Hilbert index when hilbert (the forward
+// Cell keys over the box of n_part partials (bbox_kernel): the Hilbert index with kHilbert (the forward
 // presort at d <= 3: plain workload traversal 7.78 ms against 7.88 with the Morton code, fp64
 // workload 1.41 against 1.49; at d = 8 the Morton code is faster, 90.6 against 92.2 ms), else the
 // Morton code (always for the backward's canonical order).  Every workgroup reduces the partials,
@@ -1258,10 +1288,10 @@ inline unsigned key_blocks(int64_t nq) {
     const int64_t b = (nq + kBoxBlock - 1) / kBoxBlock;
     return (unsigned)(b > kMaxKeyBlocks ? kMaxKeyBlocks : b);
 }
-template <typename T, int D>
+template <typename T, int D, bool kHilbert>
 __global__ __launch_bounds__(kBoxBlock) void morton_bucket_kernel(const T* __restrict__ queries, int64_t nq,
                                                                   const T* __restrict__ part, int n_part, int bits,
-                                                                  uint32_t* __restrict__ key, bool hilbert) {
+                                                                  uint32_t* __restrict__ key) {
     __shared__ T s_lo[kBoxBlock / 64][D], s_hi[kBoxBlock / 64][D];
     T blo[D], bhi[D];
 #pragma unroll
@@ -1285,8 +1315,13 @@ __global__ __launch_bounds__(kBoxBlock) void morton_bucket_kernel(const T* __res
     }
     const int64_t stride = (int64_t)gridDim.x * kBoxBlock;
     for (int64_t i = (int64_t)blockIdx.x * kBoxBlock + threadIdx.x; i < nq; i += stride)
-        key[i] = hilbert ? hilbert_cell<T, D>(lo, hi, bits, queries + i * D)
-                         : morton_cell<T, D>(lo, hi, bits, queries + i * D);
+        if constexpr (kHilbert) {
+            uint32_t x[D];
+            grid_cell<T, D>(lo, hi, MortonBits<D>::kBits, queries + i * D, x);
+            key[i] = hilbert_index<D, MortonBits<D>::kBits>(x);
+        } else {
+            key[i] = morton_cell<T, D>(lo, hi, bits, queries + i * D);
+        }
 }
 
 }  // namespace tk

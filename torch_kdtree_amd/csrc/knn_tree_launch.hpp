@@ -118,8 +118,9 @@ void launch_morton_bucket_t(const Tree& t, const T* q, int64_t nq, void* box, ui
 #define TK_DIMS(DD)                                                                                                  \
     case DD:                                                                                                         \
         hipLaunchKernelGGL((bbox_kernel<T, DD>), dim3(parts), dim3(kBoxBlock), 0, s, q, nq, part);                   \
-        hipLaunchKernelGGL((morton_bucket_kernel<T, DD>), dim3(key_blocks(nq)), dim3(kBoxBlock), 0, s, q, nq, part, \
-                           parts, MortonBits<DD>::kBits, key, DD <= TK_HILBERT_MAX_D);                              \
+        hipLaunchKernelGGL((morton_bucket_kernel<T, DD, (DD <= TK_HILBERT_MAX_D)>), dim3(key_blocks(nq)),           \
+                           dim3(kBoxBlock), 0, s, q, nq, part,                                                      \
+                           parts, MortonBits<DD>::kBits, key);                                                      \
         break;
     switch (t.dims) {
         TK_DIMS(1)
