@@ -159,7 +159,7 @@ BatchPlan* batch_create(const Tree* const* trees, int n_clouds, const int64_t* n
     std::unique_ptr<BatchPlan, void (*)(BatchPlan*)> p(new BatchPlan(), [](BatchPlan* x) { batch_free(x); });
     p->device = device;
     p->dtype = t0.dtype;
-    for (int c = 0; c < n_clouds; ++c) p->all_finite = p->all_finite && trees[c]->finite && trees[c]->split_bounds;
+    for (int c = 0; c < n_clouds; ++c) p->split_bounds = p->split_bounds && trees[c]->finite && trees[c]->split_bounds;
     p->dims = t0.dims;
     p->tie = tie;
     p->n_clouds = n_clouds;

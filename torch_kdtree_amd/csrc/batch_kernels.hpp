@@ -93,8 +93,18 @@ __device__ __forceinline__ void load_slots(const V* __restrict__ p, bool vec, in
     for (int j = 0; j < K; ++j) v[j] = j >= pad ? p[j - pad] : V(0);
 }
 
-// The search of the query at sorted position tpos (in the k bucket K), with its outputs.
-template <typename T, int D, int K, bool kLower, int CH, int LD>
+// The reference policy's register list (keys: record positions) behind the list interface of knn_search_one.
+template <typename T, int K>
+struct RecKeyRef {
+    KBest<T, K, false>& l;
+    __device__ __forceinline__ T worst() const { return l.worst(); }
+    __device__ __forceinline__ bool accepts(T dist, int32_t) const { return dist < l.worst(); }
+    __device__ __forceinline__ void insert(T dist, int32_t rec, int32_t) { l.insert(dist, rec); }
+};
+
+// The search of the query at sorted position tpos (in the k bucket K), with its outputs.  kWalk: by the
+// reference's own steps instead of the climb over point boxes (knn_batch_walk_kernel).
+template <typename T, int D, int K, bool kLower, int CH, int LD, bool kWalk = false>
 __device__ __forceinline__ void batch_lane(const BatchArgs<T>& ba, int64_t tpos, T* __restrict__ st_d,
                                            int32_t* __restrict__ st_o) {
     const TreeView<T, true>& arena = ba.arena;
@@ -127,11 +137,16 @@ __device__ __forceinline__ void batch_lane(const BatchArgs<T>& ba, int64_t tpos,
     int level;
     load_query<T, D>(queries, qi, q);
     lane_start<T, D, K, kLower>(tv, k, q, pp, kb, far_mask, node, level);
-    if (has_nan<T, D>(q))
+    if (has_nan<T, D>(q)) {
         nan_fill<T, D, K, kLower>(tv, q, k, kb);
-    else
+    } else if constexpr (kWalk) {
+        static_assert(!kLower, "the reference's steps under the reference policy");
+        RecKeyRef<T, K> ref{kb};
+        knn_search_one<T, D, false, false>(tv, q, ref);
+    } else {
         while (!lane_step<T, D, K, kLower, CH, LD>(tv, q, pp, kb, far_mask, node, level, st_d, st_o)) {
         }
+    }
     // keys: reference policy = arena record position, lower-index policy = the cloud's original index.
     // Every gather (index maps, and the neighbour records of the fused dL/dq) is issued for all K
     // slots before the first store or sum, so the K latencies overlap; padding slots read a valid
@@ -208,6 +223,17 @@ __global__ __launch_bounds__(kTreeBlock) TK_BATCH_OCCUPANCY(T, D, K, kLower) voi
     const int64_t t = xcd_tile(blockIdx.x, gridDim.x) * kTreeBlock + threadIdx.x;
     if (t >= count) return;
     batch_lane<T, D, K, kLower, CH, LD>(ba, begin + t, stage_d + threadIdx.x, stage_o + (kLower ? threadIdx.x : 0));
+}
+
+// The reference policy over clouds among which a split value does not bound its points (a loaded image may
+// hold one): the climb over point boxes would enter sides that the reference prunes, so every lane takes
+// the reference's own steps (knn_search_one without boxes), as knn_tree_exact_kernel does for one tree.  Every
+// k bucket runs the 32-entry list: no build makes such a tree, so one kernel a type and d is enough.
+template <typename T, int D>
+__global__ __launch_bounds__(kTreeBlock) void knn_batch_walk_kernel(BatchArgs<T> ba, int64_t begin, int64_t count) {
+    const int64_t t = xcd_tile(blockIdx.x, gridDim.x) * kTreeBlock + threadIdx.x;
+    if (t >= count) return;
+    batch_lane<T, D, kBatchMaxK, false, 1, 1, true>(ba, begin + t, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -499,7 +525,7 @@ __global__ __launch_bounds__(kBatchBlock) void batch_grad_r_kernel(const unsigne
 template <typename T>
 TreeView<T, true> batch_arena_view(const BatchPlan& p) {
     TreeView<T, true> v{static_cast<const T*>(p.split), p.recs, p.leaf_off, p.shuffled, p.inv_shuffled, p.boxes, 0, 0};
-    v.split_bounds = p.all_finite;
+    v.split_bounds = p.split_bounds;
     return v;
 }
 
@@ -538,6 +564,17 @@ void batch_traverse_td(const BatchPlan& p, const T* q, T* dist, int32_t* idx, in
     T* qs = emit ? static_cast<T*>(p.q_sorted) : nullptr;
     const BatchArgs<T> ba{batch_arena_view<T>(p), p.d_clouds, p.qcloud, q, p.order, dist, idx, orig, pk, qs,
                           p.pair_tag_shift, g, dq, gs};
+    if constexpr (!kLower) {
+        if (!p.split_bounds) {
+            for (const BatchPlan::Range& r : p.ranges) {
+                if (r.count == 0) continue;
+                hipLaunchKernelGGL((knn_batch_walk_kernel<T, D>), dim3((unsigned)((r.count + kTreeBlock - 1) / kTreeBlock)),
+                                   dim3(kTreeBlock), 0, s, ba, r.begin, r.count);
+                TK_HIP_CHECK(hipGetLastError());
+            }
+            return;
+        }
+    }
     if (p.persistent) {
         // units of 64 queries per range, largest lists first (the longest work starts first)
         BatchUnits u{};
