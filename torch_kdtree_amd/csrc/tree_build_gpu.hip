@@ -10,8 +10,8 @@
 //   3. a stable radix sort of the result by node (segment) number, which regroups the positions
 //      node by node with each node's points in coordinate order;
 //   4. the permutation is composed with that order, and each node's median is read off.
-// From the depth at which every node holds at most kTailPoints points, one kernel (gb_tail_kernel)
-// does all remaining depths: a workgroup takes a node and sorts its descendants' points in LDS by
+// From the depth at which every node of a tree holds at most kTailPoints points, one kernel (gb_tail_kernel)
+// does all its remaining depths: a workgroup takes a node and sorts its descendants' points in LDS by
 // (coordinate, previous position), the order the two stable sorts give.
 // A single tree stays on the GPU: kernels write its records, index maps, leaf offsets, point boxes and
 // group boxes straight into the device tree, and look at a sample of the cloud for exact ties.  The
@@ -112,12 +112,13 @@ enum : int32_t { kFlagNan = 1, kFlagCoord = 2, kFlagSplit = 4 };
 struct ForestDev {
     const int64_t* base;      // [nc + 1] first point of each tree in the arena
     const int32_t* levels;    // [nc]
+    const int32_t* tail;      // [nc] first depth that gb_tail_kernel does (its levels where there is none)
     const int64_t* split_base;  // [nc] first split value of each tree
     int nc;
 };
 
 // key[j] = word `word` (0 low, 1 high) of the sortable coordinate of position p = order[j] (or j);
-// positions of trees that are complete at this depth get key 0, so they keep their order.
+// positions of trees whose depths over the whole array are done get key 0, so they keep their order.
 template <typename T>
 __global__ __launch_bounds__(kGbBlock) void gb_key_kernel(const T* __restrict__ pts, int dims,
                                                           const uint32_t* __restrict__ perm,
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(kGbBlock) void gb_key_kernel(const T* __restrict__ 
     const uint32_t p = order ? order[j] : (uint32_t)j;
     const int c = tree_of(f.base, f.nc, p);
     uint32_t k = 0;
-    if (f.levels[c] > depth) {
+    if (f.tail[c] > depth) {
         const T x = pts[(size_t)perm[p] * dims + axis];
         if (x != x) atomicOr(flags, kFlagNan);
         if constexpr (sizeof(T) == 4) {
@@ -153,7 +154,7 @@ __global__ __launch_bounds__(kGbBlock) void gb_segment_kernel(const uint32_t* __
     const uint32_t p = order[j];
     const int c = tree_of(f.base, f.nc, p);
     const int64_t b = f.base[c];
-    const uint32_t s = f.levels[c] > depth ? segment_of((int64_t)p - b, f.base[c + 1] - b, depth) : 0u;
+    const uint32_t s = f.tail[c] > depth ? segment_of((int64_t)p - b, f.base[c + 1] - b, depth) : 0u;
     key[j] = seg_base[c] + s;
     val[j] = p;
 }
@@ -254,15 +255,15 @@ __device__ __forceinline__ uint64_t lane_xor(uint64_t v) {
     return (uint64_t)lane_xor<M>((uint32_t)(v >> 32)) << 32 | lane_xor<M>((uint32_t)v);
 }
 
-// Depths from l0 to the end for one node of depth l0 per workgroup.  Descendant node c of depth l0 + i
-// keeps its points in slots [c * P, (c + 1) * P), P = kTailPoints >> i (a node of at most kTailPoints points
-// has descendants of at most P).  A slot holds the sortable coordinate and a tag: the point's rank in its
-// node (the order of the depth before, which breaks ties as a stable sort does) above its index in the
-// workgroup's tile; empty slots sort last.  A bitonic sort orders all descendants of a depth at once, each
-// thread holding kTailItems consecutive slots in registers: exchanges within them are register moves,
-// within a wavefront lane permutations, and only the few of 256 slots and more go through LDS.  Bound by
-// VALU issue (500K points: 138 us for 7 depths from nodes of 3,907; with every exchange in LDS 137 us for 6 from
-// nodes of 1,954, and one more 120 us depth over the whole array).
+// Depths from l0 (ForestDev::tail) to the end for one node of depth l0 per workgroup.  Descendant node c of
+// depth l0 + i keeps its points in slots [c * P, (c + 1) * P), P = P0 >> i, where P0 <= kTailPoints is the
+// smallest power of two that holds the node (its descendants then have at most P points).  A slot holds the
+// sortable coordinate and a tag: the point's rank in its node (the order of the depth before, which breaks
+// ties as a stable sort does) above its index in the workgroup's tile; empty slots sort last.  A bitonic sort
+// orders all descendants of a depth at once, each thread holding kTailItems consecutive slots in registers:
+// exchanges within them are register moves, within a wavefront lane permutations, and only the few of 256
+// slots and more go through LDS.  Bound by VALU issue (500K points: 138 us for 7 depths from nodes of 3,907;
+// with every exchange in LDS 137 us for 6 from nodes of 1,954, and one more 120 us depth over the whole array).
 constexpr int kTailPoints = 4096;
 constexpr int kTailItems = 4;
 constexpr int kTailBlock = kTailPoints / kTailItems;
@@ -310,15 +311,18 @@ __device__ __forceinline__ void bitonic_step(K (&k)[kTailItems], uint32_t (&t)[k
 
 template <typename T>
 __global__ __launch_bounds__(kTailBlock) void gb_tail_kernel(const T* __restrict__ pts, int dims, uint32_t* perm,
-                                                             ForestDev f, int l0, const int64_t* __restrict__ task_base,
-                                                             T* __restrict__ split, int32_t* __restrict__ flags) {
+                                                             ForestDev f, const int64_t* __restrict__ task_base,
+                                                             int64_t task0, T* __restrict__ split,
+                                                             int32_t* __restrict__ flags) {
     using K = Sortable<T>;
     __shared__ K s_key[kTailPoints];
     __shared__ uint32_t s_tag[kTailPoints];  // rank << 16 | tile index
     __shared__ uint32_t point[kTailPoints];  // the tile's points (arena indices)
     const int t = threadIdx.x, e0 = t * kTailItems;
-    const int c = tree_of(task_base, f.nc, blockIdx.x);
-    const uint32_t seg = (uint32_t)((int64_t)blockIdx.x - task_base[c]);
+    const int64_t task = task0 + blockIdx.x;
+    const int c = tree_of(task_base, f.nc, task);
+    const uint32_t seg = (uint32_t)(task - task_base[c]);
+    const int l0 = f.tail[c];
     int64_t off, cnt;
     node_range(f.base[c + 1] - f.base[c], l0, seg, off, cnt);
     const int64_t first = f.base[c] + off;
@@ -332,6 +336,7 @@ __global__ __launch_bounds__(kTailBlock) void gb_tail_kernel(const T* __restrict
     __syncthreads();
     int bad = 0;
     int P = kTailPoints;
+    while (P > 1 && P / 2 >= n) P >>= 1;
     for (int l = l0; l < levels; ++l, P >>= 1) {
         const int axis = l % dims;
 #pragma unroll
@@ -741,32 +746,37 @@ struct ForestSort {
     void run(const T* pts, const int64_t* n_points, const int32_t* levels, int nc, int dims, T* split_out, hipStream_t s) {
         base.assign(nc + 1, 0);
         split_base.assign(nc, 0);
-        int max_levels = 0;
         for (int c = 0; c < nc; ++c) {
             base[c + 1] = base[c] + n_points[c];
             split_base[c] = n_split;
             n_split += total_nodes(levels[c]);
-            max_levels = std::max(max_levels, (int)levels[c]);
         }
         n = base[nc];
-        // depths [0, l0) are sorted over the whole array, the rest node by node in LDS
+        // Depths [0, tail) of a tree are sorted over the whole array, the rest node by node in LDS.  Each
+        // tree has its own: with the deepest tree's for all, the small clouds beside a big one came to the
+        // tail in nodes of a few points, a workgroup each (one cloud of 1M points and 200 of 2,048 with 12 levels,
+        // plan included: 23.3 ms, now 12.7; 14.6 with every depth over the whole array).
+        std::vector<int32_t> tail((size_t)nc);
+        std::vector<int64_t> tail_task((size_t)nc + 1, 0);
         int l0 = 0;
         for (int c = 0; c < nc; ++c) {
             int l = 0;
             while (l < levels[c] && ((n_points[c] + (int64_t(1) << l) - 1) >> l) > kTailPoints) ++l;
+            tail[(size_t)c] = l;
+            tail_task[(size_t)c + 1] = tail_task[(size_t)c] + (l < levels[c] ? int64_t(1) << l : 0);
             l0 = std::max(l0, l);
         }
-        // per depth: node numbering (segment bases) and median task bases
-        std::vector<uint32_t> seg_base((size_t)max_levels * nc);
-        std::vector<int64_t> task_base((size_t)max_levels * (nc + 1));
-        std::vector<uint64_t> seg_total(max_levels);
-        for (int l = 0; l < max_levels; ++l) {
+        // per depth of the first kind: node numbering (segment bases) and median task bases
+        std::vector<uint32_t> seg_base((size_t)l0 * nc);
+        std::vector<int64_t> task_base((size_t)l0 * (nc + 1));
+        std::vector<uint64_t> seg_total(l0);
+        for (int l = 0; l < l0; ++l) {
             uint64_t sb = 0;
             int64_t tb = 0;
             for (int c = 0; c < nc; ++c) {
                 seg_base[(size_t)l * nc + c] = (uint32_t)sb;
                 task_base[(size_t)l * (nc + 1) + c] = tb;
-                const bool active = levels[c] > l;
+                const bool active = tail[(size_t)c] > l;
                 sb += active ? (uint64_t(1) << l) : 1u;
                 tb += active ? (int64_t(1) << l) : 0;
             }
@@ -778,9 +788,11 @@ struct ForestSort {
         const size_t at_ints = pack.add(zeros.data(), zeros.size());
         const size_t at_base = pack.add(base.data(), base.size());
         const size_t at_levels = pack.add(levels, (size_t)nc);
+        const size_t at_tail = pack.add(tail.data(), tail.size());
         const size_t at_split = pack.add(split_base.data(), split_base.size());
         const size_t at_seg = pack.add(seg_base.data(), seg_base.size());
         const size_t at_task = pack.add(task_base.data(), task_base.size());
+        const size_t at_tail_task = pack.add(tail_task.data(), tail_task.size());
 
         size_t total = 0;
         const auto take = [&](size_t bytes) {
@@ -802,7 +814,7 @@ struct ForestSort {
         const unsigned char* dp = m + at_pack;
         ints = reinterpret_cast<int32_t*>(m + at_pack + at_ints);
         f = ForestDev{reinterpret_cast<const int64_t*>(dp + at_base), reinterpret_cast<const int32_t*>(dp + at_levels),
-                      reinterpret_cast<const int64_t*>(dp + at_split), nc};
+                      reinterpret_cast<const int32_t*>(dp + at_tail), reinterpret_cast<const int64_t*>(dp + at_split), nc};
         const uint32_t* d_seg = reinterpret_cast<const uint32_t*>(dp + at_seg);
         const int64_t* d_task = reinterpret_cast<const int64_t*>(dp + at_task);
         split = split_out ? split_out : reinterpret_cast<T*>(m + at_spl);
@@ -845,13 +857,14 @@ struct ForestSort {
                 TK_HIP_CHECK(hipGetLastError());
             }
         }
-        if (l0 < max_levels) {
-            const int64_t tasks = task_base[(size_t)l0 * (nc + 1) + nc];
-            if (tasks > 0) {
-                hipLaunchKernelGGL(gb_tail_kernel<T>, dim3((unsigned)tasks), dim3(kTailBlock), 0, s, pts, dims, perm, f, l0,
-                                   d_task + (size_t)l0 * (nc + 1), split, ints);
-                TK_HIP_CHECK(hipGetLastError());
-            }
+        // (a launch takes fewer than 2^32 threads; forests of very many small clouds have more workgroups than that)
+        constexpr int64_t kTailTasks = int64_t(1) << 21;
+        static_assert(kTailTasks * kTailBlock < (int64_t(1) << 32), "threads of a launch");
+        for (int64_t t0 = 0; t0 < tail_task[(size_t)nc]; t0 += kTailTasks) {
+            const unsigned tasks = (unsigned)std::min(kTailTasks, tail_task[(size_t)nc] - t0);
+            hipLaunchKernelGGL(gb_tail_kernel<T>, dim3(tasks), dim3(kTailBlock), 0, s, pts, dims, perm, f,
+                               reinterpret_cast<const int64_t*>(dp + at_tail_task), t0, split, ints);
+            TK_HIP_CHECK(hipGetLastError());
         }
     }
 };
