@@ -566,9 +566,11 @@ int canonical_morton_bits(int64_t nq, int dims) {
     return b;
 }
 
-// Queries are presorted and searched in slices of at most this many (the presort's radix sort
-// orders at most 2^28 pairs); queries are independent, so slicing changes no result.
-constexpr int64_t kQuerySlice = int64_t(1) << 28;
+// Queries are presorted and searched in slices of at most this many: the presort's radix sort orders at most
+// 2^28 pairs, and a launch takes fewer than 2^32 threads, of which a group search uses up to 16 a query.  Queries
+// are independent, so slicing changes no result.
+constexpr int64_t kQuerySlice = int64_t(1) << 27;
+static_assert(16 * kQuerySlice + kGroupBlock < (int64_t(1) << 32), "threads of a group search's launch");
 
 size_t query_gpu_workspace(const Tree& t, int64_t nq, const QueryOpts& o) {
     nq = std::min(nq, kQuerySlice);

@@ -131,8 +131,6 @@ struct GroupList {
 // Shape of a group search: U records per lane and chunk (U*G <= 32 candidates staged at a time); with
 // record-group boxes a chunk is one group of kGroupRecs records.
 // ---------------------------------------------------------------------------------------------
-constexpr int kGroupBlock = 256;
-
 template <typename T, int D, int G, bool kGroups>
 struct GroupShape {
     static constexpr int kQueries = kGroupBlock / G;  // per block
