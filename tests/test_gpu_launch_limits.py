@@ -1,4 +1,4 @@
-"""Calls whose lanes together would pass the 2^32 threads of one launch."""
+"""Calls whose lanes or words together would pass the 2^32 threads of one launch."""
 import numpy as np
 import pytest
 import torch
@@ -26,3 +26,21 @@ def test_group_search_of_more_than_2_28_queries(cuda):
     od, oi = oracle.OracleTree(ref, 5).search(qs, 1)
     assert_same(got_d, od, "distances")
     assert_same(got_i, tree.kdtree.get_shuffled_inds()[oi].astype(np.int64), "indices")
+
+
+def test_device_tree_of_2_32_coordinate_words(cuda):
+    """The largest GPU build in the widest records (2^28 points of 8 doubles): its structured points and
+    indices come from the device tree, one word of 2^32 after the other."""
+    n, levels = 1 << 28, 4
+    if torch.cuda.mem_get_info()[0] < (120 << 30):
+        pytest.skip("needs 120 GB of GPU memory")
+    ref = torch.rand((n, 8), dtype=torch.float64, generator=torch.Generator(device=cuda).manual_seed(9), device=cuda)
+    tree = tk.build_kd_tree(ref, levels=levels, builder="gpu")
+    seen = torch.zeros(n, dtype=torch.bool, device=cuda)
+    for s in range(0, n, 1 << 24):
+        idx = tree.shuffled_ind[s:s + (1 << 24)]
+        assert torch.equal(tree.structured_points[s:s + (1 << 24)], ref[idx]), s
+        seen[idx] = True
+    assert bool(seen.all())
+    del ref, tree, seen, idx
+    torch.cuda.empty_cache()

@@ -337,14 +337,17 @@ void ensure_host(const Tree& ct) {
     t.host_ready.store(true, std::memory_order_release);
 }
 
-// out[s] = coordinates of record s (words 32-bit words of each record), idx[s] = its original index.
+// out[s] = coordinates of record s (words 32-bit words of each record), idx[s] = its original index.  Threads
+// stride over the words, of which a tree can hold more than a launch takes threads.
+constexpr int64_t kExportBlocks = int64_t(1) << 22;
 __global__ __launch_bounds__(256) void export_kernel(const unsigned char* __restrict__ recs, int rec_words, int words,
                                                      const int32_t* __restrict__ shuffled, int64_t n,
                                                      uint32_t* __restrict__ out, int64_t* __restrict__ idx) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (out && i < n * words)
-        out[i] = reinterpret_cast<const uint32_t*>(recs)[(i / words) * rec_words + i % words];
-    if (idx && i < n) idx[i] = shuffled[i];
+    const int64_t stride = (int64_t)gridDim.x * 256, total = out ? n * words : n;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride) {
+        if (out) out[i] = reinterpret_cast<const uint32_t*>(recs)[(i / words) * rec_words + i % words];
+        if (idx && i < n) idx[i] = shuffled[i];
+    }
 }
 
 void export_tree_gpu(const Tree& t, void* points, int64_t* shuffled, hipStream_t stream) {
@@ -353,7 +356,8 @@ void export_tree_gpu(const Tree& t, void* points, int64_t* shuffled, hipStream_t
     DeviceGuard g(t.dev->device);
     const int words = (int)(dtype_size(t.dtype) * (size_t)t.dims / 4);
     const int64_t total = (int64_t)t.n_points * (points ? words : 1);
-    hipLaunchKernelGGL(export_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, t.dev->recs,
+    const int64_t blocks = std::min((total + 255) / 256, kExportBlocks);
+    hipLaunchKernelGGL(export_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, t.dev->recs,
                        t.dev->rec_bytes / 4, words, t.dev->shuffled, (int64_t)t.n_points,
                        static_cast<uint32_t*>(points), shuffled);
     TK_HIP_CHECK(hipGetLastError());
