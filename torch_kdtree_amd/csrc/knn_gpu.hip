@@ -323,17 +323,32 @@ void ensure_host(const Tree& ct) {
     DeviceGuard g(t.dev->device);
     const size_t n = (size_t)t.n_points, rb = (size_t)t.dev->rec_bytes;
     const size_t coord_bytes = dtype_size(t.dtype) * (size_t)t.dims;
+    // The arrays are made beside the tree and moved in whole: finish_tree also sets `finite` and `split_bounds`,
+    // which queries on other threads read meanwhile (the GPU build has set them already).
+    Tree h;
+    h.dtype = t.dtype;
+    h.dims = t.dims;
+    h.levels = t.levels;
+    h.n_points = t.n_points;
+    h.n_nodes = t.n_nodes;
+    h.n_leaves = t.n_leaves;
     std::vector<unsigned char> recs(n * rb);
-    t.split.resize((size_t)t.n_nodes * dtype_size(t.dtype));
-    t.leaf_off.resize((size_t)t.n_leaves + 1);
-    t.shuffled.resize(n);
-    t.points.resize(n * coord_bytes);
+    h.split.resize((size_t)t.n_nodes * dtype_size(t.dtype));
+    h.leaf_off.resize((size_t)t.n_leaves + 1);
+    h.shuffled.resize(n);
+    h.points.resize(n * coord_bytes);
     TK_HIP_CHECK(hipMemcpy(recs.data(), t.dev->recs, recs.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(t.split.data(), t.dev->split, t.split.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(t.leaf_off.data(), t.dev->leaf_off, 4 * t.leaf_off.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(t.shuffled.data(), t.dev->shuffled, 4 * n, hipMemcpyDeviceToHost));
-    for (size_t s = 0; s < n; ++s) std::memcpy(&t.points[s * coord_bytes], &recs[s * rb], coord_bytes);
-    finish_tree(t);
+    TK_HIP_CHECK(hipMemcpy(h.split.data(), t.dev->split, h.split.size(), hipMemcpyDeviceToHost));
+    TK_HIP_CHECK(hipMemcpy(h.leaf_off.data(), t.dev->leaf_off, 4 * h.leaf_off.size(), hipMemcpyDeviceToHost));
+    TK_HIP_CHECK(hipMemcpy(h.shuffled.data(), t.dev->shuffled, 4 * n, hipMemcpyDeviceToHost));
+    for (size_t s = 0; s < n; ++s) std::memcpy(&h.points[s * coord_bytes], &recs[s * rb], coord_bytes);
+    finish_tree(h);
+    t.axis.swap(h.axis);
+    t.split.swap(h.split);
+    t.leaf_off.swap(h.leaf_off);
+    t.points.swap(h.points);
+    t.shuffled.swap(h.shuffled);
+    t.aabb.swap(h.aabb);
     t.host_ready.store(true, std::memory_order_release);
 }
 
