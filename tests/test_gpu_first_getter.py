@@ -46,3 +46,35 @@ def test_first_getter_beside_queries(cuda, tie):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("getter", ["get_structured_points", "get_nodes", "save"])
+def test_first_getter_during_a_capture(cuda, tmp_path, getter):
+    """A stream is being captured meanwhile: the capture goes on, and the captured query replays."""
+    g = torch.Generator(device=cuda).manual_seed(3)
+    ref = torch.rand((20_000, 3), generator=g, device=cuda)
+    q = torch.rand((500, 3), generator=g, device=cuda)
+    tree = tk.build_kd_tree(ref, builder="gpu")
+    want_d, want_i = tree.query(q, nr_nns_searches=4)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        d, i = tree.query(q, nr_nns_searches=4)
+        if getter == "save":
+            tree.kdtree.save(str(tmp_path / "t.bin"))
+        else:
+            got = getattr(tree.kdtree, getter)()
+    for _ in range(3):
+        d.fill_(-1)
+        i.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(d, want_d) and torch.equal(i, want_i)
+    points = tree.structured_points.cpu().numpy()
+    if getter == "save":
+        loaded = tk.load_kd_tree(str(tmp_path / "t.bin"))
+        assert np.array_equal(loaded.structured_points.numpy(), points)
+    elif getter == "get_structured_points":
+        assert np.array_equal(got, points)
+    else:
+        assert got[2][0] == 0 and got[2][-1] == 20_000

@@ -314,6 +314,40 @@ void upload_tree(Tree& t, int device) {
     t.dev = d.release();
 }
 
+namespace {
+
+// Device-to-host copies that a stream capture elsewhere in the process does not see: on a stream of their own,
+// which waits for no other, with this thread's capture mode relaxed meanwhile (a copy on the null stream would
+// fail and end the capture).
+class QuietCopies {
+public:
+    QuietCopies() {
+        TK_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode_));
+        const hipError_t e = hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking);
+        if (e != hipSuccess) {
+            (void)hipThreadExchangeStreamCaptureMode(&mode_);
+            TK_HIP_CHECK(e);
+        }
+    }
+    ~QuietCopies() {
+        (void)hipStreamSynchronize(stream_);
+        (void)hipStreamDestroy(stream_);
+        (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    QuietCopies(const QuietCopies&) = delete;
+    QuietCopies& operator=(const QuietCopies&) = delete;
+    void copy(void* dst, const void* src, size_t bytes) {
+        TK_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_));
+        TK_HIP_CHECK(hipStreamSynchronize(stream_));
+    }
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    hipStream_t stream_ = nullptr;
+};
+
+}  // namespace
+
 void ensure_host(const Tree& ct) {
     if (ct.host_ready.load(std::memory_order_acquire)) return;
     Tree& t = const_cast<Tree&>(ct);  // the host arrays are a cache of the GPU copy
@@ -337,10 +371,13 @@ void ensure_host(const Tree& ct) {
     h.leaf_off.resize((size_t)t.n_leaves + 1);
     h.shuffled.resize(n);
     h.points.resize(n * coord_bytes);
-    TK_HIP_CHECK(hipMemcpy(recs.data(), t.dev->recs, recs.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(h.split.data(), t.dev->split, h.split.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(h.leaf_off.data(), t.dev->leaf_off, 4 * h.leaf_off.size(), hipMemcpyDeviceToHost));
-    TK_HIP_CHECK(hipMemcpy(h.shuffled.data(), t.dev->shuffled, 4 * n, hipMemcpyDeviceToHost));
+    {
+        QuietCopies q;
+        q.copy(recs.data(), t.dev->recs, recs.size());
+        q.copy(h.split.data(), t.dev->split, h.split.size());
+        q.copy(h.leaf_off.data(), t.dev->leaf_off, 4 * h.leaf_off.size());
+        q.copy(h.shuffled.data(), t.dev->shuffled, 4 * n);
+    }
     for (size_t s = 0; s < n; ++s) std::memcpy(&h.points[s * coord_bytes], &recs[s * rb], coord_bytes);
     finish_tree(h);
     t.axis.swap(h.axis);
