@@ -8,7 +8,7 @@ beyond N = 2^16 (488 points per leaf at N = 4M).  Here two choices are measured 
 * the launch variant of the traversal kernel (``torch_knn.tree_variants()``): the leaf-scan chunk
   staged in LDS per pass, the occupancy target in waves per SIMD and the threads per block.  The
   variants are prebuilt instantiations; the non-default ones exist for float searches at d = 3
-  with lists of 8 or 16 entries (k = 5..16).
+  with lists of 8 or 16 entries (k = 5..16) and one lane a query, the form that large calls take.
 
 :func:`tune` times queries over the candidates, checks that every candidate returns the same
 results, and stores the fastest in ``tuning.json`` next to this file (or the path in
@@ -131,12 +131,13 @@ def _time_query(tree, queries, k, repeats):
 def tune(points: torch.Tensor, queries: torch.Tensor, k: int, leaf_sizes=(8, 16, 24, 32, 48),
          variants=None, repeats: int = 3, write: bool = True, tie_break: str = "reference") -> dict:
     """Measures GPU queries of ``queries`` against ``points`` (k neighbours) for each leaf size with the
-    built-in launch shape, then each launch variant on the fastest depth, and keeps the fastest of
-    each.  Every variant's distances and indices must equal variant 0's on the same tree, and every
-    depth's distances must equal the first depth's (the neighbour sets are exact; only tie order and
-    structured indices depend on the tree); a mismatch raises.  With ``write`` the choice is stored
-    for this dims/dtype (leaf size, measured under the reference tie policy only) and, for the
-    tie policy ``tie_break``, list width (variant)."""
+    built-in launch shape, then each launch variant on the fastest depth with one lane a query (the
+    form that has variants), and keeps the fastest of each.  Every variant's distances and indices
+    must equal variant 0's on the same tree, and every depth's distances must equal the first depth's
+    (the neighbour sets are exact; only tie order and structured indices depend on the tree); a
+    mismatch raises.  With ``write`` the choice is stored for this dims/dtype (leaf size, measured
+    under the reference tie policy only) and, for the tie policy ``tie_break``, list width
+    (variant)."""
     from .nn_distance import build_kd_tree
     from . import torch_knn
 
@@ -158,6 +159,9 @@ def tune(points: torch.Tensor, queries: torch.Tensor, k: int, leaf_sizes=(8, 16,
         leaf_res[leaf] = {"levels": lv, "seconds": _time_query(tree, queries, k, repeats)}
     leaf_best = min(leaf_res, key=lambda s: leaf_res[s]["seconds"])
     tree = build_kd_tree(points, device=dev, levels=leaf_res[leaf_best]["levels"], variant=0, tie_break=tie_break)
+    # The variants are launch shapes of the search with one lane a query: queries that the lane rule would
+    # give several would all run the same group kernel, whatever the variant.
+    tree.kdtree.set_lanes(1)
     table = torch_knn.tree_variants()
     var_res, ref_out = {}, None
     for v in variants:
