@@ -24,11 +24,11 @@
 // and each pass clears the status words of the next.
 //
 // Bound: small sorts by the launches (about 4.6 us each), large ones by the passes' memory traffic (8M
-// pairs: 47 us to rank and write, 2.9 TB/s, and 14 to count).  The look-back costs a pass about 18 us once
-// a thousand tiles are in flight (each step back is a load past the L2), more than the two launches
-// it saves from about 2M pairs.  Against a three-kernel scan per pass (five
-// launches a pass): 4,096 pairs of 24-bit keys 57 -> 19 us, 65,537 74 -> 47, 1M 88 -> 71, 8M of 20 bits
-// 207 -> 178, 16M of 24 bits 414 -> 367.
+// pairs: 47 us to rank and write, 2.9 TB/s, and 14 to count).  The look-back costs a pass more the more tiles are in
+// flight (each step back is a load past the L2), which from 512K pairs is more than the two launches it saves.
+// Look-back with tiles of 4,096 pairs / three launches, us: 600K pairs of 8 / 24 bits 32 / 31, 62 / 59; 1M 33 / 29,
+// 69 / 60; 2M 45 / 30, 96 / 73.  Against a three-kernel scan per pass (five launches a pass): 4,096 pairs of 24-bit
+// keys 57 -> 19 us, 65,537 74 -> 37, 1M 87 -> 60, 2M 100 -> 73, 8M of 20 bits 207 -> 178, 16M of 24 bits 414 -> 367.
 #include <algorithm>
 
 #include "gpu_common.hpp"
@@ -38,16 +38,15 @@ namespace tk {
 namespace {
 
 constexpr int kRadixBlock = 256;
-constexpr int kRadixItems = 16;  // pairs per thread of a tile
-constexpr int kRadixTile = kRadixBlock * kRadixItems;
-// Smaller tiles for sorts whose 4,096-pair tiles would leave CUs idle (65,537 pairs 47 -> 37 us, 500K of
-// 32 bits 78 -> 73; 1M of 24 bits 71 -> 82: more tiles to look back over).
+constexpr int kRadixItems = 16;  // pairs per thread of a tile, three launches a pass
+// Look-back sorts take smaller tiles: 4,096 pairs a tile would leave CUs idle (65,537 pairs 47 -> 37 us, 500K of 32
+// bits 78 -> 73).
 constexpr int kRadixItemsFew = 8;
-constexpr int64_t kFewMax = int64_t(512) << 10;
+constexpr int kRadixTile = kRadixBlock * kRadixItems;
+constexpr int kRadixTileFew = kRadixBlock * kRadixItemsFew;
+constexpr int64_t kLookBackMax = int64_t(512) << 10;
 constexpr int kRadixBins = 256;
 constexpr int kMaxPasses = 4;
-constexpr int64_t kLookBackMax = int64_t(2) << 20;
-constexpr int kCountBlocks = 512;  // most workgroups of the count kernel
 constexpr int kDirectParts = 32;   // up to this many, the pass kernels sum the workgroups' counts themselves
 
 constexpr int kSmallBlock = 512;
@@ -121,11 +120,11 @@ __device__ __forceinline__ int32_t scan_256(int32_t c, int32_t* tmp) {
     return base + inc - c;
 }
 
-// Digit counts of all passes, per workgroup: part[block][pass][digit].  Also clears the tickets and
+// Digit counts of all passes, per workgroup (one tile each): part[block][pass][digit].  Also clears the tickets and
 // the first pass's status words.
-template <int P, int kItems>
+template <int P>
 __global__ __launch_bounds__(kRadixBlock) void radix_count_kernel(const uint32_t* __restrict__ keys, int64_t n,
-                                                                  int32_t n_tiles, uint32_t* __restrict__ part,
+                                                                  uint32_t* __restrict__ part,
                                                                   uint32_t* __restrict__ tickets,
                                                                   uint32_t* __restrict__ status) {
     constexpr int kWaves = kRadixBlock / 64;
@@ -136,21 +135,19 @@ __global__ __launch_bounds__(kRadixBlock) void radix_count_kernel(const uint32_t
         for (int v = 0; v < kWaves; ++v) cnt[v][p][t] = 0;
     if (blockIdx.x == 0 && t < kMaxPasses) tickets[t] = 0;
     __syncthreads();
-    for (int32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        status[(int64_t)tile * kRadixBins + t] = 0;
-        const int64_t base = (int64_t)tile * (kRadixBlock * kItems);
-        uint32_t k[kItems];
+    status[(int64_t)blockIdx.x * kRadixBins + t] = 0;
+    const int64_t base = (int64_t)blockIdx.x * kRadixTileFew;
+    uint32_t k[kRadixItemsFew];
 #pragma unroll
-        for (int s = 0; s < kItems; ++s) {
-            const int64_t i = base + (int64_t)s * kRadixBlock + t;
-            k[s] = i < n ? keys[i] : 0u;
-        }
+    for (int s = 0; s < kRadixItemsFew; ++s) {
+        const int64_t i = base + (int64_t)s * kRadixBlock + t;
+        k[s] = i < n ? keys[i] : 0u;
+    }
 #pragma unroll
-        for (int s = 0; s < kItems; ++s) {
-            if (base + (int64_t)s * kRadixBlock + t < n) {
+    for (int s = 0; s < kRadixItemsFew; ++s) {
+        if (base + (int64_t)s * kRadixBlock + t < n) {
 #pragma unroll
-                for (int p = 0; p < P; ++p) count_digit(cnt[w][p], (k[s] >> (8 * p)) & (kRadixBins - 1));
-            }
+            for (int p = 0; p < P; ++p) count_digit(cnt[w][p], (k[s] >> (8 * p)) & (kRadixBins - 1));
         }
     }
     __syncthreads();
@@ -255,13 +252,13 @@ struct PassArgs {
 };
 
 // One pass.  vals_in null: the values are the pairs' indices.
-template <bool kLookBack, int kItems>
+template <bool kLookBack>
 __global__ __launch_bounds__(kRadixBlock) void radix_pass_kernel(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int64_t n, int shift, PassArgs args,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
     constexpr int kWaves = kRadixBlock / 64;
-    constexpr int kTile = kRadixBlock * kItems;
-    constexpr int kRounds = kItems;
+    constexpr int kRounds = kLookBack ? kRadixItemsFew : kRadixItems;
+    constexpr int kTile = kRadixBlock * kRounds;
     __shared__ uint32_t tile_k[kTile];           // the tile in digit order (stable)
     __shared__ uint32_t tile_v[kTile];
     __shared__ int32_t tile_start[kRadixBins];        // first tile slot of each digit
@@ -440,20 +437,19 @@ __global__ __launch_bounds__(256) void copy_u32_kernel(const uint32_t* __restric
 inline size_t a256(size_t b) { return (b + 255) & ~size_t(255); }
 
 struct RadixLayout {
-    int32_t n_tiles, n_parts;
+    int32_t n_tiles;
     size_t keys_tmp, vals_tmp, part, base, tickets, status[2], total;
 };
 
 RadixLayout radix_layout(int64_t n) {
     RadixLayout l{};
-    const int64_t tile = kRadixBlock * (n <= kFewMax ? kRadixItemsFew : kRadixItems);
-    l.n_tiles = (int32_t)std::max<int64_t>(1, (n + tile - 1) / tile);
     const bool look_back = n <= kLookBackMax;
-    l.n_parts = std::min(l.n_tiles, kCountBlocks);
+    const int64_t tile = look_back ? kRadixTileFew : kRadixTile;
+    l.n_tiles = (int32_t)std::max<int64_t>(1, (n + tile - 1) / tile);
     size_t off = 0;
     l.keys_tmp = off; off += a256(4 * (size_t)n);
     l.vals_tmp = off; off += a256(4 * (size_t)n);
-    l.part = off; off += look_back ? a256(4 * (size_t)l.n_parts * kMaxPasses * kRadixBins) : 0;
+    l.part = off; off += look_back ? a256(4 * (size_t)l.n_tiles * kMaxPasses * kRadixBins) : 0;
     l.base = off; off += a256(4 * (size_t)kMaxPasses * kRadixBins);  // (without look-back: the digit totals)
     l.tickets = off; off += a256(4 * (size_t)kMaxPasses);
     // (without look-back the tile counts take the place of the first status words)
@@ -469,7 +465,6 @@ RadixLayout radix_layout(int64_t n) {
 // next, and a workspace taken for n serves smaller sorts too).
 size_t radix_sort_workspace(int64_t n) {
     size_t bytes = radix_layout(n).total;
-    if (n > kFewMax) bytes = std::max(bytes, radix_layout(kFewMax).total);
     if (n > kLookBackMax) bytes = std::max(bytes, radix_layout(kLookBackMax).total);
     return bytes;
 }
@@ -503,16 +498,11 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
         return;
     }
     const bool look_back = n <= kLookBackMax;
-    const bool direct = l.n_parts <= kDirectParts, few = n <= kFewMax;
+    const bool direct = l.n_tiles <= kDirectParts;
     if (look_back) {
 #define TK_COUNT(P)                                                                                               \
     case P:                                                                                                       \
-        if (few)                                                                                                  \
-            hipLaunchKernelGGL((radix_count_kernel<P, kRadixItemsFew>), dim3(l.n_parts), block, 0, stream,        \
-                               keys_in, n, l.n_tiles, part, tickets, status[0]);                                  \
-        else                                                                                                      \
-            hipLaunchKernelGGL((radix_count_kernel<P, kRadixItems>), dim3(l.n_parts), block, 0, stream, keys_in,  \
-                               n, l.n_tiles, part, tickets, status[0]);                                           \
+        hipLaunchKernelGGL(radix_count_kernel<P>, grid, block, 0, stream, keys_in, n, part, tickets, status[0]);  \
         break;
         switch (passes) {
             TK_COUNT(1)
@@ -523,7 +513,7 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
 #undef TK_COUNT
         TK_HIP_CHECK(hipGetLastError());
         if (!direct) {
-            hipLaunchKernelGGL(radix_base_kernel, dim3(passes), dim3(kBaseBlock), 0, stream, part, l.n_parts, passes,
+            hipLaunchKernelGGL(radix_base_kernel, dim3(passes), dim3(kBaseBlock), 0, stream, part, l.n_tiles, passes,
                                base);
             TK_HIP_CHECK(hipGetLastError());
         }
@@ -540,25 +530,19 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
         if (look_back) {
             args.base = direct ? nullptr : base + p * kRadixBins;
             args.part = direct ? part + p * kRadixBins : nullptr;
-            args.n_parts = l.n_parts;
+            args.n_parts = l.n_tiles;
             args.part_stride = passes * kRadixBins;
             args.ticket = tickets + p;
             args.status = status[p & 1];
             args.status_next = status[(p + 1) & 1];
-            if (few)
-                hipLaunchKernelGGL((radix_pass_kernel<true, kRadixItemsFew>), grid, block, 0, stream, ks, vs, n, 8 * p,
-                                   args, kd, vd);
-            else
-                hipLaunchKernelGGL((radix_pass_kernel<true, kRadixItems>), grid, block, 0, stream, ks, vs, n, 8 * p, args,
-                                   kd, vd);
+            hipLaunchKernelGGL(radix_pass_kernel<true>, grid, block, 0, stream, ks, vs, n, 8 * p, args, kd, vd);
         } else {
             args.hist = status[0];
             args.total = base;
             hipLaunchKernelGGL(radix_hist_kernel, grid, block, 0, stream, ks, n, 8 * p, l.n_tiles, status[0]);
             hipLaunchKernelGGL(radix_scan_kernel, dim3(kRadixBins), dim3(kScanBlock), 0, stream, status[0], l.n_tiles,
                                base);
-            hipLaunchKernelGGL((radix_pass_kernel<false, kRadixItems>), grid, block, 0, stream, ks, vs, n, 8 * p, args,
-                               kd, vd);
+            hipLaunchKernelGGL(radix_pass_kernel<false>, grid, block, 0, stream, ks, vs, n, 8 * p, args, kd, vd);
         }
         TK_HIP_CHECK(hipGetLastError());
         ks = kd;
