@@ -136,7 +136,7 @@ int tk_tree_get_variant(const tk_tree* tree, int* variant);
 
 /* Lanes per query of the tree's later GPU searches (no counterpart in the reference, whose kernel
  * gives every query a fixed number of threads, src/kdtree_g.cu:281-283): 0 (the default) = chosen from
- * the call's size, k, dims and dtype; 1 = one lane per query (d <= 3, k <= 32); 4 (d <= 3, k <= 8),
+ * the call's size, k, tie policy and the tree; 1 = one lane per query (k <= 32); 4 (d <= 3, k <= 8),
  * 8 (d <= 3, k <= 16) or 16 lanes share a query.  A choice that is not prebuilt for a search is
  * ignored by it.  Results never depend on it. */
 int tk_tree_set_lanes(tk_tree* tree, int lanes);

@@ -502,8 +502,8 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 // ------------------------------------------------------------------------------------------
 // Lanes per query, measured on MI355X (whole queries in us or ms; "/" separates the forms, "s" marks one
 // with the presort, which one lane always has).
-// * k > 32 and d = 8: 16 lanes at every size.  One lane's list does not fit its registers (100K queries, k =
-//   100: 0.85 ms; 19.3 ms with one lane's list in LDS), and at d = 8 the walks of 64 lanes part (500K
+// * k > 32, and d = 8 but on few points: 16 lanes at every size.  One lane's list does not fit its registers (100K
+//   queries, k = 100: 0.85 ms; 19.3 ms with one lane's list in LDS), and at d = 8 the walks of 64 lanes part (500K
 //   queries, k = 32: 19 ms against 45).
 // * few queries leave the chip idle with one lane each, and a search is then one chain of dependent
 //   loads, which more lanes shorten.  d = 3, k = 8, 16 / 8 / 4 / 1 lanes: cloud of 100K points, 1,000 queries
@@ -521,23 +521,82 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 //   777 / 788 / 1,450; 1.5M 1,937 / 1,890 / 2,428; 2M of a uniform cloud - / 2.11 / 1.96 ms.
 // * trees of big leaves (record-group boxes), k <= 8: 4s at every larger size (depth 13, k = 8: 1M of 1M points
 //   588 / 658; 4M of 4M points 3.48 / 3.92 ms, 16M 11.7 / 11.9).
-int search_lanes(const Tree& t, int64_t nq, int k) {
+// * from some size on one lane is faster, the sooner the shorter the walks (few axes, few points) and the longer
+//   the list.  Where the two cross, in thousands of queries (clustered clouds of 1M points in brackets; "l" the
+//   lower-index policy):
+//     one axis     16 entries 515-595 (595), "l" 350-730 (435);  32: 310-380 (360), "l" 240-320 (280)
+//     two axes     8: 635-810 (2,330);  16: 310-540 (1,220), "l" 250-370 (800);  32: 160-325 (890), "l" 160-240
+//     three axes   8: 500-910 (3,000);  16: 255-350 below 10K points, 580-850 (1,970) above, "l" 250-480 (1,010);
+//                  32: 165-370, 640-1,320 (2,530), "l" 125-340 (800)
+//   A list that k does not fill costs one lane more (its rows go out in 4-byte stores): 12 of 16 entries, one axis none
+//   up to 3M, two 810 and more, three 470 and more; 24 of 32, one none, two 305-455 (1,500), three 235-475, 880 and more.
+//   So does the (distance, index) list, of doubles and of clouds that tie often: doubles "l", 16 and 32, two axes
+//   500-520 at 300 points, 1,430 and more above.  Doubles: two axes, 8: 545-820 (1,920), 16: 250-395 (970), 32: 165-360 (1,630);
+//   three axes, 16: 220 at 300 points, 830 at 100K, 2,000 at 1M; 32: 165, 1,430, 2,000.
+// * doubles on one axis or two, k <= 8, 16 / 8 / 4 / 1 lanes: d = 2, 100K points, k = 4, 120K 54 / 46 / 39 / 95; 1M 379 / 299 /
+//   223 / 222; k = 8, 120K 67 / 56 / 49 / 105; 1M 472 / 371 / 290 / 266; d = 1, k = 4, 1M 212 / 162 / 114 / 168.
+// * d = 8 on few points: with hundreds of queries a point, presorted neighbours take the same walk and the 64 lanes
+//   of a wavefront stay together.  16 / 1 lanes, k = 16: 500 points, 120K 144 / 155, 250K 278 / 236, 1M 1,046 / 743; 2,000 points, 600K
+//   1,853 / 1,835, 1M 3,039 / 2,865; 10,000 points, 1M 8.3 / 10.3 ms.  f64: 500 points, 60K 164 / 181, 120K 319 / 235, 1M 2,473 / 1,457;
+//   2,000 points, 250K 2,054 / 1,670, 1M 7,987 / 6,240; 10,000 points, 1M 18.4 / 24.6 ms; k = 32 no gain.  "l", 500 points, k = 16, 250K
+//   316 / 367, 600K 719 / 581; f64 640 / 646, 1,470 / 1,440.  Lists of one or two entries gain only on fewer points
+//   (2,000 points, k = 1, 1M 1.74 / 2.18 ms).
+namespace {
+
+constexpr int32_t kFewPoints = 10000, kManyPoints = 500000;
+
+// Queries up to which a group search at d <= 3 and k <= 32 is taken.  keyed: the (distance, index) list; flagged: the
+// lower-index policy's list with tie flags, cheaper beside a group's (distance, index) list.
+int64_t group_search_to(const Tree& t, int k, bool keyed, bool flagged) {
+    const bool f64 = t.dtype == kF64, few = t.n_points < kFewPoints, many = t.n_points >= kManyPoints;
+    const int d = t.dims;
+    if (k <= 8) {
+        if (!f64 && d == 3 && t.dev && t.dev->group_boxes) return INT64_MAX;
+        if (k > 4 && (few ? flagged || (keyed && d > 1) : flagged && d == 2 && !many)) return few ? 600000 : 800000;
+        if (d == 1) return f64 ? 1750000 : 4000000;
+        if (few || (d == 2 && !(f64 && many))) return 1000000;
+        return f64 ? 1750000 : 1500000;
+    }
+    const bool wide = k > 16, full = k == 16 || k == 32;
+    const int64_t most = f64 ? 1750000 : wide ? 1200000 : 1000000;
+    if (keyed) {
+        if (!full || !(few || d == 1)) return most;
+        return d > 1 || f64 ? 1000000 : wide ? 300000 : 600000;
+    }
+    int64_t to;
+    if (d == 1)
+        to = wide ? 300000 : 600000;
+    else if (d == 2)
+        to = wide ? (few ? 165000 : !many ? 320000 : f64 ? most : 900000) : few ? 300000 : !many ? 450000 : 1000000;
+    else
+        to = few ? (wide ? 200000 : 250000) : wide && !f64 && !many ? 650000 : most;
+    if (!full) to = std::min(most, d == 1 ? 3 * to : wide ? to * 3 / 2 : 2 * to);
+    return flagged && (wide || !many) ? to * 3 / 5 : to;
+}
+
+}  // namespace
+
+int search_lanes(const Tree& t, int64_t nq, int k, bool lower) {
     const auto prebuilt = [&](int lanes) {
-        return lanes == 16 || (t.dims <= 3 && (lanes == 1 ? k <= 32 : lanes == 4 ? k <= 8 : k <= 16));
+        return lanes == 16 || (lanes == 1 ? k <= 32 : t.dims <= 3 && (lanes == 4 ? k <= 8 : k <= 16));
     };
     if (t.lanes && prebuilt(t.lanes)) return t.lanes;
-    if (t.dims == 8 || k > 32) return 16;
-    if (t.dtype == kF64) {
-        if (nq > 1750000) return 1;
-        return k > 16 || nq <= 500000 ? 16 : 8;
+    if (k > 32) return 16;
+    const bool f64 = t.dtype == kF64, few = t.n_points < kFewPoints, many = t.n_points >= kManyPoints;
+    if (t.dims == 8) {
+        const int32_t points = k <= (f64 && !lower ? 2 : 4) ? 1000 : 5000;
+        const int64_t a_point = f64 ? (lower ? 400 : k > 8 ? 50 : 100) : lower ? 800 : 250;
+        return t.n_points < points && (!f64 || k <= 16) && nq > a_point * t.n_points ? 1 : 16;
     }
     if (nq <= 24000) return 16;
-    if (k > 16) return nq <= 1200000 ? 16 : 1;
-    if (k > 8) return nq <= 60000 ? 16 : nq <= 1000000 ? 8 : 1;
-    if (t.dims <= 2) return nq <= (t.dims == 1 ? 4000000 : 1000000) ? 4 : 1;
-    if (nq <= 250000) return 8;
-    if (nq <= 1500000) return 4;
-    return t.dev && t.dev->group_boxes ? 4 : 1;
+    const bool keyed = lower && (f64 || t.lower_keyed());
+    if (nq > group_search_to(t, k, keyed, lower && !keyed)) return 1;
+    if (k > 16) return 16;
+    const bool deep = f64 && !few && (t.dims == 3 || (t.dims == 2 && many && lower));
+    if (deep) return nq <= 500000 ? 16 : k > 8 || nq <= 1000000 || lower || (t.dev && t.dev->group_boxes) ? 8 : 4;
+    if (k > 8) return nq <= 60000 ? 16 : 8;
+    if (f64) return nq <= (few ? 30000 : 60000) ? 16 : 4;
+    return t.dims == 3 && nq <= (few ? 100000 : 250000) ? 8 : 4;
 }
 
 namespace {
@@ -551,25 +610,29 @@ inline size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 // always needs the order, to keep its wavefront's walks together; groups gain cache hits.  Without / with:
 // d = 8, k = 32, 500K queries 27.4 / 23.6 ms, equal at 100K; k = 100, 1M 7.6 / 6.4 ms, equal at 100K; d = 3, k = 8: 600K
 // 384 / 365 us (1M points), 274 / 303 (100K points), 1M 618 / 533; k = 16: 300K 276 / 300, 600K 528 / 486; k = 32: 300K
-// 515 / 519, 600K 1,003 / 900; doubles, k = 16: 150K 302 / 320, 500K 835 / 777; d = 2, k = 8, 1M 243 / 267.
+// 515 / 519, 600K 1,003 / 900; doubles, k = 16: 150K 302 / 320, 500K 835 / 777; d = 2, k = 8, 1M 243 / 267, doubles, 100K
+// points, k = 4, 1M 223 / 263.  d = 8 on trees of few points, k = 16, without / leaf / curve: 2,000 points, 250K 795 / 861 /
+// 855, 1M 2,980 / 3,049 / 2,899 (k = 1: 1,632 / 1,730 / 1,522); 10,000 points, 250K 2,197 / 2,324 / 2,095.
 int64_t group_presort_from(const Tree& t, int k) {
-    if (t.dims == 8) return 65536;
+    if (t.dims == 8) return t.n_points < kFewPoints ? 750000 : 65536;
     if (k > 32) return 131072;
+    if (t.dims <= 2 && k <= 8 && !(t.dtype == kF64 && t.n_points >= kManyPoints)) return INT64_MAX;
     if (t.dtype == kF64) return 400000;
-    if (t.dims <= 2 && k <= 8) return INT64_MAX;
     return k > 16 ? 400000 : k > 8 ? 550000 : 700000;
 }
 
 // The presort of a call.  Asked for by name it always runs.  Auto: from kPresortMinQueries queries, and for
-// groups from group_presort_from.  The order: the space-filling curve at d <= 3; the near-leaf order at d = 8,
-// where the curve over a 3-bit-per-axis grid groups queries more coarsely.
+// groups from group_presort_from.  The order: the space-filling curve at d <= 3 and, for groups, on trees of
+// few points; the near-leaf order at d = 8, where the curve over a 3-bit-per-axis grid groups queries more
+// coarsely.
 int presort_mode(const Tree& t, int64_t nq, int k, const QueryOpts& o) {
     if (nq <= 0) return kPresortOff;
     if (o.presort == kPresortAuto) {
         if (nq < kPresortMinQueries || t.levels <= 1) return kPresortOff;
         const bool exact = o.tie != kTieLowerIndex && !(t.finite && t.split_bounds);
-        if (!exact && search_lanes(t, nq, k) > 1 && nq < group_presort_from(t, k)) return kPresortOff;
-        return t.dims == 8 ? kPresortLeaf : kPresortMorton;
+        const bool groups = !exact && search_lanes(t, nq, k, o.tie == kTieLowerIndex) > 1;
+        if (groups && nq < group_presort_from(t, k)) return kPresortOff;
+        return t.dims == 8 && !(groups && t.n_points < kFewPoints) ? kPresortLeaf : kPresortMorton;
     }
     if (o.presort != kPresortOff && o.presort != kPresortMorton && o.presort != kPresortLeaf)
         throw std::runtime_error("unknown presort mode");
@@ -630,10 +693,9 @@ static_assert(16 * kQuerySlice + kGroupBlock < (int64_t(1) << 32), "threads of a
 
 size_t query_gpu_workspace(const Tree& t, int64_t nq, const QueryOpts& o) {
     nq = std::min(nq, kQuerySlice);
-    // (auto: what a call of this size takes if it presorts, which depends on k)
-    const int mode = o.presort != kPresortAuto ? presort_mode(t, nq, 1, o)
+    // (auto: what a call of this size takes if it presorts, which depends on k; either order takes the same)
+    const int mode = o.presort != kPresortAuto                  ? presort_mode(t, nq, 1, o)
                      : nq < kPresortMinQueries || t.levels <= 1 ? kPresortOff
-                     : t.dims == 8                              ? kPresortLeaf
                                                                 : kPresortMorton;
     if (mode == kPresortOff) return 0;
     return presort_layout(t, nq, mode).total;

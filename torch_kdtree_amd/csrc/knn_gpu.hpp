@@ -89,9 +89,9 @@ constexpr int kNumTreeVariants = (int)(sizeof(kTreeVariants) / sizeof(kTreeVaria
 bool launch_tree_variant_f32_d3(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, int kb,
                                 float* dist, int32_t* idx, int64_t* orig, bool lower, int variant, hipStream_t s);
 
-// Lanes per query of a tree search (finite trees, or the lower-index policy): 1 (knn_tree.hpp, d <= 3
-// and k <= 32), 4, 8 or 16 (knn_group.hpp).  Results never depend on it.
-int search_lanes(const Tree& t, int64_t nq, int k);
+// Lanes per query of a tree search (finite trees, or the lower-index policy): 1 (knn_tree.hpp, k <= 32), 4, 8
+// or 16 (knn_group.hpp).  Results never depend on it.
+int search_lanes(const Tree& t, int64_t nq, int k, bool lower);
 constexpr int kGroupBlock = 256;  // threads per block of a group search
 // Group searches (knn_group_f32.hip / knn_group_f64.hip).
 void launch_group_search_f32(const Tree& t, const float* q, int64_t nq, const int32_t* order, int k, float* dist,

@@ -11,7 +11,7 @@ void launch_tree_search_f32(const Tree& t, const float* q, int64_t nq, const int
         launch_exact_search_t<float>(t, q, nq, order, k, dist, idx, orig, s);
         return;
     }
-    const int lanes = search_lanes(t, nq, k);
+    const int lanes = search_lanes(t, nq, k, tie == kTieLowerIndex);
     if (lanes > 1) {
         launch_group_search_f32(t, q, nq, order, k, dist, idx, orig, tie == kTieLowerIndex, lanes, s);
         return;

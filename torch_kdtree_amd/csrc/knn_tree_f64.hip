@@ -11,7 +11,7 @@ void launch_tree_search_f64(const Tree& t, const double* q, int64_t nq, const in
         launch_exact_search_t<double>(t, q, nq, order, k, dist, idx, orig, s);
         return;
     }
-    const int lanes = search_lanes(t, nq, k);
+    const int lanes = search_lanes(t, nq, k, tie == kTieLowerIndex);
     if (lanes > 1)
         launch_group_search_f64(t, q, nq, order, k, dist, idx, orig, tie == kTieLowerIndex, lanes, s);
     else

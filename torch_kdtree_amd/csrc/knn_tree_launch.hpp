@@ -12,7 +12,7 @@ TreeView<T> tree_view(const Tree& t) {
     TreeView<T> v{static_cast<const T*>(t.dev->split), t.dev->recs, t.dev->leaf_off, t.dev->shuffled,
                   t.dev->inv_shuffled, t.dev->boxes, t.levels, t.n_nodes};
     v.split_bounds = t.finite && t.split_bounds;
-    v.lower_direct = t.lower_list == 2 || (t.lower_list == 0 && t.tie_prone);
+    v.lower_direct = t.lower_keyed();
     v.group_boxes = t.dev->group_boxes;
     v.group_base = t.dev->group_base;
     return v;
@@ -73,7 +73,7 @@ void launch_tree_exact(const TreeView<T>& tv, const T* q, int64_t nq, const int3
     TK_HIP_CHECK(hipGetLastError());
 }
 
-// The search with one lane per query: d <= 3, k <= 32 (search_lanes picks it).
+// The search with one lane per query: k <= 32 (search_lanes picks it).
 template <typename T>
 void launch_lane_search_t(const Tree& t, const T* q, int64_t nq, const int32_t* order, int k, T* dist, int32_t* idx,
                           int64_t* orig, int tie, hipStream_t s) {
@@ -89,7 +89,8 @@ void launch_lane_search_t(const Tree& t, const T* q, int64_t nq, const int32_t* 
         TK_DIMS(1)
         TK_DIMS(2)
         TK_DIMS(3)
-        default: throw std::runtime_error("unsupported dims in a one-lane search");
+        TK_DIMS(8)
+        default: throw std::runtime_error("unsupported dims");
     }
 #undef TK_DIMS
 }

@@ -63,6 +63,8 @@ struct Tree {
     // Set at upload: exact distance ties look common among this cloud's neighbours (duplicated
     // points, coordinates on few distinct values), or the tree holds a non-finite value.
     bool tie_prone = false;
+    // Whether lower-index float searches keep the (distance, original index) list from the start.
+    bool lower_keyed() const { return lower_list == 2 || (lower_list == 0 && tie_prone); }
     DeviceTree* dev = nullptr;          // GPU copy, owned
     // A tree built on the GPU has its arrays there alone until something asks for them on the host:
     // axis, split, leaf_off, points, shuffled and aabb are then filled from the GPU copy
