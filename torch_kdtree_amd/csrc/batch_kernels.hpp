@@ -142,7 +142,7 @@ __device__ __forceinline__ void batch_lane(const BatchArgs<T>& ba, int64_t tpos,
     } else if constexpr (kWalk) {
         static_assert(!kLower, "the reference's steps under the reference policy");
         RecKeyRef<T, K> ref{kb};
-        knn_search_one<T, D, false, false>(tv, q, ref);
+        knn_search_one<T, D, false>(tv, q, ref);
     } else {
         while (!lane_step<T, D, K, kLower, CH, LD>(tv, q, pp, kb, far_mask, node, level, st_d, st_o)) {
         }

@@ -166,7 +166,8 @@ constexpr int kTreeBlock = TK_TREE_BLOCK;
 constexpr int kTreeBlockStride = kTreeBlock;
 
 // The reference's own list, for trees with non-finite values under the reference tie policy.  Held
-// in LDS: slot j of lane t lives at base[j * blockDim + t] (consecutive lanes hit consecutive banks).  A candidate is rejected only when d >= worst (src/nndistance.hpp:77) and
+// in LDS: slot j of lane t lives at base[j * blockDim + t] (consecutive lanes hit consecutive banks).  A
+// candidate is rejected only when d >= worst (src/nndistance.hpp:77) and
 // is placed by the reference's binary search (upperBound, src/nndistance.hpp:41-60), so a NaN
 // distance is taken and goes to the front, and the search's path through a list holding NaN
 // entries decides where each later value lands; a NaN reaching the last slot makes worst NaN,
@@ -268,8 +269,7 @@ struct KBestTie : KBest<T, K, false> {
 // 32 take KBestTie (TK_LOWER_TIE_LIST 1): the 64-bit keyed list spends more issue slots per
 // insertion than the med3 list plus the tie flags, and needs the original indices staged with the
 // distances (plain workload, k = 16: 9.96-9.99 ms against 8.29-8.63; k = 32: 22.1-22.2 against
-// 16.9-17.1; d8_mixture, k = 32, 500K queries: 87.1-90.4 against 78.1-79.1).  Lists of at most 4
-// keep it: their insertions are short.
+// 16.9-17.1).  Lists of at most 4 keep it: their insertions are short.
 // kTieOK false: the 64-bit keyed list in any case (trees whose clouds tie often, Tree::tie_prone).
 template <typename T, int K, bool kLower, bool kTieOK = true>
 struct TreeList {
@@ -328,23 +328,14 @@ __device__ __forceinline__ bool lower_split_passes(const TreeView<T, kB>& tv, co
     return !tv.split_bounds || lower_passes(clean_bound<T, D>(q, pp, a, m), worst);
 }
 
-// Far side test for the child `far_child` of split (a, m).  Reference policy: the reference's own
-// test (proj_bound < worst) decides whether the reference would look at the far side; the
-// distance to the box of the points there then tells whether that look could change anything:
-// when it is >= worst every point there has d >= worst and would be rejected.  Lower-index
-// policy: the cell bound with one rounding per term and the box distance, both non-strict, so
-// that a point at exactly the worst distance with a lower index is still found.
-// Returns 0: skip (the reference skips too), 1: enter, 2: skip a side the reference enters.
-template <typename T, int D, bool kLower, bool kB>
-__device__ __forceinline__ int far_side(const TreeView<T, kB>& tv, const Pt<T, D>& q, const Pt<T, D>& pp, int a, T m,
-                                       int32_t far_child, T worst) {
-    if constexpr (kLower) {
-        if (!lower_split_passes<T, D>(tv, q, pp, a, m, worst)) return 0;
-        return lower_passes(aabb_bound<T, D>(tv.boxes, tv.box_of(far_child), q), worst) ? 1 : 0;
-    } else {
-        if (!(proj_bound<T, D>(q, pp, a, m) < worst)) return 0;
-        return aabb_bound<T, D>(tv.boxes, tv.box_of(far_child), q) < worst ? 1 : 2;
-    }
+// The lower-index policy's far side test for the child `far_child` of split (a, m): the cell bound with one
+// rounding per term and the box distance, both non-strict, so that a point at exactly the worst distance
+// with a lower index is still found.
+template <typename T, int D, bool kB>
+__device__ __forceinline__ bool far_side_lower(const TreeView<T, kB>& tv, const Pt<T, D>& q, const Pt<T, D>& pp, int a,
+                                               T m, int32_t far_child, T worst) {
+    return lower_split_passes<T, D>(tv, q, pp, a, m, worst) &&
+           lower_passes(aabb_bound<T, D>(tv.boxes, tv.box_of(far_child), q), worst);
 }
 
 // Whether a leaf can hold a point the list accepts (the reference scans it anyway; when the
@@ -649,12 +640,11 @@ __device__ __forceinline__ bool lane_step(const TreeView<T, kB>& tv, const Pt<T,
     }
 }
 
-// Reference-order search with a generic list: the same walk as lane_start/lane_step, one node at a
-// time (re-searches, and trees with non-finite values).  kBoxes false: no point-box tests, so the walk is
-// the reference's own (src/kdtree.cpp:16-110), step for step (trees with non-finite values).
-template <typename T, int D, bool kLower, bool kBoxes = true, typename List, bool kB>
+// The search with a generic list, one node at a time.  Reference policy: the reference's own walk
+// (src/kdtree.cpp:16-110), step for step and without point boxes (trees with non-finite values, or splits that
+// do not bound their points).  Lower-index policy: the same walk with that policy's tests (research_lower).
+template <typename T, int D, bool kLower, typename List, bool kB>
 __device__ __forceinline__ void knn_search_one(const TreeView<T, kB>& tv, const Pt<T, D>& q, List& kb) {
-    static_assert(kBoxes || !kLower, "the lower-index policy always prunes with boxes");
     Pt<T, D> pp = q;
     const int L = tv.levels;
     const int32_t nn = tv.n_nodes;
@@ -673,11 +663,11 @@ __device__ __forceinline__ void knn_search_one(const TreeView<T, kB>& tv, const 
             const bool lower = qa < m;
             const int32_t near_leaf = 2 * node + (lower ? 1 : 2) - nn;
             const int32_t far_leaf = 2 * node + (lower ? 2 : 1) - nn;
-            if (!kBoxes || leaf_useful<T, D, kLower>(tv, q, near_leaf, kb.worst()))
+            if (!kLower || leaf_useful<T, D, kLower>(tv, q, near_leaf, kb.worst()))
                 scan_leaf<T, D>(tv, near_leaf, q, kb);
-            if ((kLower ? lower_split_passes<T, D>(tv, q, pp, a, m, kb.worst())
-                        : proj_bound<T, D>(q, pp, a, m) < kb.worst()) &&
-                (!kBoxes || leaf_useful<T, D, kLower>(tv, q, far_leaf, kb.worst())))
+            if (kLower ? lower_split_passes<T, D>(tv, q, pp, a, m, kb.worst()) &&
+                             leaf_useful<T, D, kLower>(tv, q, far_leaf, kb.worst())
+                       : proj_bound<T, D>(q, pp, a, m) < kb.worst())
                 scan_leaf<T, D>(tv, far_leaf, q, kb);
             if (level == 0) return;
             ax_set(pp, a, qa);
@@ -694,22 +684,13 @@ __device__ __forceinline__ void knn_search_one(const TreeView<T, kB>& tv, const 
             if (child == 2 * node + (lower2 ? 1 : 2)) {
                 const int32_t far_child = 2 * node + (lower2 ? 2 : 1);
                 ax_set(pp, a, m2);
-                const int f = kBoxes ? far_side<T, D, kLower>(tv, q, pp, a, m2, far_child, kb.worst())
-                                     : (proj_bound<T, D>(q, pp, a, m2) < kb.worst() ? 1 : 0);
-                if (f == 1) {
+                if (kLower ? far_side_lower<T, D>(tv, q, pp, a, m2, far_child, kb.worst())
+                           : proj_bound<T, D>(q, pp, a, m2) < kb.worst()) {
                     node = far_child;
                     ++level;
                     a = ax_next<D>(a);
                     entered = true;
                     break;
-                }
-                if (f == 2) {
-                    const int nlev = min(D, L - 1 - level);
-#pragma unroll
-                    for (int i = 0; i < D; ++i) {
-                        const int off = (i - a - 1 + 2 * D) % D;
-                        if (off < nlev) pp[i] = q[i];
-                    }
                 }
             }
             ax_set(pp, a, q2);
@@ -1051,7 +1032,7 @@ __global__ __launch_bounds__(kLdsBlock) void knn_tree_exact_kernel(TreeView<T> t
     kb.init();
     Pt<T, D> q;
     load_query<T, D>(queries, qi, q);
-    knn_search_one<T, D, false, false>(tv, q, kb);
+    knn_search_one<T, D, false>(tv, q, kb);
     for (int j = 0; j < k; ++j) {
         const int32_t sj = kb.s[j * kLdsBlock];
         out_d[qi * k + j] = kb.d[j * kLdsBlock];
