@@ -10,7 +10,8 @@
 //   * leaf scan: each lane takes one record of every G, so records are read as contiguous runs;
 //   * list: sorted over the lanes, E entries each; an insertion moves the entries of all lanes one
 //     slot at once, the last entry of a lane going to the next lane by DPP;
-//   * climb: each lane tests one level of the path (the box of its far child), all at the same time, and a ballot picks the deepest level whose far side is to be entered.
+//   * climb: each lane tests one level of the path (the box of its far child), all at the same time, and a ballot
+//     picks the deepest level whose far side is to be entered.
 // Every test uses the values and the rounding of knn_tree.hpp's search, so the visited leaves,
 // their order and the outputs are the same bits.
 //
@@ -161,9 +162,11 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
     constexpr int CH = U * G;
     static_assert(CH <= 32 && G - 1 <= kRecPad, "candidate mask and padding records");
     static_assert(D <= G, "a lane per axis");
+    static_assert(kMaxLevels <= 24, "32-bit offsets of 2^25 boxes of 128 bytes");
     __shared__ T stage_d[QB * (CH + 1)];
     __shared__ int32_t stage_o[kLower ? QB * (CH + 1) : 1];
-    constexpr int kLevelQs = 24 + 4;  // kMaxLevels and the levels a descent round may look past them
+    constexpr int kLevelQs = kMaxLevels + 4;  // with the levels that a descent round may look past the last
+    static_assert(S <= 4, "levels of a descent round");
     __shared__ T s_q[QB * kLevelQs];
 
     const int g = (int)(threadIdx.x & (G - 1));
@@ -231,7 +234,7 @@ __global__ __launch_bounds__(kGroupBlock) void knn_group_kernel(
         // lane) bound the search (500K queries, k = 32: 23.2 -> 19.0 ms); at d <= 3 the bookkeeping costs more
         // than the loads (depth-13 tree, k = 8, 1M queries: 0.58 -> 0.63 ms).
         constexpr bool kKeep = D > 3;
-        constexpr int NB = (24 + G - 1) / G;  // kMaxLevels
+        constexpr int NB = (kMaxLevels + G - 1) / G;
         T tb[kKeep ? NB : 1];
 #pragma unroll
         for (int b = 0; b < (kKeep ? NB : 1); ++b) tb[b] = T(0);
