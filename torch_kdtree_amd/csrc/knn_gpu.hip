@@ -570,7 +570,7 @@ int64_t group_search_to(const Tree& t, int k, bool keyed, bool flagged) {
         to = wide ? (few ? 165000 : !many ? 320000 : f64 ? most : 900000) : few ? 300000 : !many ? 450000 : 1000000;
     else
         to = few ? (wide ? 200000 : 250000) : wide && !f64 && !many ? 650000 : most;
-    if (!full) to = std::min(most, d == 1 ? 3 * to : wide ? to * 3 / 2 : 2 * to);
+    if (!full) to = !wide && !f64 ? most : std::min(most, d == 1 ? 3 * to : wide ? to * 3 / 2 : 2 * to);
     return flagged && (wide || !many) ? to * 3 / 5 : to;
 }
 
