@@ -1,6 +1,6 @@
 """A tree that the GPU build left on the GPU against the same tree written to a file, loaded and uploaded
 from the host: structured points, index maps, nodes, the choice of the lower-index list, and query
-results under both policies.  Sizes around the node sort in LDS (nodes of at most 2,048 points), leaves
+results under both policies.  Sizes around the node sort in LDS (nodes of at most 4,096 points), leaves
 of 0 to 2, 16, 64 and more points (record-group boxes from 64), and one leaf pair of everything; with
 ties, repeated points, and infinite coordinates."""
 import numpy as np

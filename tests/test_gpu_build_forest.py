@@ -43,3 +43,18 @@ def test_more_tail_nodes_than_one_launch_would_take(cuda):
     rng = np.random.default_rng(5300)
     clouds = [rng.random((1 << 24, 1), dtype=np.float32)] + [rng.random((4096, 1), dtype=np.float32) for _ in range(1024)]
     _forest_equals_single_builds(cuda, clouds, [13] + [13] * 1024, (1, 513, 1024))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,levels", [(4095, 5), (8191, 4), (8192, 4), (8193, 4), (8193, 14), (16_383, 3), (16_385, 6)])
+def test_nodes_around_the_workgroup_size(cuda, dtype, n, levels):
+    """Nodes of just under, exactly and just over 4,096 points, which one workgroup sorts to the leaves: the tree is
+    the host build's, point by point (no two coordinates are equal)."""
+    rng = np.random.default_rng(n + levels)
+    pts = np.stack([rng.permutation(n) for _ in range(3)], axis=1).astype(dtype)
+    host = tk.build_kd_tree(torch.from_numpy(pts), device="cpu", levels=levels)
+    built = tk.build_kd_tree(torch.from_numpy(pts), device=cuda, levels=levels, builder="gpu")
+    assert_same(built.structured_points.cpu().numpy(), host.structured_points.numpy(), "structured points")
+    assert_same(built.shuffled_ind.cpu().numpy(), host.shuffled_ind.numpy(), "indices")
+    for a, b, what in zip(built.kdtree.get_nodes(), host.kdtree.get_nodes(), ("axis", "split", "leaf offsets")):
+        assert_same(a, b, what)

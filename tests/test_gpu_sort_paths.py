@@ -1,6 +1,5 @@
-"""The radix sort's paths against torch's stable sort, at the sizes where one hands over to the next: one
-workgroup (4,096 pairs), counts summed by the passes (32 tiles of 4,096) and look-back
-(2^21 pairs)."""
+"""The radix sort's paths against torch's stable sort: one workgroup (up to 4,096 pairs), look-back passes (up
+to 2^19 pairs), and three launches a pass."""
 import pytest
 import torch
 
