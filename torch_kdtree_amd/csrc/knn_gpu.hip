@@ -722,6 +722,8 @@ void query_gpu(const Tree& t, const void* queries, int64_t nq, int k, void* dist
         }
         return;
     }
+    // (a workspace is one for calls of this size, whether or not this k presorts)
+    if (workspace && workspace_bytes < query_gpu_workspace(t, nq, o)) throw std::runtime_error("query workspace too small");
     DeviceGuard g(t.dev->device);
     const int32_t* order = nullptr;
     std::unique_ptr<StreamScratch> own;
@@ -733,8 +735,6 @@ void query_gpu(const Tree& t, const void* queries, int64_t nq, int k, void* dist
         if (!ws) {
             own.reset(new StreamScratch(l.total, stream));
             ws = static_cast<unsigned char*>(own->ptr);
-        } else if (workspace_bytes < l.total) {
-            throw std::runtime_error("query workspace too small");
         }
         uint32_t* key = reinterpret_cast<uint32_t*>(ws + l.key);
         uint32_t* key_s = reinterpret_cast<uint32_t*>(ws + l.key_s);
