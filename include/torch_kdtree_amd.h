@@ -48,7 +48,7 @@ enum { TK_TIE_REFERENCE = 0, TK_TIE_LOWER_INDEX = 1 };
 /* Query presort before the traversal, so that the lanes of a wavefront get nearby queries:
  * TK_PRESORT_MORTON orders queries along a space-filling curve over a grid on the queries'
  * bounding box (the Hilbert curve for d <= 3, the Morton code for d = 8; the name is kept),
- * TK_PRESORT_LEAF by the tree leaf they fall into; AUTO = MORTON (LEAF at d = 8) in calls large enough
+ * TK_PRESORT_LEAF by the tree leaf they fall into; AUTO = one of them by the tree's d and points, in calls large enough
  * that the search gains more than the sort costs, never below 4096 queries.  The presort changes the order
  * of work only, never the results. */
 enum { TK_PRESORT_AUTO = -1, TK_PRESORT_OFF = 0, TK_PRESORT_MORTON = 1, TK_PRESORT_LEAF = 2 };

@@ -5,7 +5,8 @@
 //   2. one look-back radix_pass_kernel per pass.  Workgroups take tiles of pairs by a ticket, rank
 //      their tile, publish its digit counts and find the pairs of each digit in all earlier
 //      tiles by looking back over the earlier tiles' published counts (each tile publishes first its
-//      own counts, then the sum up to and including it), so a pass is one launch.
+//      own counts, then the sum up to and including it), so a pass is one launch: the single-pass scan of
+//      D. Merrill and M. Garland, "Single-pass parallel prefix scan with decoupled look-back", 2016.
 // More, per pass:
 //   1. radix_hist_kernel counts the digits of every tile;
 //   2. radix_scan_kernel scans the counts of each digit over the tiles;

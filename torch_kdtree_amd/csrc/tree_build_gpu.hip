@@ -601,8 +601,8 @@ __global__ __launch_bounds__(kGbBlock) void gb_groups_kernel(const unsigned char
 
 // The sample of cloud_ties_often (knn_gpu.hip): up to kTieLeaves leaves, kTieLeafPoints points of each.
 // Workgroup a < D counts the distinct values on axis a (a hash set in LDS; -0 equals 0, and a double
-// enters as a 32-bit mix of its bits); the last ones count, per leaf, the points that repeat an
-// earlier point of the leaf's sample.
+// enters as a 32-bit mix of its bits, a step of MurmurHash3's 64-bit finaliser); the last ones count, per
+// leaf, the points that repeat an earlier point of the leaf's sample.
 constexpr int kTieLeaves = 256;
 constexpr int kTieLeafPoints = 64;
 constexpr int kTieBlock = 1024;
