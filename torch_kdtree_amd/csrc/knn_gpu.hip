@@ -533,6 +533,18 @@ int64_t valu_probe_gpu(float* out, int64_t threads, int iters, int mode, hipStre
 //   So does the (distance, index) list, of doubles and of clouds that tie often: doubles "l", 16 and 32, two axes
 //   500-520 at 300 points, 1,430 and more above.  Doubles: two axes, 8: 545-820 (1,920), 16: 250-395 (970), 32: 165-360 (1,630);
 //   three axes, 16: 220 at 300 points, 830 at 100K, 2,000 at 1M; 32: 165, 1,430, 2,000.
+// * big leaves on one axis or two: presorted lanes scan the same records, groups each their own, so the line is a number
+//   of records scanned; on few queries one lane each leaves the chip idle, so it is never below the floors.  Best group / 1,
+//   (s) presorted: d = 1, 64K points, leaves of 500, k = 1, 100K queries 118 / 116, 300K 253 (s) / 146, k = 32, 300K 677 (s) / 650;
+//   1M, leaves of 122, k = 1, 700K 176 / 146, 1.5M 354 (s) / 218; 50K, leaves of 3,125, k = 1, 30K 307 / 356, 60K, k = 8, 565 / 625;
+//   d = 2, 64K, leaves of 250, k = 8, 300K 186 (s) / 196, 700K 304 (s) / 263; 50K, leaves of 3,125, k = 8, 100K 464 / 569, "l" 661 /
+//   1,934.  f64, d = 1, leaves of 250, k = 1, 30K, 16 / 4 lanes 71 / 34.
+// * one pair of leaves (levels 1, no walk; one lane takes no presort): 150 points, d = 1, k = 1, 30K 14.8 / 14.6, 100K 22.3 /
+//   15.0; d = 3, k = 8, 60K 23 / 28, 80K 26 / 29, 100K 33 / 29, k = 16, 60K 35 / 41, 100K 50 / 42; d = 1, k = 32, 80K 60 / 84, 300K 190 /
+//   161; "l", d = 3, k = 8, 80K 35 / 51, 300K 95 / 64; doubles "l", k = 32, 80K 138 / 278, 300K 450 / 634.
+// * leaves of a few points, which a chunk of a group's records exceeds: leaves of 4, d = 3, k = 16, 300K 425 / 416, 700K 897
+//   (s) / 705; f64, k = 8, 8 lanes, 300K 530 / 532, 700K 1,105 (s) / 861, k = 16 1,593 (s) / 1,226; leaves of 2, d = 2, k = 32, 100K 218 /
+//   257, 300K 620 / 406.
 // * doubles on one axis or two, k <= 8, 16 / 8 / 4 / 1 lanes: d = 2, 100K points, k = 4, 120K 54 / 46 / 39 / 95; 1M 379 / 299 /
 //   223 / 222; k = 8, 120K 67 / 56 / 49 / 105; 1M 472 / 371 / 290 / 266; d = 1, k = 4, 1M 212 / 162 / 114 / 168.
 // * d = 8 on few points: with hundreds of queries a point, presorted neighbours take the same walk and the 64 lanes
@@ -549,29 +561,46 @@ constexpr int32_t kFewPoints = 10000, kManyPoints = 500000;
 // lower-index policy's list with tie flags, cheaper beside a group's (distance, index) list.
 int64_t group_search_to(const Tree& t, int k, bool keyed, bool flagged) {
     const bool f64 = t.dtype == kF64, few = t.n_points < kFewPoints, many = t.n_points >= kManyPoints;
-    const int d = t.dims;
-    if (k <= 8) {
-        if (!f64 && d == 3 && t.dev && t.dev->group_boxes) return INT64_MAX;
-        if (k > 4 && (few ? flagged || (keyed && d > 1) : flagged && d == 2 && !many)) return few ? 600000 : 800000;
-        if (d == 1) return f64 ? 1750000 : 4000000;
-        if (few || (d == 2 && !(f64 && many))) return 1000000;
-        return f64 ? 1750000 : 1500000;
-    }
     const bool wide = k > 16, full = k == 16 || k == 32;
+    const int d = t.dims;
+    if (!f64 && d == 3 && k <= 8 && t.dev && t.dev->group_boxes) return INT64_MAX;
     const int64_t most = f64 ? 1750000 : wide ? 1200000 : 1000000;
-    if (keyed) {
-        if (!full || !(few || d == 1)) return most;
-        return d > 1 || f64 ? 1000000 : wide ? 300000 : 600000;
-    }
     int64_t to;
-    if (d == 1)
-        to = wide ? 300000 : 600000;
-    else if (d == 2)
-        to = wide ? (few ? 165000 : !many ? 320000 : f64 ? most : 900000) : few ? 300000 : !many ? 450000 : 1000000;
-    else
-        to = few ? (wide ? 200000 : 250000) : wide && !f64 && !many ? 650000 : most;
-    if (!full) to = !wide && !f64 ? most : std::min(most, d == 1 ? 3 * to : wide ? to * 3 / 2 : 2 * to);
-    return flagged && (wide || !many) ? to * 3 / 5 : to;
+    if (k <= 8) {
+        if (k > 4 && (few ? flagged || (keyed && d > 1) : flagged && d == 2 && !many))
+            to = few ? 600000 : 800000;
+        else if (d == 1)
+            to = f64 ? 1750000 : 4000000;
+        else
+            to = few || (d == 2 && !(f64 && many)) ? 1000000 : f64 ? 1750000 : 1500000;
+    } else if (keyed) {
+        to = !full || !(few || d == 1) ? most : d > 1 || f64 ? 1000000 : wide ? 300000 : 600000;
+    } else {
+        if (d == 1)
+            to = wide ? 300000 : 600000;
+        else if (d == 2)
+            to = wide ? (few ? 165000 : !many ? 320000 : f64 ? most : 900000) : few ? 300000 : !many ? 450000 : 1000000;
+        else
+            to = few ? (wide ? 200000 : 250000) : wide && !f64 && !many ? 650000 : most;
+        if (!full) to = !wide && !f64 ? most : std::min(most, d == 1 ? 3 * to : wide ? to * 3 / 2 : 2 * to);
+        if (flagged && (wide || !many)) to = to * 3 / 5;
+    }
+    const int64_t leaf = t.n_points >> t.levels;  // points of a leaf
+    if (leaf < 8) {
+        if (f64 && d == 3 && !keyed && k > 2)
+            to = std::min<int64_t>(to, 600000);
+        else if (d == 1 && k <= 8)
+            to = k > 4 ? std::min<int64_t>(to, 1200000) : to;
+        else if (k > 8 || (flagged && k > 4))
+            to /= 2;
+    }
+    if (d <= 2 && leaf >= 32) {
+        const bool listed = keyed || flagged;
+        const int64_t scans = !many ? (k <= 8 ? 60000000 : 40000000) : d == 1 || (listed && k > 8) ? 80000000 : 175000000;
+        const int64_t least = d == 1 ? (k > 1 ? 75000 : f64 ? 24000 : 45000) : listed && k > 4 ? 250000 : 150000;
+        to = std::min(to, std::max(least, scans / leaf));
+    }
+    return to;
 }
 
 }  // namespace
@@ -590,12 +619,14 @@ int search_lanes(const Tree& t, int64_t nq, int k, bool lower) {
     }
     if (nq <= 24000) return 16;
     const bool keyed = lower && (f64 || t.lower_keyed());
+    if (t.levels == 1 && !(f64 && keyed && k > 4) && nq > (k == 1 ? 24000 : k > 16 || (lower && k > 4) ? 100000 : 70000)) return 1;
     if (nq > group_search_to(t, k, keyed, lower && !keyed)) return 1;
     if (k > 16) return 16;
     const bool deep = f64 && !few && (t.dims == 3 || (t.dims == 2 && many && lower));
     if (deep) return nq <= 500000 ? 16 : k > 8 || nq <= 1000000 || lower || (t.dev && t.dev->group_boxes) ? 8 : 4;
     if (k > 8) return nq <= 60000 ? 16 : 8;
-    if (f64) return nq <= (few ? 30000 : 60000) ? 16 : 4;
+    const bool scanned = t.dims == 1 && (t.n_points >> t.levels) >= 32;
+    if (f64) return !scanned && nq <= (few ? 30000 : 60000) ? 16 : 4;
     return t.dims == 3 && nq <= (few ? 100000 : 250000) ? 8 : 4;
 }
 
